@@ -52,19 +52,67 @@ struct RedBuf {
     int i[NT / 64];
 };
 
-__device__ inline double wave_jmax(double v) {
-    for (int o = 32; o > 0; o >>= 1) v = jmax(v, __shfl_xor(v, o));
-    return v;
+// a value every lane holds, as a scalar
+__device__ inline int uni(int v) { return __builtin_amdgcn_readfirstlane(v); }
+
+// max(m, |a|), a NaN in a passed over (fmax would first quiet both operands)
+__device__ inline double max_abs(double m, double a) {
+    double r;
+    asm("v_max_f64 %0, %1, |%2|" : "=v"(r) : "v"(m), "v"(a));
+    return r;
+}
+// a wave's largest v (v >= 0 in every lane; a NaN is passed over) in its last lane: row shifts and
+// row broadcasts, no LDS round trip per step
+template <int CTRL, int ROWS>
+__device__ inline double dpp_max_step(double v) {
+    const int2 x = __builtin_bit_cast(int2, v);
+    int2 y;
+    y.x = __builtin_amdgcn_update_dpp(0, x.x, CTRL, ROWS, 0xf, true);
+    y.y = __builtin_amdgcn_update_dpp(0, x.y, CTRL, ROWS, 0xf, true);
+    return max_abs(v, __builtin_bit_cast(double, y));
+}
+__device__ inline double wave_max_last(double v) {
+    v = dpp_max_step<0x111, 0xf>(v);  // row_shr 1, 2, 4, 8
+    v = dpp_max_step<0x112, 0xf>(v);
+    v = dpp_max_step<0x114, 0xf>(v);
+    v = dpp_max_step<0x118, 0xf>(v);
+    v = dpp_max_step<0x142, 0xa>(v);  // row_bcast 15, 31
+    return dpp_max_step<0x143, 0xc>(v);
+}
+__device__ inline double last_lane(double v) {
+    int2 x = __builtin_bit_cast(int2, v);
+    x.x = __builtin_amdgcn_readlane(x.x, 63);
+    x.y = __builtin_amdgcn_readlane(x.y, 63);
+    return __builtin_bit_cast(double, x);
+}
+// a wave's smallest i in its last lane
+template <int CTRL, int ROWS>
+__device__ inline int dpp_min_step(int v) {
+    return min(v, __builtin_amdgcn_update_dpp(0x7fffffff, v, CTRL, ROWS, 0xf, false));
+}
+__device__ inline int wave_min_last(int v) {
+    v = dpp_min_step<0x111, 0xf>(v);
+    v = dpp_min_step<0x112, 0xf>(v);
+    v = dpp_min_step<0x114, 0xf>(v);
+    v = dpp_min_step<0x118, 0xf>(v);
+    v = dpp_min_step<0x142, 0xa>(v);
+    return dpp_min_step<0x143, 0xc>(v);
 }
 
+// (values >= 0) every lane gets the wave's maximum
+__device__ inline double wave_jmax(double v) {
+    const double m = last_lane(wave_max_last(v));
+    return __any(v != v) ? __builtin_nan("") : m;
+}
+
+// (candidates' values >= 0) every lane gets the wave's best candidate; a NaN value, which every
+// lane then holds, stays
 __device__ inline void wave_argmax(double& v, int& i) {
-    for (int o = 32; o > 0; o >>= 1) {
-        const double ov = __shfl_xor(v, o);
-        const int oi = __shfl_xor(i, o);
-        if (vi_better(ov, oi, v, i)) {
-            v = ov;
-            i = oi;
-        }
+    const double m = last_lane(wave_max_last(i >= 0 ? v : 0.0));
+    const int first = __builtin_amdgcn_readlane(wave_min_last(i >= 0 && v == m ? i : 0x7fffffff), 63);
+    if (first != 0x7fffffff) {
+        v = m;
+        i = first;
     }
 }
 
@@ -831,363 +879,462 @@ __global__ void __launch_bounds__(256) k_ldlt_update(DevSym S, const Task* __res
 }
 
 // ---------------------------------------------------------------------------
-// large fronts with deferred updates: k_ldlt_panel (one workgroup per front) takes the pivots
-// of a panel of at least LP_NB columns one after the other. The front's columns from the current
-// pivot on keep, in the panel memory, their values of the panel's start; the columns the pivot
-// choice reads are formed when it reads them, by applying the panel's pivots to them in the
-// reference's order: x - L(i, p) U(p, j) for a 1x1 pivot p, x - (L(i, p) U(p, j) + L(i, p + 1)
-// U(p + 1, j)) for a 2x2 one, pivot after pivot. U(p, j), the row of pivot p in column j at
-// the time of pivot p (the upper mirror entry the reference's update reads), is formed once per
-// pivot for every later column. k_ldlt_trail then applies the panel's pivots to the columns
-// after it in the same way over the GPU. Every entry thus goes through the operations of
-// ldlt_front in the same order, later: the factor is bitwise that of one pivot at a time. The
-// symmetric interchanges act on the stored values, as in the reference; a row interchange of
+// large fronts in panels: k_ldlt_panel (one workgroup per front) takes the pivots of a panel of
+// NBP columns with the columns held in registers: thread t holds the rows k0 + t + NT u of every
+// panel column (R rows, R NBP entries). The usual pivot (column k its own acceptable 1x1 pivot)
+// is one pass: the column's two maxima by lane reductions, one barrier (LDS only: the L column's
+// global stores stay in flight), the scaling and the rank-1 update of the panel's later columns,
+// which moves each column one register to the left. Everything after the panel keeps its values
+// of the panel's start; k_ldlt_trail then applies the panel's pivots to it over the GPU.
+//
+// Any other pivot (a 2x2, an interchange, a perturbation) is decided from the panel memory: the
+// columns the choice reads are formed when it reads them, by applying the panel's pivots to the
+// stored values in the reference's order: x - L(i, p) U(p, j) for a 1x1 pivot p, x - (L(i, p) U(p, j) +
+// L(i, p + 1) U(p + 1, j)) for a 2x2 one. U(p, j), the row of pivot p in column j at the time of
+// pivot p (the upper mirror entry the reference's update reads), is formed for a run of usual
+// pivots at once, before such a pivot and at the panel's end. Every entry thus goes through the
+// operations of ldlt_front in the same order: the factor is bitwise that of one pivot at a time.
+// The symmetric interchanges act on the stored values, as in the reference; a row interchange of
 // two positions at or after the current pivot commutes with the pending updates, since it
-// exchanges the L rows of the panel's pivots too.
+// exchanges the L rows of the panel's pivots too. After such a pivot the rest of the panel is
+// loaded again and brought up to date.
 
-constexpr int LP_NB = 32;           // columns per panel (a 2x2 pivot at its end takes one more)
+constexpr int LP_NB = 16;           // most columns of a panel (a 2x2 pivot at its end takes one more)
 constexpr int LP_MAXP = LP_NB + 1;  // pivot rows of one panel
 
-// scratch of one front during a panel (element offsets from its base): the current columns X0,
-// X1, X2 (f entries each), the pivot rows U (LP_MAXP x w, U[q w + j] = U(k0 + q, j)) and the
-// current diagonal DG (w)
-__host__ __device__ inline int64_t lp_scratch(int f, int w) { return 3 * (int64_t)f + (int64_t)(LP_MAXP + 1) * w; }
+// scratch of one front during a panel (element offsets from its base): the pivot rows U (LP_MAXP x
+// w, U[q w + j] = U(k0 + q, j)), the current diagonal DG (w) and the saved panel columns V (cols x f)
+inline int64_t lp_scratch(int f, int w, int cols) { return (int64_t)(LP_MAXP + 1) * w + (int64_t)cols * f; }
 
-template <typename T, int NT>
+// entry `off` bytes into the column `col` (a wave-uniform address: scalar base, 32-bit offset)
+template <typename T>
+__device__ inline T load_at(const T* col, uint32_t off) {
+    return *reinterpret_cast<const T*>(reinterpret_cast<const char*>(col) + off);
+}
+template <typename T>
+__device__ inline void store_at(T* col, uint32_t off, T v) {
+    *reinterpret_cast<T*>(reinterpret_cast<char*>(col) + off) = v;
+}
+
+// a thread's rows k0 + tid + NT u of a front: their byte offsets in a column and how many lie above an
+// end. Both start from values hidden from the optimizer (empty asm): hoisted out of the pivot loop, the
+// R comparisons of every loop would take R scalar register pairs each.
+template <int NT, int SIZE>
+struct PanelRows {
+    uint32_t o0, olast;
+    int left;  // k0 + tid
+    __device__ __attribute__((always_inline)) PanelRows(int k0, int f) {
+        left = k0 + (int)threadIdx.x;
+        asm volatile("" : "+v"(left));
+        o0 = (uint32_t)left * SIZE;
+        olast = (uint32_t)(f - 1) * SIZE;
+    }
+    __device__ uint32_t off(int u) const { return o0 + (uint32_t)(NT * SIZE) * u; }
+    __device__ uint32_t clamped(int u) const { return min(off(u), olast); }
+    // slots u < count(end) hold rows below end
+    __device__ int count(int end) const { return (end - left + NT - 1) >> (NT == 512 ? 9 : NT == 1024 ? 10 : 8); }
+};
+
+// a front during a panel, as its NT threads see it
+template <typename T, int NT, int R, int MAXP>
 struct PanelFront {
     T* P;
     int f, w, k0;
     int* lp;
     RedBuf<NT>* rb;
-    T *X0, *X1, *X2, *U, *DG;
+    T *U, *DG;
+    T* V;  // the panel's columns kv, kv + 1, ... (MAXP - 1 of them, ld f) as they were before the pivot kv
     // LDS: per column q of the panel (k0 + q) the kind of its pivot step: 0 none yet, 1 a 1x1,
     // 2 the first and 3 the second column of a 2x2
     int* ctype;
-    T* Uc;  // U(., j) of the column being formed
-    T* Lr;  // L(r, .) of the pivot row whose U row is being formed
-    double* skey;
-    int* sidx;
-    int scap;
+    T* Uc;          // U(., j) of the column being formed
+    T* Lr;          // L(r, .) of the pivot row whose U row is being formed
+    T (*Ls)[MAXP];  // Ls[r][q] = L(k0 + r, k0 + q), q < r, of the panel's pivots
+    double* pk;     // picked entries (pick)
 
-    // x minus the panel's pivots in order, lv[q] = L(row, k0 + q) and u(q) = U(k0 + q, column)
-    // (the operations and their order of ldlt_front's updates)
-    template <class UF>
-    __device__ __attribute__((always_inline)) T apply(T x, const T (&lv)[LP_MAXP], UF u) const {
+    // x minus the panel's first np pivots in order, l(q) = L(row, k0 + q) and u(q) = U(k0 + q,
+    // column) (the operations and their order of ldlt_front's updates); eight pivots' entries are
+    // loaded together (the ninth: the second column of a 2x2)
+    template <class LF, class UF>
+    __device__ __attribute__((always_inline)) T apply(T x, int np, LF l, UF u) const {
+#pragma unroll 1
+        for (int q0 = 0; q0 < np; q0 += 8) {
+            T lv[9], uv[9];
 #pragma unroll
-        for (int q = 0; q < LP_MAXP; ++q) {
-            const int ct = ctype[q];
-            if (ct == 1) {
-                x = x - lv[q] * u(q);
-            } else if (ct == 2 && q + 1 < LP_MAXP) {
-                x = x - (lv[q] * u(q) + lv[q + 1] * u(q + 1));
+            for (int q = 0; q < 9; ++q) {
+                lv[q] = l(min(q0 + q, np - 1));
+                uv[q] = u(min(q0 + q, np - 1));
+            }
+#pragma unroll
+            for (int q = 0; q < 8; ++q) {
+                const int ct = q0 + q < np ? uni(ctype[q0 + q]) : 0;
+                if (ct == 1)
+                    x = x - lv[q] * uv[q];
+                else if (ct == 2)
+                    x = x - (lv[q] * uv[q] + lv[q + 1] * uv[q + 1]);
             }
         }
         return x;
     }
-    // L(i, k0 .. k0 + np - 1) into registers, all loads issued before any is used
-    __device__ __attribute__((always_inline)) void load_l(int i, int np, T (&lv)[LP_MAXP]) const {
-#pragma unroll
-        for (int q = 0; q < LP_MAXP; ++q) lv[q] = q < np ? P[(int64_t)(k0 + q) * f + i] : T(0);
+    __device__ __attribute__((always_inline)) PanelRows<NT, (int)sizeof(T)> rows() const { return {k0, f}; }
+    // the thread and the slot of row i
+    __device__ __attribute__((always_inline)) void owner(int i, int& t, int& u) const {
+        const int o = uni(i - k0);
+        u = o / NT;
+        t = o - u * NT;
     }
-    // current values of column j at rows k..f-1 into X (all threads; ends with a barrier)
-    __device__ __attribute__((always_inline)) void form_col(int j, int k, T* X) const {
-        const int np = k - k0;
+    // the thread's rows of a column
+    __device__ __attribute__((always_inline)) void load_rows(const T* col, T (&y)[R]) const {
+        const auto rw = rows();
+#pragma unroll
+        for (int u = 0; u < R; ++u) y[u] = load_at(col, rw.clamped(u));
+    }
+    __device__ __attribute__((always_inline)) void store_rows(T* col, const T (&y)[R]) const {
+        const auto rw = rows();
+        const int nf = rw.count(f);
+#pragma unroll
+        for (int u = 0; u < R; ++u)
+            if (u < nf) store_at(col, rw.off(u), y[u]);
+    }
+    // current values of column j at the thread's rows (all threads; ends with a barrier): from V for
+    // a column of the panel, else the L entries of G pivots in flight together
+    __device__ __attribute__((always_inline)) void form_col(int j, int np, T (&y)[R]) const {
+        if (j < k0 + MAXP - 1) {
+            load_rows(V + (int64_t)(j - k0 - np) * f, y);
+            __syncthreads();
+            return;
+        }
+        constexpr int G = R <= 6 ? 8 : R <= 12 ? 4 : 2;
         for (int q = threadIdx.x; q < np; q += NT) Uc[q] = U[(int64_t)q * w + j];
         __syncthreads();
-        const T* cj = P + (int64_t)j * f;
-        for (int i = k + threadIdx.x; i < f; i += NT) {
-            T lv[LP_MAXP];
-            load_l(i, np, lv);
-            X[i] = apply(cj[i], lv, [&](int q) { return Uc[q]; });
+        load_rows(P + (int64_t)j * f, y);
+        for (int q0 = 0; q0 < np; q0 += G) {
+            const auto rw = rows();
+            T l[G][R];
+#pragma unroll
+            for (int g = 0; g < G; ++g) {
+                const T* cq = P + (int64_t)(k0 + min(q0 + g, np - 1)) * f;
+#pragma unroll
+                for (int u = 0; u < R; ++u) l[g][u] = load_at(cq, rw.clamped(u));
+            }
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int g = 0; g < G; ++g) {
+                const int ct = q0 + g < np ? uni(ctype[q0 + g]) : 0;
+                if (ct == 1) {
+                    const T v = Uc[q0 + g];
+#pragma unroll
+                    for (int u = 0; u < R; ++u) y[u] = y[u] - l[g][u] * v;
+                } else if (ct == 2) {
+                    const T v = Uc[q0 + g], v2 = Uc[q0 + g + 1];
+                    const T* c2 = P + (int64_t)(k0 + q0 + g + 1) * f;
+#pragma unroll
+                    for (int u = 0; u < R; ++u) y[u] = y[u] - (l[g][u] * v + load_at(c2, rw.clamped(u)) * v2);
+                }
+            }
         }
         __syncthreads();
+    }
+    // entry of row i of a column in registers, into pk[slot] (a barrier later)
+    __device__ __attribute__((always_inline)) void pick(const T (&y)[R], int i, int slot) const {
+        int t, us;
+        owner(i, t, us);
+        T v = y[0];
+#pragma unroll
+        for (int u = 1; u < R; ++u) v = u == us ? y[u] : v;
+        if ((int)threadIdx.x == t) pk[slot] = (double)v;
+    }
+    // rows a and b of a column in registers exchanged (pk[sa], pk[sb]: its entries there)
+    __device__ __attribute__((always_inline)) void exchange(T (&y)[R], int a, int b, int sa, int sb) const {
+        const T va = T(pk[sa]), vb = T(pk[sb]);
+        int ta, ua, tb, ub;
+        owner(a, ta, ua);
+        owner(b, tb, ub);
+        const bool ma = (int)threadIdx.x == ta, mb = (int)threadIdx.x == tb;
+#pragma unroll
+        for (int u = 0; u < R; ++u) {
+            y[u] = ma && u == ua ? vb : y[u];
+            y[u] = mb && u == ub ? va : y[u];
+        }
+    }
+    // largest |y_i| over the rows k..f-1 but s1 and s2, NaN-propagating (ldlt.jl:240-260)
+    __device__ __attribute__((always_inline)) double colmax(const T (&y)[R], int k, int end, int s1, int s2) const {
+        // (rows above k: only among the first slot's, the panel is narrower than the block)
+        double m = 0.0;
+        const int n = rows().count(end);
+        int t1, u1, t2, u2;
+        owner(s1, t1, u1);
+        owner(s2, t2, u2);
+        const bool up = (int)threadIdx.x >= k - k0, m1 = (int)threadIdx.x == t1, m2 = (int)threadIdx.x == t2;
+#pragma unroll
+        for (int u = 0; u < R; ++u) {
+            bool on = u < n;
+            if (u == 0) on = on && up;
+            if (u == u1) on = on && !m1;
+            if (u == u2) on = on && !m2;
+            m = on ? jmax(m, fabs((double)y[u])) : m;
+        }
+        return block_jmax<NT>(m, *rb);
     }
     // current diagonal entries of the columns k..w-1 into DG (all threads; ends with a barrier)
     __device__ __attribute__((always_inline)) void form_diag(int k) const {
-        const int np = k - k0;
-        for (int j = k + threadIdx.x; j < w; j += NT) {
-            T lv[LP_MAXP], uv[LP_MAXP];
-            load_l(j, np, lv);
-#pragma unroll
-            for (int q = 0; q < LP_MAXP; ++q) uv[q] = q < np ? U[(int64_t)q * w + j] : T(0);
-            DG[j] = apply(P[(int64_t)j * f + j], lv, [&](int q) { return uv[q]; });
-        }
+        for (int j = k + threadIdx.x; j < w; j += NT)
+            DG[j] = apply(P[(int64_t)j * f + j], k - k0, [&](int q) { return P[(int64_t)(k0 + q) * f + j]; },
+                          [&](int q) { return U[(int64_t)q * w + j]; });
         __syncthreads();
     }
     // U row of the pivot row r (a position at or after the current pivot, before the current
     // pivot's own step is recorded) for the columns j0..w-1 (all threads; ends with a barrier)
     __device__ __attribute__((always_inline)) void form_urow(int r, int j0) const {
         const int np = r - k0;
-        for (int q = threadIdx.x; q < LP_MAXP; q += NT) Lr[q] = q < np ? P[(int64_t)(k0 + q) * f + r] : T(0);
+        for (int q = threadIdx.x; q < np; q += NT) Lr[q] = P[(int64_t)(k0 + q) * f + r];
         __syncthreads();
-        T lv[LP_MAXP];
-#pragma unroll
-        for (int q = 0; q < LP_MAXP; ++q) lv[q] = Lr[q];
-        T* ur = U + (int64_t)(r - k0) * w;
-        for (int j = j0 + threadIdx.x; j < w; j += NT) {
-            T uv[LP_MAXP];
-#pragma unroll
-            for (int q = 0; q < LP_MAXP; ++q) uv[q] = q < np ? U[(int64_t)q * w + j] : T(0);
-            ur[j] = apply(P[(int64_t)j * f + r], lv, [&](int q) { return uv[q]; });
-        }
+        T* ur = U + (int64_t)np * w;
+        for (int j = j0 + threadIdx.x; j < w; j += NT)
+            ur[j] = apply(P[(int64_t)j * f + r], np, [&](int q) { return Lr[q]; },
+                          [&](int q) { return U[(int64_t)q * w + j]; });
         __syncthreads();
     }
-    // largest |X[i]| over the rows k..f-1 but s1 and s2, NaN-propagating (ldlt.jl:240-260)
-    __device__ __attribute__((always_inline)) double colmax(const T* X, int k, int s1, int s2) const {
-        double m = 0.0;
-        for (int i = k + threadIdx.x; i < f; i += NT)
-            if (i != s1 && i != s2) m = jmax(m, fabs((double)X[i]));
-        return block_jmax<NT>(m, *rb);
-    }
-    // the same for the current column j, formed by one wave (lanes along the rows)
-    __device__ __attribute__((always_inline)) double wave_colmax(int j, int k, int s1) const {
-        const int lane = threadIdx.x & 63, np = k - k0;
-        T uv[LP_MAXP];
+    // U rows n0..n1-1 (all of them 1x1 pivots) for the columns k0 + n1..w-1, the rows before n0 being
+    // there: a thread per column, eight rows at a time (all threads; ends with a barrier)
+    __device__ __attribute__((always_inline)) void form_urows(int n0, int n1) const {
+        for (int j = k0 + n1 + threadIdx.x; j < w; j += NT) {
+            const T* cj = P + (int64_t)j * f + k0;
+#pragma unroll 1
+            for (int b0 = n0; b0 < n1; b0 += 8) {
+                T a[8];
 #pragma unroll
-        for (int q = 0; q < LP_MAXP; ++q) uv[q] = q < np ? U[(int64_t)q * w + j] : T(0);
-        double m = 0.0;
-        const T* cj = P + (int64_t)j * f;
-        for (int i = k + lane; i < f; i += 64) {
-            T lv[LP_MAXP];
-            load_l(i, np, lv);
-            const T x = apply(cj[i], lv, [&](int q) { return uv[q]; });
-            if (i != s1) m = jmax(m, fabs((double)x));
-        }
-        return wave_jmax(m);
-    }
-    __device__ __attribute__((always_inline)) bool accept_1x1(const T* X, int c, int k, const LdltPrm& p) const {
-        const double d = fabs((double)X[c]);
-        if (!(d >= p.eps)) return false;
-        return d >= p.u * colmax(X, k, c, -1);
-    }
-    // the 2x2 block (k, r) from the current columns k (Xk) and r (Xr)
-    __device__ __attribute__((always_inline)) bool nonsingular_2x2(const T* Xk, const T* Xr, int k, int r, const LdltPrm& p) const {
-        const double akk = Xk[k], arr = Xr[r], akr = Xr[k], ark = Xk[r];
-        const double det = akk * arr - akr * ark;
-        const double mx = jmax(jmax(fabs(akk), fabs(ark)), fabs(arr));
-        return det != 0.0 && isfinite(det) && mx >= p.eps;
-    }
-    __device__ __attribute__((always_inline)) bool accept_2x2(const T* Xk, const T* Xr, int k, int r, const LdltPrm& p) const {
-        if (!nonsingular_2x2(Xk, Xr, k, r, p)) return false;
-        const double akk = Xk[k], arr = Xr[r], akr = Xr[k], ark = Xk[r];
-        const double det = akk * arr - akr * ark;
-        const double e11 = fabs(arr / det), e12 = fabs(akr / det), e21 = fabs(ark / det), e22 = fabs(akk / det);
-        const double m1 = colmax(Xk, k, k, r), m2 = colmax(Xr, k, r, k);
-        return p.u * (e11 * m1 + e21 * m2) <= 1.0 && p.u * (e12 * m1 + e22 * m2) <= 1.0;
-    }
-    // best_1x1 (ldlt.jl:264-276) on the current diagonal DG (formed here): the acceptable 1x1
-    // pivot of k..w-1 with the largest |a_jj|, first on ties, -1 if none. The largest
-    // candidate is tested first by the whole block (its column formed in X2, which holds it on
-    // return); else the candidates in sorted order, sixteen at a time, one wave per column.
-    __device__ __attribute__((always_inline)) int best_1x1(int k, const LdltPrm& p) const {
-        form_diag(k);
-        const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
-        double v = -1.0;
-        int bi = -1;
-        for (int j = k + tid; j < w; j += NT) {
-            const double a = fabs((double)DG[j]);
-            if (a >= p.eps && vi_better(a, j, v, bi)) {
-                v = a;
-                bi = j;
-            }
-        }
-        block_argmax<NT>(v, bi, *rb);
-        if (bi < 0) return -1;
-        form_col(bi, k, X2);
-        if (v >= p.u * colmax(X2, k, bi, -1)) return bi;
-        const int n = w - k;
-        if (n <= scap) {
-            int np = 1;
-            while (np < n) np <<= 1;
-            for (int q = tid; q < np; q += NT) {
-                double key = -1.0;
-                if (q < n) {
-                    const double a = fabs((double)DG[k + q]);
-                    key = a >= p.eps ? a : -1.0;
-                }
-                skey[q] = key;
-                sidx[q] = k + q;
-            }
-            __syncthreads();
-            for (int size = 2; size <= np; size <<= 1)
-                for (int stride = size >> 1; stride > 0; stride >>= 1) {
-                    for (int i = tid; i < np; i += NT) {
-                        const int l = i ^ stride;
-                        if (l <= i) continue;
-                        const bool lbefore = skey[l] > skey[i] || (skey[l] == skey[i] && sidx[l] < sidx[i]);
-                        const bool ibefore = skey[i] > skey[l] || (skey[i] == skey[l] && sidx[i] < sidx[l]);
-                        if ((i & size) == 0 ? lbefore : ibefore) {
-                            const double tk = skey[i];
-                            skey[i] = skey[l];
-                            skey[l] = tk;
-                            const int ti = sidx[i];
-                            sidx[i] = sidx[l];
-                            sidx[l] = ti;
+                for (int r = 0; r < 8; ++r) a[r] = cj[min(b0 + r, n1 - 1)];
+#pragma unroll 1
+                for (int q0 = 0; q0 < b0; q0 += 8) {
+                    T uv[9];
+#pragma unroll
+                    for (int q = 0; q < 9; ++q) uv[q] = U[(int64_t)min(q0 + q, b0 - 1) * w + j];
+#pragma unroll
+                    for (int q = 0; q < 8; ++q) {
+                        const int ct = q0 + q < b0 ? uni(ctype[q0 + q]) : 0;
+                        if (ct == 1) {
+#pragma unroll
+                            for (int r = 0; r < 8; ++r) a[r] = a[r] - Ls[min(b0 + r, n1 - 1)][q0 + q] * uv[q];
+                        } else if (ct == 2) {
+#pragma unroll
+                            for (int r = 0; r < 8; ++r)
+                                a[r] = a[r] - (Ls[min(b0 + r, n1 - 1)][q0 + q] * uv[q] +
+                                               Ls[min(b0 + r, n1 - 1)][q0 + q + 1] * uv[q + 1]);
                         }
                     }
-                    __syncthreads();
                 }
-            // the first entry is bi, already rejected
-            for (int base = 1; base < n && skey[base] >= 0.0; base += NT / 64) {
-                const int q = base + wv;
-                int found = 0x7fffffff;
-                if (q < n && skey[q] >= 0.0) {
-                    const int j = sidx[q];
-                    const double m = wave_colmax(j, k, j);
-                    if (skey[q] >= p.u * m) found = q;
-                }
-                if (lane == 0) rb->i[wv] = found;
-                __syncthreads();
-                int best = rb->i[0];
-                for (int w2 = 1; w2 < NT / 64; ++w2) best = min(best, rb->i[w2]);
-                __syncthreads();
-                if (best != 0x7fffffff) {
-                    const int j = sidx[best];
-                    form_col(j, k, X2);
-                    return j;
+#pragma unroll
+                for (int r = 0; r < 8; ++r) {
+                    if (b0 + r >= n1) break;
+                    U[(int64_t)(b0 + r) * w + j] = a[r];
+#pragma unroll
+                    for (int r2 = r + 1; r2 < 8; ++r2) a[r2] = a[r2] - Ls[min(b0 + r2, n1 - 1)][b0 + r] * a[r];
                 }
             }
-            return -1;
-        }
-        // too many candidates to sort: every column, one wave each; a column that cannot beat
-        // its wave's current best is not tested
-        double bv = 0.0;
-        int bj = -1;
-        for (int j = k + wv; j < w; j += NT / 64) {
-            const double a = fabs((double)DG[j]);
-            if (!(a >= p.eps)) continue;
-            if (bj >= 0 && !(a > bv)) continue;
-            if (!(a >= p.u * wave_colmax(j, k, j))) continue;
-            bv = a;
-            bj = j;
-        }
-        if (lane == 0) {
-            rb->v[wv] = bv;
-            rb->i[wv] = bj;
         }
         __syncthreads();
-        double rv = rb->v[0];
-        int ri = rb->i[0];
-        for (int q = 1; q < NT / 64; ++q)
-            if (vi_better(rb->v[q], rb->i[q], rv, ri)) {
-                rv = rb->v[q];
-                ri = rb->i[q];
-            }
-        __syncthreads();
-        if (ri >= 0) form_col(ri, k, X2);
-        return ri;
     }
-    // pivot choice at column k (ldlt.jl:280-325), as Front::choose on the current columns:
-    // c = pivot column, r = 2x2 partner or -1; on return the current column c is in *Xc (1x1),
-    // or the columns k and r are in X0 and X1 (2x2)
-    __device__ __attribute__((always_inline)) void choose(int k, const LdltPrm& p, int& c, int& r, T*& Xc) const {
-        r = -1;
-        form_col(k, k, X0);
-        Xc = X0;
-        if (p.pivot == PV_NONE) {
-            c = k;
-            return;
+    // the update of the pivot at q = k - k0 (1x1: its L column la; TWO: a 2x2's la and lb) on V's later
+    // columns, G columns in flight together
+    template <bool TWO>
+    __device__ __attribute__((always_inline)) void update_v(int q, const T (&la)[R], const T (&lb)[R]) const {
+        constexpr int G = R <= 3 ? 8 : R <= 6 ? 4 : R <= 12 ? 2 : 1;
+        const int n = min(MAXP - 1, w - k0) - q;  // V's columns inside the panel
+        const T* u0 = U + (int64_t)q * w + k0 + q;
+        for (int c0 = TWO ? 2 : 1; c0 < n; c0 += G) {
+            const auto rw = rows();
+            const int nf = rw.count(f);
+            T v[G][R], ua[G], ub[G];
+#pragma unroll
+            for (int g = 0; g < G; ++g) {
+                const int c = min(c0 + g, n - 1);
+                ua[g] = u0[c];
+                ub[g] = TWO ? u0[w + c] : T(0);
+#pragma unroll
+                for (int u = 0; u < R; ++u) v[g][u] = load_at(V + (int64_t)c * f, rw.clamped(u));
+            }
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int g = 0; g < G; ++g) {
+                if (c0 + g < n) {
+#pragma unroll
+                    for (int u = 0; u < R; ++u) {
+                        const T x = TWO ? v[g][u] - (la[u] * ua[g] + lb[u] * ub[g]) : v[g][u] - la[u] * ua[g];
+                        if (u < nf) store_at(V + (int64_t)(c0 + g) * f, rw.off(u), x);
+                    }
+                }
+            }
         }
-        if (p.pivot == PV_DIAG) {
-            if (accept_1x1(X0, k, k, p)) {
-                c = k;
-                return;
-            }
-            const int best = best_1x1(k, p);
-            if (best >= 0) {
-                c = best;
-                Xc = X2;
-                return;
-            }
-            // the largest diagonal entry, first on ties; a NaN |a_kk| keeps k (DG was formed by
-            // best_1x1)
-            double v = fabs((double)X0[k]);
-            int bi = k;
-            for (int j = k + 1 + threadIdx.x; j < w; j += NT) {
+    }
+    // best_1x1 (ldlt.jl:264-276) on the current diagonal (formed here): the acceptable 1x1 pivot of
+    // k..w-1 with the largest |a_jj|, first on ties, -1 if none: the candidates (|a_jj| >= eps) in
+    // that order, each one's current column formed in y (which holds the answer's on return) and
+    // tested by the whole block. The first one is usually the answer, and where none is, few are
+    // left (KKT, n = 12,000: the first of 367 of 619 searches, none of 6 candidates on average in 169).
+    __device__ __attribute__((always_inline)) int best_1x1(int k, const LdltPrm& p, T (&y)[R]) const {
+        form_diag(k);
+        double last = 0.0;
+        int lj = -1;
+        while (true) {
+            double v = -1.0;
+            int bi = -1;
+            for (int j = k + threadIdx.x; j < w; j += NT) {
                 const double a = fabs((double)DG[j]);
-                if (a > v) {
+                if (a >= p.eps && (lj < 0 || a < last || (a == last && j > lj)) && vi_better(a, j, v, bi)) {
                     v = a;
                     bi = j;
                 }
             }
             block_argmax<NT>(v, bi, *rb);
-            c = fabs((double)DG[bi]) >= p.eps ? bi : k;
-            if (c != k) {
-                form_col(c, k, X2);
-                Xc = X2;
+            bi = uni(bi);
+            if (bi < 0) return -1;
+            form_col(bi, k - k0, y);
+            if (uni(v >= p.u * colmax(y, k, f, bi, bi))) return bi;
+            last = v;
+            lj = bi;
+        }
+    }
+    // pivot choice at column k (ldlt.jl:280-325), as Front::choose on the current columns, column k
+    // in xa: c = pivot column, r = 2x2 partner or -1; on return the column c is in xa (1x1), or the
+    // columns k and r are in xa and xb (2x2)
+    __device__ __attribute__((always_inline)) void choose(int k, const LdltPrm& p, int& c, int& r, T (&xa)[R],
+                                                          T (&xb)[R]) const {
+        const int np = k - k0;
+        r = -1;
+        c = k;
+        if (p.pivot == PV_NONE) return;
+        pick(xa, k, 0);
+        T y[R];
+        if (p.pivot == PV_DIAG) {
+            const double m = colmax(xa, k, f, k, k);
+            const double akk = fabs(pk[0]);
+            if (uni(akk >= p.eps && akk >= p.u * m)) return;
+            int best = best_1x1(k, p, y);
+            if (best < 0) {
+                // the largest diagonal entry, first on ties; a NaN |a_kk| keeps k (DG was formed by
+                // best_1x1)
+                double v = akk;
+                int bi = k;
+                for (int j = k + 1 + threadIdx.x; j < w; j += NT) {
+                    const double a = fabs((double)DG[j]);
+                    if (a > v) {
+                        v = a;
+                        bi = j;
+                    }
+                }
+                block_argmax<NT>(v, bi, *rb);
+                best = uni(fabs((double)DG[bi]) >= p.eps ? bi : k);
+                if (best == k) return;
+                form_col(best, np, y);
             }
+            c = best;
+#pragma unroll
+            for (int u = 0; u < R; ++u) xa[u] = y[u];
             return;
         }
         const double alpha = (1.0 + sqrt(17.0)) / 8.0;  // Bunch-Kaufman constant (ldlt.jl:22)
         double lambda = 0.0;
         int rr = -1;
-        for (int i = k + 1 + threadIdx.x; i < w; i += NT) {
-            const double a = fabs((double)X0[i]);
-            if (a > lambda) {
-                lambda = a;
-                rr = i;
+        {
+            const int n = rows().count(w);
+            const bool up = (int)threadIdx.x > k - k0;
+#pragma unroll
+            for (int u = 0; u < R; ++u) {
+                const double a = fabs((double)xa[u]);
+                if (u < n && (u > 0 || up) && a > lambda) {
+                    lambda = a;
+                    rr = u;
+                }
             }
+            if (rr >= 0) rr = k0 + (int)threadIdx.x + NT * rr;
         }
         block_argmax<NT>(lambda, rr, *rb);
+        rr = uni(rr);
         if (rr < 0) lambda = 0.0;
-        const double akk = fabs((double)X0[k]);
-        int bc = k, br = -1;
-        T* Xb = X0;
-        if (rr < 0 || akk >= alpha * lambda) {
-            bc = k;
+        const double akk = fabs(pk[0]);
+        const double mk = colmax(xa, k, f, k, k);
+        bool ok, two = false;
+        double det = 0.0, mx = 0.0;
+        if (rr < 0 || uni(akk >= alpha * lambda)) {
+            ok = akk >= p.eps && akk >= p.u * mk;
         } else {
-            form_col(rr, k, X1);
-            double sigma = 0.0;
-            for (int i = k + threadIdx.x; i < w; i += NT)
-                if (i != rr) sigma = jmax(sigma, fabs((double)X1[i]));
-            sigma = block_jmax<NT>(sigma, *rb);
-            if (akk * sigma >= alpha * lambda * lambda) {
-                bc = k;
-            } else if (fabs((double)X1[rr]) >= alpha * sigma) {
-                bc = rr;
-                Xb = X1;
+            form_col(rr, np, xb);
+            pick(xa, rr, 1);
+            pick(xb, k, 2);
+            pick(xb, rr, 3);
+            const double sigma = colmax(xb, k, w, rr, rr);
+            const double arr = pk[3], ark = pk[1], akr = pk[2];
+            if (uni(akk * sigma >= alpha * lambda * lambda)) {
+                ok = akk >= p.eps && akk >= p.u * mk;
+            } else if (uni(fabs(arr) >= alpha * sigma)) {
+                c = rr;
+                ok = fabs(arr) >= p.eps && fabs(arr) >= p.u * colmax(xb, k, f, rr, rr);
             } else {
-                bc = k;
-                br = rr;
+                two = true;
+                det = pk[0] * arr - akr * ark;
+                mx = jmax(jmax(akk, fabs(ark)), fabs(arr));
+                ok = det != 0.0 && isfinite(det) && mx >= p.eps;
+                if (uni(ok)) {
+                    const double e11 = fabs(arr / det), e12 = fabs(akr / det), e21 = fabs(ark / det),
+                                 e22 = fabs(pk[0] / det);
+                    const double m1 = colmax(xa, k, f, k, rr), m2 = colmax(xb, k, f, rr, k);
+                    ok = p.u * (e11 * m1 + e21 * m2) <= 1.0 && p.u * (e12 * m1 + e22 * m2) <= 1.0;
+                }
             }
         }
-        const bool ok = br < 0 ? accept_1x1(Xb, bc, k, p) : accept_2x2(X0, X1, k, br, p);
-        if (ok) {
-            c = bc;
-            r = br;
-            Xc = Xb;
-            return;
+        if (!uni(ok)) {
+            const int best = best_1x1(k, p, y);
+            if (best >= 0) {
+                c = best;
+#pragma unroll
+                for (int u = 0; u < R; ++u) xa[u] = y[u];
+                return;
+            }
+            two = uni(two && det != 0.0 && isfinite(det) && mx >= p.eps);  // (a singular 2x2: k as a 1x1)
         }
-        const int best = best_1x1(k, p);
-        if (best >= 0) {
-            c = best;
-            Xc = X2;
-            return;
+        if (two) {
+            r = rr;
+        } else if (c != k) {
+#pragma unroll
+            for (int u = 0; u < R; ++u) xa[u] = xb[u];
         }
-        if (br >= 0 && nonsingular_2x2(X0, X1, k, br, p)) {
-            c = bc;
-            r = br;
-            return;
-        }
-        c = bc;
-        Xc = Xb;
     }
-    // symmetric interchange of positions a and b (ldlt.jl:328-340) on the stored values, the
-    // pivot rows' entries of those columns, and the rows of the current columns held in Xa, Xb
-    __device__ __attribute__((always_inline)) void swap(int a, int b, int k, T* Xa, T* Xb) const {
-        __syncthreads();  // the pivot choice's last reads are done
+    // symmetric interchange of the positions a (the pivot position, whose column is written next)
+    // and b (ldlt.jl:328-340): the stored column of a moves to b, the rows a and b of every other
+    // stored column, of V and of the columns in registers are exchanged, and the pivot rows' entries
+    // (xa, with TWO also xb; np pivots taken, the current pivot is k0 + np; ends with a barrier)
+    template <bool TWO>
+    __device__ __attribute__((always_inline)) void swap(int a, int b, int np, T (&xa)[R], T (&xb)[R]) const {
         if (a == b) return;
-        for (int i = threadIdx.x; i < f; i += NT) {
-            const T t = P[(int64_t)a * f + i];
-            P[(int64_t)a * f + i] = P[(int64_t)b * f + i];
-            P[(int64_t)b * f + i] = t;
-        }
-        for (int q = threadIdx.x; q < k - k0; q += NT) {
+        pick(xa, a, 0);
+        pick(xa, b, 1);
+        const int kv = k0 + np;
+        T col[R];
+        load_rows(P + (int64_t)a * f, col);
+        for (int q = threadIdx.x; q < np; q += NT) {
             const T t = U[(int64_t)q * w + a];
             U[(int64_t)q * w + a] = U[(int64_t)q * w + b];
             U[(int64_t)q * w + b] = t;
         }
+        store_rows(P + (int64_t)b * f, col);
+        if (b < k0 + MAXP - 1) {
+            load_rows(V + (int64_t)(a - kv) * f, col);
+            store_rows(V + (int64_t)(b - kv) * f, col);
+        }
         __syncthreads();
+        for (int c = threadIdx.x; c < MAXP - 1; c += NT) {
+            const T t = V[(int64_t)c * f + a];
+            V[(int64_t)c * f + a] = V[(int64_t)c * f + b];
+            V[(int64_t)c * f + b] = t;
+        }
+        exchange(xa, a, b, 0, 1);
+        if (TWO) {
+            pick(xb, a, 2);
+            pick(xb, b, 3);
+            __syncthreads();
+            exchange(xb, a, b, 2, 3);
+        }
         for (int j = threadIdx.x; j < w; j += NT) {
             const T t = P[(int64_t)j * f + a];
             P[(int64_t)j * f + a] = P[(int64_t)j * f + b];
@@ -1197,38 +1344,296 @@ struct PanelFront {
             const int t = lp[a];
             lp[a] = lp[b];
             lp[b] = t;
-            if (Xa) {
-                const T x = Xa[a];
-                Xa[a] = Xa[b];
-                Xa[b] = x;
-            }
-            if (Xb) {
-                const T x = Xb[a];
-                Xb[a] = Xb[b];
-                Xb[b] = x;
-            }
         }
         __syncthreads();
     }
 };
 
-// panel e of every large front of a level: its pivots until LP_NB columns are taken or the
-// front is done (the first panel also sets up the front). task: (s, scratch offset)
+// N values computed here, not where they are used next (empty asm statements, which also order the
+// memory accesses around them): without it the register allocator meets the loads of a whole panel
+// update before the first of its sums, and the panel spills
+template <int N, typename T>
+__device__ __attribute__((always_inline)) inline void pin(T* v) {
+#pragma unroll
+    for (int c = 0; c < N; ++c) asm volatile("" : "+v"(v[c])::"memory");
+}
+// x[c - 1] = x[c] - l u[c] for 1 <= c < W: a row's rank-1 update, each column moving one register left;
+// eight entries of u in flight together
+template <int W, int C0 = 1, int N, typename T>
+__device__ __attribute__((always_inline)) inline void shift_update(T (&x)[N], T l, const T* u) {
+    constexpr int C1 = C0 + 8 < W ? C0 + 8 : W;
+#pragma unroll
+    for (int c = C0; c < C1; ++c) x[c - 1] = x[c] - l * u[c];
+    pin<C1 - C0>(x + C0 - 1);
+    if constexpr (C1 < W) shift_update<W, C1>(x, l, u);
+}
+
+// the state of a panel's usual pivots
+template <typename T, int R, int NBP>
+struct PanelRegs {
+    T x[R][NBP];  // x[u][c] = entry (k0 + tid + NT u, k + c)
+    int nr;       // row slots in use
+    int buf;
+    int npos, nneg;
+};
+
+// usual pivots k, k + 1, ... of the panel while the panel's remaining columns number more than W - 8
+// (of W registers per row); false: column k is not its own acceptable 1x1 pivot
+template <typename T, int NT, int R, int NBP, int W, class Z>
+__device__ __attribute__((always_inline)) inline bool panel_pivots(PanelRegs<T, R, NBP>& X, const Z& F, int& k, int kend,
+                                                                   const LdltPrm& p, double (*red)[NT / 64][2],
+                                                                   T (*urow)[NBP], int8_t* kind, T* dd) {
+    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6, f = F.f, w = F.w, k0 = F.k0;
+    const double alpha = (1.0 + sqrt(17.0)) / 8.0;  // Bunch-Kaufman constant (ldlt.jl:22)
+    const int kstop = min(kend, k0 + NBP - (W > 8 ? W - 8 : 0));
+    while (k < kstop) {
+        // the largest |a_ik| below the pivot: fully summed rows, then the others
+        double lam = 0.0, mx = 0.0;
+        bool nan = false;
+        const auto rw = F.rows();
+        const int nf = rw.count(f), nw = rw.count(w);
+        const bool up = tid > k - k0;  // (the pivot's row is among the first slot's)
+#pragma unroll
+        for (int u = 0; u < R; ++u) {
+            if (u < X.nr) {  // (only the last slot can hold rows past the front's end)
+                double a = (double)X.x[u][0];
+                if (u == 0) a = up ? a : 0.0;
+                if (u + 1 == X.nr) a = u < nf ? a : 0.0;
+                nan |= a != a;
+                mx = max_abs(mx, a);
+                if (NT * u < w - k0) lam = max_abs(lam, u < nw ? a : 0.0);
+            }
+        }
+        lam = wave_max_last(lam);
+        mx = wave_max_last(mx);
+        if (__any(nan)) mx = __builtin_nan("");
+        X.buf ^= 1;
+        if (lane == 63) {
+            red[X.buf][wv][0] = lam;
+            red[X.buf][wv][1] = mx;
+        }
+        if (tid == k - k0) {
+#pragma unroll
+            for (int c = 0; c < W; ++c) urow[X.buf][c] = X.x[0][c];
+        }
+        __syncthreads();  // (waits for LDS only: the L columns' stores stay in flight)
+        nan = false;
+        lam = 0.0;
+        mx = 0.0;
+#pragma unroll
+        for (int q = 0; q < NT / 64; ++q) {
+            lam = max_abs(lam, red[X.buf][q][0]);
+            const double v = red[X.buf][q][1];
+            nan |= v != v;
+            mx = max_abs(mx, v);
+        }
+        const T d = urow[X.buf][0];
+        const double akk = fabs((double)d);
+        bool fast = akk >= p.eps && d != T(0);
+        if (p.pivot != PV_NONE) fast = fast && !nan && akk >= p.u * mx;
+        if (p.pivot == PV_BK) fast = fast && akk >= alpha * lam;
+        if (!uni(fast)) return false;
+        T* col = F.P + (int64_t)k * f;
+        // the scaling of three row slots at a time (independent divisions), then their updates
+#pragma unroll
+        for (int u0 = 0; u0 < R; u0 += 3) {
+            if (u0 < X.nr) {
+                T l[3] = {};
+#pragma unroll
+                for (int u = 0; u < 3 && u0 + u < R; ++u) l[u] = X.x[u0 + u][0] / d;
+                pin<3>(l);
+#pragma unroll
+                for (int u = 0; u < 3 && u0 + u < R; ++u) {
+                    if (u0 + u < nf && (u0 + u > 0 || up)) store_at(col, rw.off(u0 + u), l[u]);
+                    if (u0 + u == 0 && up && tid < NBP) F.Ls[tid][k - k0] = l[0];
+                    shift_update<W>(X.x[u0 + u], l[u], urow[X.buf]);
+                }
+            }
+        }
+        if (tid == 0) {
+            kind[k] = KIND_1X1;
+            dd[k] = d;
+            F.ctype[k - k0] = 1;
+        }
+        if (d > T(0))
+            X.npos++;
+        else
+            X.nneg++;
+        ++k;
+    }
+    return true;
+}
+
+// the LDS words of a panel
+template <typename T, int NBP>
+struct PanelLds {
+    RedBuf<512> rb;
+    double pk[4];
+    int ctype[NBP + 1];
+    T Uc[NBP + 1], Lr[NBP + 1];
+    T Ls[NBP + 1][NBP + 1];
+    __align__(16) double red[2][512 / 64][2];
+    __align__(16) T urow[2][NBP];
+};
+template <typename T, int NBP>
+__device__ inline PanelLds<T, NBP>& panel_lds() {
+    __shared__ PanelLds<T, NBP> lds;
+    return lds;
+}
+
+// a front's arrays during a panel
 template <typename T>
-__global__ void __launch_bounds__(512) k_ldlt_panel(DevSym S, const Task* __restrict__ tasks, int e,
+struct PanelArgs {
+    T *P, *U, *dd, *ee;
+    int f, w, k0;
+    int* lp;
+    int8_t* kind;
+    int64_t* st;
+    const int8_t* sreq_row;
+    const int32_t* perm_c0;
+    LdltPrm prm;
+};
+template <typename T, int R, int NBP>
+__device__ __attribute__((always_inline)) inline PanelFront<T, 512, R, NBP + 1> panel_front(const PanelArgs<T>& A) {
+    PanelLds<T, NBP>& S = panel_lds<T, NBP>();
+    T* DG = A.U + (int64_t)LP_MAXP * A.w;
+    return PanelFront<T, 512, R, NBP + 1>{A.P,     A.f,     A.w,  A.k0, A.lp, &S.rb, A.U, DG, DG + A.w,
+                                          S.ctype, S.Uc, S.Lr, S.Ls, S.pk};
+}
+
+// any pivot but the usual one, at column k, from the panel memory (V holds the panel's columns from k
+// on, nu pivot rows are formed); returns the next column. A function of its own: the panel's
+// registers are free while it runs.
+template <typename T, int R, int NBP>
+__device__ __attribute__((noinline)) int panel_general(const PanelArgs<T> A,
+                                                                                             int k, int nu) {
+    const auto Z = panel_front<T, R, NBP>(A);
+    const int tid = threadIdx.x, f = uni(A.f), k0 = uni(A.k0);
+    const LdltPrm& prm = A.prm;
+    T* P = A.P;
+    T *dd = A.dd, *ee = A.ee;
+    int* lp = A.lp;
+    int* ctype = Z.ctype;
+    double* pk = Z.pk;
+    int8_t* kind = A.kind;
+    int64_t* st = A.st;
+    const int8_t* sreq_row = A.sreq_row;
+    const int32_t* perm_c0 = A.perm_c0;
+    T xa[R], xb[R];
+    Z.load_rows(Z.V, xa);
+    if (nu < k - k0) Z.form_urows(nu, k - k0);
+    int c, r;
+    Z.choose(k, prm, c, r, xa, xb);
+    __syncthreads();
+    T* ck = P + (int64_t)k * f;
+    if (r < 0) {
+        Z.template swap<false>(k, c, k - k0, xa, xb);
+        Z.pick(xa, k, 0);
+        __syncthreads();
+        if (tid == 0) {
+            double d = pk[0];
+            int8_t kd = KIND_1X1;
+            if (!(fabs(d) >= prm.eps) || d == 0.0) {
+                if (d == 0.0) st[ST_NZERO]++;
+                const int req = sreq_row ? (int)sreq_row[perm_c0[lp[k]]] : 0;
+                const double sg = req != 0 ? (double)req : (d < 0.0 ? -1.0 : 1.0);
+                d = sg * prm.eps;
+                kd = KIND_PERTURBED;
+                st[ST_NPERT]++;
+                if (d == 0.0 && st[ST_INFO] == 0) st[ST_INFO] = lp[k] + 1;
+            }
+            ck[k] = T(d);
+            kind[k] = kd;
+            dd[k] = T(d);
+            if (d > 0.0)
+                st[ST_NPOS]++;
+            else if (d < 0.0)
+                st[ST_NNEG]++;
+            pk[1] = d;
+            ctype[k - k0] = 0;
+        }
+        __syncthreads();
+        const T d = T(pk[1]);
+        const auto rw = Z.rows();
+        const int nf = rw.count(f);
+#pragma unroll
+        for (int u = 0; u < R; ++u) {
+            xa[u] = xa[u] / d;
+            if (u < nf && (u > 0 || tid > k - k0)) store_at(ck, rw.off(u), xa[u]);
+        }
+        Z.form_urow(k, k + 1);
+        Z.template update_v<false>(k - k0, xa, xb);
+        if (tid == 0) ctype[k - k0] = 1;
+        k += 1;
+    } else {
+        Z.template swap<true>(k + 1, r, k - k0, xa, xb);
+        Z.pick(xa, k, 0);
+        Z.pick(xa, k + 1, 1);
+        Z.pick(xb, k + 1, 2);
+        __syncthreads();
+        const T a = T(pk[0]), b = T(pk[1]), c2 = T(pk[2]);
+        const T up = b;
+        const T det = a * c2 - up * b;
+        const T e11 = c2 / det, e12 = -up / det, e21 = -b / det, e22 = a / det;
+        if (tid == 0) {
+            kind[k] = KIND_2X2_FIRST;
+            kind[k + 1] = KIND_2X2_SECOND;
+            dd[k] = a;
+            dd[k + 1] = c2;
+            ee[k] = b;
+            st[ST_N2X2]++;
+            if (det < T(0)) {
+                st[ST_NPOS]++;
+                st[ST_NNEG]++;
+            } else if (a > T(0)) {
+                st[ST_NPOS] += 2;
+            } else {
+                st[ST_NNEG] += 2;
+            }
+            ck[k] = a;
+            ck[f + k + 1] = c2;
+            ck[k + 1] = T(0);  // the reference clears it
+        }
+        const auto rw = Z.rows();
+        const int nf = rw.count(f);
+#pragma unroll
+        for (int u = 0; u < R; ++u) {
+            const T x1 = xa[u], x2 = xb[u];
+            xa[u] = x1 * e11 + x2 * e21;
+            xb[u] = x1 * e12 + x2 * e22;
+            if (u < nf && (u > 0 || tid > k + 1 - k0)) {
+                store_at(ck, rw.off(u), xa[u]);
+                store_at(ck + f, rw.off(u), xb[u]);
+            }
+        }
+        Z.form_urow(k, k + 2);
+        Z.form_urow(k + 1, k + 2);
+        Z.template update_v<true>(k - k0, xa, xb);
+        if (tid == 0) {
+            ctype[k - k0] = 2;
+            ctype[k + 1 - k0] = 3;
+        }
+        k += 2;
+    }
+    __syncthreads();
+    return k;
+}
+
+// the next panel of every large front of a level: its pivots until NBP columns are taken or the
+// front is done (the first panel also sets up the front; the upper triangle of the fully summed
+// square was mirrored by k_ldlt_mirror). task: (s, scratch offset).
+//
+// Bound: latency, one workgroup per front walks the pivots one after another. NT = 512 (two waves
+// per SIMD) leaves 256 registers a thread, 192 of them for the panel: NBP R <= 96.
+template <typename T, int R, int NBP>
+__global__ void __launch_bounds__(512) k_ldlt_panel(DevSym S, const Task* __restrict__ tasks, int first,
                                                     T* __restrict__ factor, T* __restrict__ dvec,
                                                     int32_t* __restrict__ piv, int8_t* __restrict__ pkind,
                                                     int64_t* __restrict__ stats, int32_t* __restrict__ lstep,
                                                     T* __restrict__ scratch, LdltPrm prm, int scaled,
                                                     const double* __restrict__ aux, const int8_t* __restrict__ psign) {
     constexpr int NT = 512;
-    constexpr int SCAP = 2048;
-    __shared__ RedBuf<NT> rb;
-    __shared__ double sh[4];
-    __shared__ double skey[SCAP];
-    __shared__ int sidx[SCAP];
-    __shared__ int ctype[LP_MAXP];
-    __shared__ T Uc[LP_MAXP], Lr[LP_MAXP];
+    constexpr int MAXP = NBP + 1;
     const Task tk = tasks[blockIdx.x];
     const int s = tk.s;
     const int f = S.fnrows[s], w = S.fncols[s];
@@ -1243,137 +1648,106 @@ __global__ void __launch_bounds__(512) k_ldlt_panel(DevSym S, const Task* __rest
     int64_t* st = stats + (int64_t)s * NF;
     int32_t* ls = lstep + 3 * s;
     int k;
-    if (e == 0) {
+    if (first) {
         for (int q = tid; q < w; q += NT) {
             lp[q] = q;
             kind[q] = 0;
             dd[q] = ee[q] = T(0);
         }
         if (tid < NF) st[tid] = 0;
-        // the upper triangle of the fully summed square mirrors the lower (the reference's
-        // full square)
-        for (int q = tid; q < w * w; q += NT) {
-            const int j = q / w, i = q - j * w;
-            if (i > j) P[(int64_t)i * f + j] = P[(int64_t)j * f + i];
-        }
         k = 0;
     } else {
-        k = ls[2];
+        k = uni(ls[2]);
     }
     __syncthreads();
     if (k >= w) {
         if (tid == 0) ls[1] = 0;
         return;
     }
-    const int k0 = k;
-    for (int q = tid; q < LP_MAXP; q += NT) ctype[q] = 0;
+    const int k0 = k, kend = min(w, k0 + NBP);
+    PanelLds<T, NBP>& D = panel_lds<T, NBP>();
+    auto& Ls = D.Ls;
+    for (int q = tid; q < MAXP; q += NT) D.ctype[q] = 0;
     T* base = scratch + tk.a;
-    PanelFront<T, NT> Z{P, f, w, k0, lp, &rb, base, base + f, base + 2 * (int64_t)f, base + 3 * (int64_t)f,
-                        base + 3 * (int64_t)f + (int64_t)LP_MAXP * w, ctype, Uc, Lr, skey, sidx, SCAP};
-    const int8_t* sreq_row = psign;
-    const int32_t* perm_c0 = S.perm + c0;
-    __syncthreads();
-    while (k < w && k - k0 < LP_NB) {
-        int c, r;
-        T* Xc;
-        Z.choose(k, prm, c, r, Xc);
-        if (r < 0) {
-            Z.swap(k, c, k, Xc, nullptr);
-            if (tid == 0) {
-                double d = (double)Xc[k];
-                int8_t kd = KIND_1X1;
-                if (!(fabs(d) >= prm.eps) || d == 0.0) {
-                    if (d == 0.0) st[ST_NZERO]++;
-                    const int req = sreq_row ? (int)sreq_row[perm_c0[lp[k]]] : 0;
-                    const double sg = req != 0 ? (double)req : (d < 0.0 ? -1.0 : 1.0);
-                    d = sg * prm.eps;
-                    kd = KIND_PERTURBED;
-                    st[ST_NPERT]++;
-                    if (d == 0.0 && st[ST_INFO] == 0) st[ST_INFO] = lp[k] + 1;
-                }
-                P[(int64_t)k * f + k] = T(d);
-                kind[k] = kd;
-                dd[k] = T(d);
-                ee[k] = T(0);
-                if (d > 0.0)
-                    st[ST_NPOS]++;
-                else if (d < 0.0)
-                    st[ST_NNEG]++;
-                sh[0] = d;
-            }
-            __syncthreads();
-            const T d = T(sh[0]);
-            for (int i = k + 1 + tid; i < f; i += NT) P[(int64_t)k * f + i] = Xc[i] / d;
-            __syncthreads();
-            Z.form_urow(k, k + 1);
-            if (tid == 0) ctype[k - k0] = 1;
-            __syncthreads();
-            k += 1;
-        } else {
-            Z.swap(k + 1, r, k, Z.X0, Z.X1);
-            if (tid == 0) {
-                const T a = Z.X0[k], b = Z.X0[k + 1], c2 = Z.X1[k + 1];
-                const T up = b;
-                const T det = a * c2 - up * b;
-                sh[0] = (double)(c2 / det);
-                sh[1] = (double)(-up / det);
-                sh[2] = (double)(-b / det);
-                sh[3] = (double)(a / det);
-                kind[k] = KIND_2X2_FIRST;
-                kind[k + 1] = KIND_2X2_SECOND;
-                dd[k] = a;
-                dd[k + 1] = c2;
-                ee[k] = b;
-                ee[k + 1] = T(0);
-                st[ST_N2X2]++;
-                if (det < T(0)) {
-                    st[ST_NPOS]++;
-                    st[ST_NNEG]++;
-                } else if (a > T(0)) {
-                    st[ST_NPOS] += 2;
-                } else {
-                    st[ST_NNEG] += 2;
-                }
-                P[(int64_t)k * f + k] = a;
-                P[(int64_t)(k + 1) * f + k + 1] = c2;
-                P[(int64_t)k * f + k + 1] = T(0);  // the reference clears it
-            }
-            __syncthreads();
-            const T e11 = T(sh[0]), e12 = T(sh[1]), e21 = T(sh[2]), e22 = T(sh[3]);
-            for (int i = k + 2 + tid; i < f; i += NT) {
-                const T x1 = Z.X0[i], x2 = Z.X1[i];
-                P[(int64_t)k * f + i] = x1 * e11 + x2 * e21;
-                P[(int64_t)(k + 1) * f + i] = x1 * e12 + x2 * e22;
-            }
-            __syncthreads();
-            Z.form_urow(k, k + 2);
-            Z.form_urow(k + 1, k + 2);
-            if (tid == 0) {
-                ctype[k - k0] = 2;
-                ctype[k + 1 - k0] = 3;
-            }
-            __syncthreads();
-            k += 2;
+    const PanelArgs<T> A{P, base, dd, ee, f, w, k0, lp, kind, st, psign, S.perm + c0, prm};
+    const auto Z = panel_front<T, R, NBP>(A);
+    const int nr = (f - k0 + NT - 1) / NT;
+    int nu = 0;  // U rows formed
+    int kv = k0;  // the last general pivot
+    int npos = 0, nneg = 0;
+    while (k < kend) {
+        __syncthreads();
+        PanelRegs<T, R, NBP> X;
+        X.nr = nr;
+        X.buf = 0;
+        X.npos = X.nneg = 0;
+        // the panel's columns k.. in registers: the stored values, or after a general pivot V's
+        const int np = k - k0, last = k - kv;  // (last: columns of that pivot, 0 at the panel's start)
+        for (int q = tid; q < MAXP * np; q += NT) {
+            const int pp = q / MAXP, r = q - pp * MAXP;
+            if (r > pp && k0 + r < f) Ls[r][pp] = P[(int64_t)(k0 + pp) * f + k0 + r];
         }
+        const T* src = last ? Z.V + (int64_t)last * f : P + (int64_t)k * f;
+        const int cmax = last ? NBP - 1 - last : w - 1 - k;
+        {
+            const auto rw = Z.rows();
+#pragma unroll
+            for (int u = 0; u < R; ++u) {
+                const uint32_t off = rw.clamped(u);
+#pragma unroll
+                for (int c = 0; c < NBP; ++c) X.x[u][c] = load_at(src + (int64_t)max(min(c, cmax), 0) * f, off);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        }
+        __syncthreads();
+        bool go = true;
+        if constexpr (NBP > 8) go = panel_pivots<T, NT, R, NBP, NBP>(X, Z, k, kend, prm, D.red, D.urow, kind, dd);
+        if (go) go = panel_pivots<T, NT, R, NBP, (NBP < 8 ? NBP : 8)>(X, Z, k, kend, prm, D.red, D.urow, kind, dd);
+        __syncthreads();  // the L columns are stored, the LDS words of the last pivot read
+        npos += X.npos;
+        nneg += X.nneg;
+        if (go) break;
+        // any other pivot, from the panel memory
+        kv = k;
+        {
+            const auto rw = Z.rows();
+            const int nf = rw.count(f);
+#pragma unroll
+            for (int u = 0; u < R; ++u) {
+                if (u < nf) {
+#pragma unroll
+                    for (int c = 0; c < NBP; ++c) store_at(Z.V + (int64_t)c * f, rw.off(u), X.x[u][c]);
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        }
+        __syncthreads();
+        k = uni(panel_general<T, R, NBP>(A, k, nu));
+        nu = k - k0;
     }
+    // the rest of the pivot rows for the columns after the panel
+    if (nu < k - k0 && k < w) Z.form_urows(nu, k - k0);
     if (tid == 0) {
+        st[ST_NPOS] += npos;
+        st[ST_NNEG] += nneg;
         ls[0] = k0;
         ls[1] = k - k0;
         ls[2] = k;
     }
 }
 
-// the update of panel e's pivots on the columns after it: the tile rows [I0, I0 + 64) x columns
+// the update of a panel's pivots on the columns after it: the tile rows [I0, I0 + 64) x columns
 // [J0, J0 + 64) of the entries at or after the panel's end (every row below, the fully summed
 // square's upper mirror included), each entry applying the panel's pivots in order as ldlt_front
-// does. task: (s, I0, J0, scratch offset)
+// does. task: (s, I0, J0, scratch offset). Lanes along the rows, sixteen columns a wave: the
+// thread's sixteen entries are loaded together, its row of L eight pivots at a time, the U rows
+// come from LDS by broadcast. Bound: HBM / L2 (two accesses per entry and panel).
 template <typename T>
 __global__ void __launch_bounds__(256) k_ldlt_trail(DevSym S, const Task* __restrict__ tasks, T* __restrict__ factor,
                                                    const int8_t* __restrict__ pkind, const int32_t* __restrict__ lstep,
                                                    const T* __restrict__ scratch) {
-    __shared__ T Ls[LP_MAXP][TILE];
-    __shared__ T Us[LP_MAXP][TILE];
-    __shared__ int stp[LP_MAXP], ssz[LP_MAXP], nsh;
+    __shared__ __align__(16) T Us[LP_MAXP][TILE];
+    __shared__ int8_t ks[LP_MAXP + 1];
     const Task t = tasks[blockIdx.x];
     const int s = t.s, f = S.fnrows[s], w = S.fncols[s];
     const int32_t* ls = lstep + 3 * s;
@@ -1381,49 +1755,46 @@ __global__ void __launch_bounds__(256) k_ldlt_trail(DevSym S, const Task* __rest
     if (np == 0) return;
     const int k0 = ls[0], kend = ls[2];
     const int I0 = t.a, J0 = t.b;
-    if (I0 + TILE <= kend || J0 + TILE <= kend || I0 >= f || J0 >= w) return;
-    const T* P = factor + S.panel_off[s];
-    T* Pw = factor + S.panel_off[s];
+    if (I0 + TILE <= kend || J0 + TILE <= kend) return;
+    T* P = factor + S.panel_off[s];
     const int8_t* kind = pkind + S.super_ptr[s];
-    const T* U = scratch + t.c + 3 * (int64_t)f;
-    const int tid = threadIdx.x;
+    const T* U = scratch + t.c;
+    const int tid = threadIdx.x, i = I0 + (tid & 63), ic = min(i, f - 1), cb = (tid >> 6) * 16;
     for (int q = tid; q < np * TILE; q += 256) {
         const int pp = q / TILE, c = q - pp * TILE;
-        const int i = I0 + c, j = J0 + c;
-        Ls[pp][c] = i < f ? P[(int64_t)(k0 + pp) * f + i] : T(0);
-        Us[pp][c] = j < w ? U[(int64_t)pp * w + j] : T(0);
+        Us[pp][c] = U[(int64_t)pp * w + min(J0 + c, w - 1)];
     }
-    if (tid == 0) {
-        int n = 0;
-        for (int p = k0; p < kend; ++p) {
-            if (kind[p] == KIND_2X2_SECOND) continue;
-            stp[n] = p - k0;
-            ssz[n] = kind[p] == KIND_2X2_FIRST ? 2 : 1;
-            ++n;
-        }
-        nsh = n;
-    }
+    if (tid < np) ks[tid] = kind[k0 + tid];
+    T x[16];
+#pragma unroll
+    for (int c = 0; c < 16; ++c) x[c] = P[(int64_t)min(J0 + cb + c, w - 1) * f + ic];
     __syncthreads();
-    const int ns = nsh;
-    const int tx = tid & 15, ty = tid >> 4;
+    const T* Li = P + (int64_t)k0 * f + ic;
+    for (int q0 = 0; q0 < np; q0 += 8) {
+        T l[9];  // (one past the eight: the second column of a 2x2 pivot)
 #pragma unroll
-    for (int a = 0; a < 4; ++a) {
-        const int r = 4 * ty + a, i = I0 + r;
-        if (i < kend || i >= f) continue;
+        for (int q = 0; q < 9; ++q) l[q] = Li[(int64_t)min(q0 + q, np - 1) * f];
+        __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int b = 0; b < 4; ++b) {
-            const int c = 4 * tx + b, j = J0 + c;
-            if (j < kend || j >= w) continue;
-            T x = P[(int64_t)j * f + i];
-            for (int q = 0; q < ns; ++q) {
-                const int pp = stp[q];
-                if (ssz[q] == 1)
-                    x = x - Ls[pp][r] * Us[pp][c];
-                else
-                    x = x - (Ls[pp][r] * Us[pp][c] + Ls[pp + 1][r] * Us[pp + 1][c]);
+        for (int q = 0; q < 8; ++q) {
+            if (q0 + q >= np) break;
+            const int kd = ks[q0 + q];
+            if (kd == KIND_2X2_SECOND) continue;
+            if (kd == KIND_2X2_FIRST) {
+#pragma unroll
+                for (int c = 0; c < 16; ++c)
+                    x[c] = x[c] - (l[q] * Us[q0 + q][cb + c] + l[q + 1] * Us[q0 + q + 1][cb + c]);
+            } else {
+#pragma unroll
+                for (int c = 0; c < 16; ++c) x[c] = x[c] - l[q] * Us[q0 + q][cb + c];
             }
-            Pw[(int64_t)j * f + i] = x;
         }
+    }
+    if (i < kend || i >= f) return;
+#pragma unroll
+    for (int c = 0; c < 16; ++c) {
+        const int j = J0 + cb + c;
+        if (j >= kend && j < w) P[(int64_t)j * f + i] = x[c];
     }
 }
 
@@ -1586,12 +1957,19 @@ void launch_ldlt_pivot(hipStream_t st, const DevSym& S, const Task* tasks, int n
 }
 
 template <typename T>
-void launch_ldlt_panel(hipStream_t st, const DevSym& S, const Task* tasks, int n, int e, T* factor, T* dvec,
-                       int32_t* piv, int8_t* kind, int64_t* stats, int32_t* lstep, T* scratch, int pivot, double u,
-                       double eps, int scaled, const double* aux, const int8_t* psign) {
+void launch_ldlt_panel(hipStream_t st, const DevSym& S, const Task* tasks, int n, int first, int cols, T* factor,
+                       T* dvec, int32_t* piv, int8_t* kind, int64_t* stats, int32_t* lstep, T* scratch, int pivot,
+                       double u, double eps, int scaled, const double* aux, const int8_t* psign) {
     LdltPrm p{pivot, u, eps};
-    hipLaunchKernelGGL(k_ldlt_panel<T>, dim3(n), dim3(512), 0, st, S, tasks, e, factor, dvec, piv, kind, stats,
-                       lstep, scratch, p, scaled, aux, psign);
+#define PANEL(R, C)                                                                                                  \
+    hipLaunchKernelGGL((k_ldlt_panel<T, R, C>), dim3(n), dim3(512), 0, st, S, tasks, first, factor, dvec, piv, kind, \
+                       stats, lstep, scratch, p, scaled, aux, psign)
+    switch (cols) {
+        case 16: PANEL(6, 16); break;
+        case 8: PANEL(10, 8); break;
+        default: PANEL(14, 4); break;
+    }
+#undef PANEL
 }
 
 template <typename T>
@@ -1600,8 +1978,15 @@ void launch_ldlt_trail(hipStream_t st, const DevSym& S, const Task* tasks, int n
     hipLaunchKernelGGL(k_ldlt_trail<T>, dim3(n), dim3(256), 0, st, S, tasks, factor, kind, lstep, scratch);
 }
 
-int64_t ldlt_panel_scratch(int f, int w) { return lp_scratch(f, w); }
-int ldlt_panel_cols() { return LP_NB; }
+int64_t ldlt_panel_scratch(int f, int w, int cols) { return lp_scratch(f, w, cols); }
+// columns of the next panel of fronts with at most `rows` rows and `cols` columns left (0: too tall
+// for the registers of one workgroup). The widest panel whose rows fit: a panel pays two launches
+// and its loads and stores once, whatever its columns; no wider than the columns left need.
+int ldlt_panel_cols(int rows, int cols) {
+    if (rows <= 6 * 512 && cols > 8) return 16;
+    if (rows <= 10 * 512) return 8;
+    return rows <= 14 * 512 ? 4 : 0;
+}
 
 template <typename T>
 void launch_ldlt_mirror(hipStream_t st, const DevSym& S, const Task* tasks, int n, T* factor) {
@@ -1647,7 +2032,7 @@ void launch_info_from_stats(hipStream_t st, const DevSym& S, const int64_t* stat
                                        const int8_t*);                                                             \
     template void launch_ldlt_update<T>(hipStream_t, const DevSym&, const Task*, int, T*, const int32_t*);        \
     template void launch_ldlt_mirror<T>(hipStream_t, const DevSym&, const Task*, int, T*);                        \
-    template void launch_ldlt_panel<T>(hipStream_t, const DevSym&, const Task*, int, int, T*, T*, int32_t*,        \
+    template void launch_ldlt_panel<T>(hipStream_t, const DevSym&, const Task*, int, int, int, T*, T*, int32_t*,   \
                                        int8_t*, int64_t*, int32_t*, T*, int, double, double, int, const double*,   \
                                        const int8_t*);                                                             \
     template void launch_ldlt_trail<T>(hipStream_t, const DevSym&, const Task*, int, T*, const int8_t*,           \

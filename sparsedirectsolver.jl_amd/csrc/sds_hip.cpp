@@ -83,8 +83,8 @@ struct Launch {
     int64_t off;
     int n;
     double flops, bytes;  // algorithmic work of the launch
-    int nstep = 0, ncopy = 0;  // k_big_step launches: step tasks, then copies, then update tiles
-    int k = 0;                 // pivot step of the k_lu_pivot / k_lu_update launches
+    int nstep = 0, ncopy = 0;  // k_big_step launches: step tasks, then copies, then update tiles; panel columns
+    int k = 0;                 // pivot step of the pivot and panel launches
 };
 
 struct Level {
@@ -247,7 +247,7 @@ struct sds_handle {
     int small_kind = 0;  // small-front kernels (Cholesky): 0 one wave per tiny front + blocked,
                          // 1 one wave per tiny front + column by column, 2 column by column
     int panel_block = 0;  // Cholesky large fronts: panel block width (a multiple of NB; 0 = one block)
-    int pivot_panels = 0;  // LDL^T large fronts: 1 deferred-update panels, 0 one pivot per launch pair
+    int pivot_panels = 0;  // LDL^T large fronts: 0 panels of pivot columns, 1 one pivot per launch pair
     int64_t ldlt_scr = 0;  // ... the panels' scratch (elements)
     void* lscratch = nullptr;
     int32_t* status = nullptr;
@@ -849,83 +849,69 @@ int build_schedule(sds_handle* h, int dtype) {
             }
             L.plan.push_back({L_LU_FINISH, off_p, (int)tp.size(), 0.0, 0.0});
             wmax = 0;
-        } else if (h->method != M_CHOLESKY && h->pivot_panels) {
-            // LDL^T of the large fronts in panels of deferred updates: per panel e one launch takes
-            // each front's next pivots until ldlt_panel_cols() columns are done (one workgroup per
-            // front, its scratch at the offset in the task), then one launch applies them to the
-            // entries after the panel (64 x 64 tiles). A panel takes at least that many columns,
-            // so ceil(wmax / cols) panels finish every front of the level.
-            const int nbp = ldlt_panel_cols();
-            std::vector<Task> tp;
+        } else if (h->method != M_CHOLESKY) {
+            // LDL^T of the large fronts, after the mirror tiles of their fully summed squares, in
+            // panels: one launch takes every front's next `cols` pivot columns (one workgroup per
+            // front, its scratch at the offset in the task), the next applies them to the columns
+            // after (64 x 64 tiles: the remaining fully summed columns, all rows; one tile list per
+            // 64 columns). A panel takes at least `cols` columns (a 2x2 pivot at its end one more),
+            // so the panels' widths add up to the level's widest front. While a front has more rows
+            // left than a panel's registers hold (or with pivot_panels = 1): one pivot (1x1 or 2x2)
+            // per launch pair, the choice by one workgroup per front, its update by the same tiles.
+            std::vector<std::pair<int, int>> pan;  // the launches: first column at least, panel columns (0: a pair)
+            int maxcols = 0;
+            for (int k = 0; k < wmax;) {
+                int rows = 0;
+                for (int32_t s : L.big)
+                    if (h->fncols[s] > k) rows = std::max(rows, h->fnrows[s] - k);
+                pan.push_back({k, h->pivot_panels ? 0 : ldlt_panel_cols(rows, wmax - k)});
+                maxcols = std::max(maxcols, pan.back().second);
+                k += std::max(pan.back().second, 1);
+            }
+            std::vector<Task> tp, tm;
             int64_t off = 0;
             for (int32_t s : L.big) {
                 tp.push_back({s, (int32_t)off, 0, 0});
-                off += ldlt_panel_scratch(h->fnrows[s], h->fncols[s]);
-            }
-            h->ldlt_scr = std::max(h->ldlt_scr, off);
-            const int64_t off_p = (int64_t)tasks.size();
-            tasks.insert(tasks.end(), tp.begin(), tp.end());
-            const int npan = (wmax + nbp - 1) / nbp;
-            for (int e = 0; e < npan; ++e) {
-                std::vector<Task> tu;
-                double fl1 = 0, by1 = 0;
-                const int kmin = (e + 1) * nbp, lo = kmin / TILE * TILE;
-                for (size_t q = 0; q < L.big.size(); ++q) {
-                    const int32_t s = L.big[q];
-                    const int f = h->fnrows[s], w = h->fncols[s];
-                    if (kmin >= w) continue;
-                    for (int J0 = lo; J0 < w; J0 += TILE)
-                        for (int I0 = lo; I0 < f; I0 += TILE) tu.push_back({s, I0, J0, tp[q].a});
-                    // a panel of nbp 1x1 pivots on the (f - kmin) x (w - kmin) entries after it
-                    const double ent = (double)(f - kmin) * (w - kmin);
-                    fl1 += 2.0 * nbp * ent;
-                    by1 += 2.0 * dbl_es * ent;
-                }
-                L.plan.push_back({L_LDLT_PANEL, off_p, (int)tp.size(), 0.0, 0.0});
-                L.plan.back().k = e;
-                push_launch(L, L_LDLT_TRAIL, tu, fl1, by1);
-            }
-            L.plan.push_back({L_LDLT_FINISH, off_p, (int)tp.size(), 0.0, 0.0});
-            wmax = 0;
-        } else if (h->method != M_CHOLESKY) {
-            // LDL^T of the large fronts, one pivot (1x1 or 2x2) per launch pair over all of them:
-            // the pivot (one workgroup per front) and its update tiles (the remaining fully summed
-            // columns, all rows, 64 x 64 tiles; one tile list per 64 pairs; a pair takes at least
-            // one column, so pair t works on columns >= t), after the mirror tiles of the fully
-            // summed squares
-            std::vector<Task> tp, tm;
-            for (int32_t s : L.big) {
-                tp.push_back({s, 0, 0, 0});
+                if (maxcols) off += ldlt_panel_scratch(h->fnrows[s], h->fncols[s], maxcols);
                 const int w = h->fncols[s];
                 for (int J0 = 0; J0 < w; J0 += 64)
                     for (int I0 = J0; I0 < w; I0 += 64) tm.push_back({s, I0, J0, 0});
             }
+            if (off >= ((int64_t)1 << 31)) return fail(h, SDS_NOT_SUPPORTED, "panel scratch beyond 2^31 entries");
+            h->ldlt_scr = std::max(h->ldlt_scr, off);
             push_launch(L, L_LDLT_MIRROR, tm, 0.0, 0.0);
             const int64_t off_p = (int64_t)tasks.size();
             tasks.insert(tasks.end(), tp.begin(), tp.end());
-            for (int e = 0; e * 64 < wmax; ++e) {
-                std::vector<Task> tu;
-                for (int32_t s : L.big) {
-                    const int f = h->fnrows[s], w = h->fncols[s];
-                    if (64 * e >= w) continue;
-                    for (int J0 = 64 * e; J0 < w; J0 += 64)
-                        for (int I0 = 64 * e; I0 < f; I0 += 64) tu.push_back({s, I0, J0, 0});
-                }
-                const int64_t off_u = (int64_t)tasks.size();
-                tasks.insert(tasks.end(), tu.begin(), tu.end());
-                for (int k = 64 * e; k < std::min(wmax, 64 * e + 64); ++k) {
-                    double fl1 = 0, by1 = 0;
-                    for (int32_t s : L.big) {
-                        const double f = h->fnrows[s], w = h->fncols[s];
-                        if (k >= w) continue;
-                        const double ent = (f - k - 1) * (w - k - 1);
-                        fl1 += 2.0 * ent;
-                        by1 += 2.0 * dbl_es * ent;
+            int64_t off_u = 0;
+            int n_u = 0, e_u = -1;
+            for (const auto& pn : pan) {
+                const int k = pn.first, cols = std::max(pn.second, 1);
+                const bool panel = pn.second > 0;
+                if (k / 64 != e_u) {
+                    e_u = k / 64;
+                    off_u = (int64_t)tasks.size();
+                    for (size_t q = 0; q < L.big.size(); ++q) {
+                        const int32_t s = L.big[q];
+                        const int f = h->fnrows[s], w = h->fncols[s];
+                        if (64 * e_u >= w) continue;
+                        for (int J0 = 64 * e_u; J0 < w; J0 += 64)
+                            for (int I0 = 64 * e_u; I0 < f; I0 += 64) tasks.push_back({s, I0, J0, tp[q].a});
                     }
-                    L.plan.push_back({L_LDLT_PIVOT, off_p, (int)tp.size(), 0.0, 0.0});
-                    L.plan.back().k = k;
-                    L.plan.push_back({L_LDLT_UPDATE, off_u, (int)tu.size(), fl1, by1});
+                    n_u = (int)((int64_t)tasks.size() - off_u);
                 }
+                double fl1 = 0, by1 = 0;
+                for (int32_t s : L.big) {
+                    const double f = h->fnrows[s], w = h->fncols[s];
+                    if (k + cols >= w) continue;
+                    const double ent = (f - k - cols) * (w - k - cols);
+                    fl1 += 2.0 * cols * ent;
+                    by1 += 2.0 * dbl_es * ent;
+                }
+                L.plan.push_back({panel ? L_LDLT_PANEL : L_LDLT_PIVOT, off_p, (int)tp.size(), 0.0, 0.0});
+                L.plan.back().k = k;
+                L.plan.back().nstep = cols;
+                if (k + cols < wmax)
+                    L.plan.push_back({panel ? L_LDLT_TRAIL : L_LDLT_UPDATE, off_u, n_u, fl1, by1});
             }
             L.plan.push_back({L_LDLT_FINISH, off_p, (int)tp.size(), 0.0, 0.0});
             wmax = 0;
@@ -1472,8 +1458,8 @@ int factorize_ldlt(sds_handle* h, const double* nz, int pivot, double u, double 
                     case L_LDLT_UPDATE: launch_ldlt_update<T>(st, h->dsym, t, ln.n, factor, h->lstep); break;
                     case L_LDLT_MIRROR: launch_ldlt_mirror<T>(st, h->dsym, t, ln.n, factor); break;
                     case L_LDLT_PANEL:
-                        launch_ldlt_panel<T>(st, h->dsym, t, ln.n, ln.k, factor, dv, h->piv, h->pkind, h->stats,
-                                             h->lstep, static_cast<T*>(h->lscratch), pivot, u, eps, scaled, h->aux,
+                        launch_ldlt_panel<T>(st, h->dsym, t, ln.n, ln.k == 0, ln.nstep, factor, dv, h->piv, h->pkind,
+                                             h->stats, h->lstep, static_cast<T*>(h->lscratch), pivot, u, eps, scaled, h->aux,
                                              psign);
                         break;
                     case L_LDLT_TRAIL:
