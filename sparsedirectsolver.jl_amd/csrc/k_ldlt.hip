@@ -24,6 +24,7 @@
 // device statistics src/numeric/ldlt.jl:1276-1356.
 #pragma clang fp contract(off)
 #include "k_front.h"
+#include "k_panel.h"
 #include "sds_common.h"
 #include "sds_kernels.h"
 
@@ -51,53 +52,6 @@ struct RedBuf {
     double v[NT / 64];
     int i[NT / 64];
 };
-
-// a value every lane holds, as a scalar
-__device__ inline int uni(int v) { return __builtin_amdgcn_readfirstlane(v); }
-
-// max(m, |a|), a NaN in a passed over (fmax would first quiet both operands)
-__device__ inline double max_abs(double m, double a) {
-    double r;
-    asm("v_max_f64 %0, %1, |%2|" : "=v"(r) : "v"(m), "v"(a));
-    return r;
-}
-// a wave's largest v (v >= 0 in every lane; a NaN is passed over) in its last lane: row shifts and
-// row broadcasts, no LDS round trip per step
-template <int CTRL, int ROWS>
-__device__ inline double dpp_max_step(double v) {
-    const int2 x = __builtin_bit_cast(int2, v);
-    int2 y;
-    y.x = __builtin_amdgcn_update_dpp(0, x.x, CTRL, ROWS, 0xf, true);
-    y.y = __builtin_amdgcn_update_dpp(0, x.y, CTRL, ROWS, 0xf, true);
-    return max_abs(v, __builtin_bit_cast(double, y));
-}
-__device__ inline double wave_max_last(double v) {
-    v = dpp_max_step<0x111, 0xf>(v);  // row_shr 1, 2, 4, 8
-    v = dpp_max_step<0x112, 0xf>(v);
-    v = dpp_max_step<0x114, 0xf>(v);
-    v = dpp_max_step<0x118, 0xf>(v);
-    v = dpp_max_step<0x142, 0xa>(v);  // row_bcast 15, 31
-    return dpp_max_step<0x143, 0xc>(v);
-}
-__device__ inline double last_lane(double v) {
-    int2 x = __builtin_bit_cast(int2, v);
-    x.x = __builtin_amdgcn_readlane(x.x, 63);
-    x.y = __builtin_amdgcn_readlane(x.y, 63);
-    return __builtin_bit_cast(double, x);
-}
-// a wave's smallest i in its last lane
-template <int CTRL, int ROWS>
-__device__ inline int dpp_min_step(int v) {
-    return min(v, __builtin_amdgcn_update_dpp(0x7fffffff, v, CTRL, ROWS, 0xf, false));
-}
-__device__ inline int wave_min_last(int v) {
-    v = dpp_min_step<0x111, 0xf>(v);
-    v = dpp_min_step<0x112, 0xf>(v);
-    v = dpp_min_step<0x114, 0xf>(v);
-    v = dpp_min_step<0x118, 0xf>(v);
-    v = dpp_min_step<0x142, 0xa>(v);
-    return dpp_min_step<0x143, 0xc>(v);
-}
 
 // (values >= 0) every lane gets the wave's maximum
 __device__ inline double wave_jmax(double v) {
@@ -906,35 +860,6 @@ constexpr int LP_MAXP = LP_NB + 1;  // pivot rows of one panel
 // w, U[q w + j] = U(k0 + q, j)), the current diagonal DG (w) and the saved panel columns V (cols x f)
 inline int64_t lp_scratch(int f, int w, int cols) { return (int64_t)(LP_MAXP + 1) * w + (int64_t)cols * f; }
 
-// entry `off` bytes into the column `col` (a wave-uniform address: scalar base, 32-bit offset)
-template <typename T>
-__device__ inline T load_at(const T* col, uint32_t off) {
-    return *reinterpret_cast<const T*>(reinterpret_cast<const char*>(col) + off);
-}
-template <typename T>
-__device__ inline void store_at(T* col, uint32_t off, T v) {
-    *reinterpret_cast<T*>(reinterpret_cast<char*>(col) + off) = v;
-}
-
-// a thread's rows k0 + tid + NT u of a front: their byte offsets in a column and how many lie above an
-// end. Both start from values hidden from the optimizer (empty asm): hoisted out of the pivot loop, the
-// R comparisons of every loop would take R scalar register pairs each.
-template <int NT, int SIZE>
-struct PanelRows {
-    uint32_t o0, olast;
-    int left;  // k0 + tid
-    __device__ __attribute__((always_inline)) PanelRows(int k0, int f) {
-        left = k0 + (int)threadIdx.x;
-        asm volatile("" : "+v"(left));
-        o0 = (uint32_t)left * SIZE;
-        olast = (uint32_t)(f - 1) * SIZE;
-    }
-    __device__ uint32_t off(int u) const { return o0 + (uint32_t)(NT * SIZE) * u; }
-    __device__ uint32_t clamped(int u) const { return min(off(u), olast); }
-    // slots u < count(end) hold rows below end
-    __device__ int count(int end) const { return (end - left + NT - 1) >> (NT == 512 ? 9 : NT == 1024 ? 10 : 8); }
-};
-
 // a front during a panel, as its NT threads see it
 template <typename T, int NT, int R, int MAXP>
 struct PanelFront {
@@ -1348,25 +1273,6 @@ struct PanelFront {
         __syncthreads();
     }
 };
-
-// N values computed here, not where they are used next (empty asm statements, which also order the
-// memory accesses around them): without it the register allocator meets the loads of a whole panel
-// update before the first of its sums, and the panel spills
-template <int N, typename T>
-__device__ __attribute__((always_inline)) inline void pin(T* v) {
-#pragma unroll
-    for (int c = 0; c < N; ++c) asm volatile("" : "+v"(v[c])::"memory");
-}
-// x[c - 1] = x[c] - l u[c] for 1 <= c < W: a row's rank-1 update, each column moving one register left;
-// eight entries of u in flight together
-template <int W, int C0 = 1, int N, typename T>
-__device__ __attribute__((always_inline)) inline void shift_update(T (&x)[N], T l, const T* u) {
-    constexpr int C1 = C0 + 8 < W ? C0 + 8 : W;
-#pragma unroll
-    for (int c = C0; c < C1; ++c) x[c - 1] = x[c] - l * u[c];
-    pin<C1 - C0>(x + C0 - 1);
-    if constexpr (C1 < W) shift_update<W, C1>(x, l, u);
-}
 
 // the state of a panel's usual pivots
 template <typename T, int R, int NBP>

@@ -18,6 +18,7 @@
 // (:137-145).
 #pragma clang fp contract(off)
 #include "k_front.h"
+#include "k_panel.h"
 #include "sds_common.h"
 #include "sds_kernels.h"
 
@@ -304,7 +305,7 @@ __global__ void __launch_bounds__(256) k_big_lu_extend_add(DevSym S, const Task*
 }
 
 // ---------------------------------------------------------------------------
-// large fronts, one pivot per pair of launches: k_lu_pivot (one workgroup per front) takes
+// large fronts too tall for the panels below, one pivot per pair of launches: k_lu_pivot (one workgroup per front) takes
 // the previous pivot's deferred scaling, searches column k, swaps the rows and sets d_k;
 // k_lu_update (64 x 64 tiles over every front of the level) applies the rank-1 update of
 // step k to the fully summed columns (all rows) and to U12 (the fully summed rows). Each
@@ -604,6 +605,352 @@ __global__ void __launch_bounds__(1024) k_lu_finish(DevSym S, const Task* __rest
     for (int q = tid; q < w; q += NT) piv[c0 + q] = c0 + piv[c0 + q];
 }
 
+// ---------------------------------------------------------------------------
+// large fronts in panels of NBP columns, three launches each: k_lu_panel (one workgroup per front)
+// takes the panel's pivots with its columns in registers (thread t: the rows k0 + t + NT u, R rows,
+// R NBP entries); k_lu_urows forms the panel's U rows in every column after it (a thread per
+// column); k_lu_trail (64 x 64 tiles) applies the panel to the fully summed columns and to U12. Each
+// entry goes through the operations of lu_front above, in the same order: L = a / d first, then
+// a - L u with the unscaled row entry u, and U = u / d stored in its place in Q.
+//
+// A pivot of k_lu_panel costs one barrier: the column's two maxima (all rows for the threshold, the
+// fully summed rows below for the row choice) by lane reductions, the scaling, the rank-1 update of
+// the panel's later columns, which moves each column one register to the left. An interchange adds
+// two barriers (the row of the largest entry, the two rows through LDS) and exchanges the two
+// rows of the columns in memory (L, the columns after the panel, U12).
+
+template <typename T, int R, int NBP>
+struct LuPanel {
+    T x[R][NBP];  // x[u][c] = entry (k0 + tid + NT u, k + c)
+    int nr;       // row slots in use
+    int buf;
+};
+template <typename T, int NBP>
+struct LuPanelLds {
+    __align__(16) double red[2][512 / 64][2];
+    int found[512 / 64];
+    __align__(16) T urow[2][NBP];
+    __align__(16) T rrow[NBP];
+};
+struct LuPrm {
+    int pivoting;
+    double u, eps;
+};
+
+// pivots k, k + 1, ... of the panel while its remaining columns number more than W - 8 (of W registers
+// per row)
+template <typename T, int NT, int R, int NBP, int W>
+__device__ __attribute__((always_inline)) inline void lu_panel_pivots(LuPanel<T, R, NBP>& X, const LuFront<T>& F, int k0,
+                                                                      int& k, int kend, const LuPrm& p,
+                                                                      LuPanelLds<T, NBP>& D, int* lp, int8_t* kind,
+                                                                      T* dd, int64_t* st) {
+    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6, f = F.f, w = F.w;
+    const int kstop = min(kend, k0 + NBP - (W > 8 ? W - 8 : 0));
+    while (k < kstop) {
+        const PanelRows<NT, (int)sizeof(T)> rw(k0, f);
+        const int nf = rw.count(f), nw = rw.count(w);
+        const bool up = tid > k - k0;  // (the pivot's row is among the first slot's)
+        double lam = 0.0, mx = 0.0;
+        bool nan = false;
+#pragma unroll
+        for (int u = 0; u < R; ++u) {
+            if (u < X.nr) {  // (only the last slot can hold rows past the front's end)
+                double a = (double)X.x[u][0];
+                if (u == 0) a = tid >= k - k0 ? a : 0.0;
+                if (u + 1 == X.nr) a = u < nf ? a : 0.0;
+                nan |= a != a;
+                mx = max_abs(mx, a);
+                if (NT * u < w - k0) lam = max_abs(lam, u < nw && (u > 0 || up) ? a : 0.0);
+            }
+        }
+        lam = wave_max_last(lam);
+        mx = wave_max_last(mx);
+        if (__any(nan)) mx = __builtin_nan("");
+        X.buf ^= 1;
+        if (lane == 63) {
+            D.red[X.buf][wv][0] = lam;
+            D.red[X.buf][wv][1] = mx;
+        }
+        if (tid == k - k0) {
+#pragma unroll
+            for (int c = 0; c < W; ++c) D.urow[X.buf][c] = X.x[0][c];
+        }
+        __syncthreads();  // (waits for LDS only: the L columns' stores stay in flight)
+        nan = false;
+        lam = 0.0;
+        mx = 0.0;
+#pragma unroll
+        for (int q = 0; q < NT / 64; ++q) {
+            lam = max_abs(lam, D.red[X.buf][q][0]);
+            const double v = D.red[X.buf][q][1];
+            nan |= v != v;
+            mx = max_abs(mx, v);
+        }
+        const double akk = fabs((double)D.urow[X.buf][0]);
+        // keep the diagonal when |a_kk| >= u max |a_ik|; else the largest fully summed row, the first
+        // on ties, k if none is larger
+        if (uni(p.pivoting && !(!nan && akk >= p.u * mx) && lam > akk)) {
+            int ri = 0x7fffffff;
+#pragma unroll
+            for (int u = R - 1; u >= 0; --u)
+                if (u < nw && (u > 0 || up) && fabs((double)X.x[u][0]) == lam) ri = k0 + tid + NT * u;
+            ri = wave_min_last(ri);
+            if (lane == 63) D.found[wv] = ri;
+            __syncthreads();
+            int r = D.found[0];
+#pragma unroll
+            for (int q = 1; q < NT / 64; ++q) r = min(r, D.found[q]);
+            r = uni(r);
+            // rows k and r of the panel's columns through LDS (the old row k is in urow)
+            const int ur = (r - k0) / NT, tr = r - k0 - ur * NT;
+#pragma unroll
+            for (int u = 0; u < R; ++u)
+                if (u == ur && tid == tr) {
+#pragma unroll
+                    for (int c = 0; c < W; ++c) {
+                        D.rrow[c] = X.x[u][c];
+                        X.x[u][c] = D.urow[X.buf][c];
+                    }
+                }
+            __syncthreads();
+            if (tid < W) D.urow[X.buf][tid] = D.rrow[tid];
+            for (int j = tid; j < w; j += NT)
+                if (j < k || j >= kend) {
+                    T& a = F.l(k, j);
+                    T& b = F.l(r, j);
+                    const T t = a;
+                    a = b;
+                    b = t;
+                }
+            for (int j = w + tid; j < f; j += NT) {
+                T& a = F.u(k, j);
+                T& b = F.u(r, j);
+                const T t = a;
+                a = b;
+                b = t;
+            }
+            if (tid == 0) {
+                const int t = lp[k];
+                lp[k] = lp[r];
+                lp[r] = t;
+            }
+            __syncthreads();
+        }
+        double dk = (double)D.urow[X.buf][0];
+        const bool pert = !(fabs(dk) >= p.eps) || dk == 0.0;
+        if (tid == 0) {
+            kind[k] = pert ? KIND_PERTURBED : KIND_1X1;
+            if (pert) {
+                if (dk == 0.0) st[LST_NZERO]++;
+                st[LST_NPERT]++;
+            }
+        }
+        if (pert) dk = (dk < 0.0 ? -1.0 : 1.0) * p.eps;
+        const T d = T(dk);
+        if (tid == 0) {
+            if (pert && dk == 0.0 && st[LST_INFO] == 0) st[LST_INFO] = k + 1;
+            dd[k] = d;
+        }
+        // row k of U in the panel's later columns
+        if (tid > 0 && tid < min(W, kend - k)) F.Q[(int64_t)k * f + k + tid] = D.urow[X.buf][tid] / d;
+        T* col = F.P + (int64_t)k * f;
+        // the scaling of three row slots at a time (independent divisions), then their updates
+#pragma unroll
+        for (int u0 = 0; u0 < R; u0 += 3) {
+            if (u0 < X.nr) {
+                T l[3] = {};
+#pragma unroll
+                for (int u = 0; u < 3 && u0 + u < R; ++u) l[u] = X.x[u0 + u][0] / d;
+                pin<3>(l);
+#pragma unroll
+                for (int u = 0; u < 3 && u0 + u < R; ++u) {
+                    if (u0 + u < nf && (u0 + u > 0 || up)) store_at(col, rw.off(u0 + u), l[u]);
+                    shift_update<W>(X.x[u0 + u], l[u], D.urow[X.buf]);
+                }
+            }
+        }
+        ++k;
+    }
+}
+
+// the panel of columns [k0, k0 + NBP) of every large front of a level that has them. task: (s)
+//
+// Bound: latency, one workgroup per front walks the pivots one after another. NT = 512 (two waves
+// per SIMD) leaves 256 registers a thread, 192 of them for the panel: NBP R <= 96.
+template <typename T, int R, int NBP>
+__global__ void __launch_bounds__(512) k_lu_panel(DevSym S, const Task* __restrict__ tasks, int k0,
+                                                  T* __restrict__ factor, T* __restrict__ ufactor,
+                                                  T* __restrict__ dvec, int32_t* __restrict__ piv,
+                                                  int8_t* __restrict__ pkind, int64_t* __restrict__ stats, LuPrm prm,
+                                                  int scaled, const double* __restrict__ aux) {
+    constexpr int NT = 512;
+    __shared__ LuPanelLds<T, NBP> D;
+    const int s = tasks[blockIdx.x].s;
+    const int f = S.fnrows[s], w = S.fncols[s];
+    if (k0 >= w) return;
+    const int c0 = S.super_ptr[s], tid = threadIdx.x;
+    if (scaled && aux[0] > 0) prm.eps = prm.eps * aux[0];
+    const LuFront<T> F{factor + S.panel_off[s], ufactor + S.panel_off[s], f, w};
+    int* lp = piv + c0;
+    int8_t* kind = pkind + c0;
+    T* dd = dvec + c0;
+    int64_t* st = stats + (int64_t)s * NF;
+    if (k0 == 0) {
+        for (int q = tid; q < w; q += NT) {
+            lp[q] = q;
+            dvec[S.n + c0 + q] = T(0);
+        }
+        if (tid < NF) st[tid] = 0;
+    }
+    const int kend = min(w, k0 + NBP);
+    LuPanel<T, R, NBP> X;
+    X.nr = (f - k0 + NT - 1) / NT;
+    X.buf = 0;
+    {
+        const PanelRows<NT, (int)sizeof(T)> rw(k0, f);
+#pragma unroll
+        for (int u = 0; u < R; ++u) {
+            const uint32_t off = rw.clamped(u);
+#pragma unroll
+            for (int c = 0; c < NBP; ++c) X.x[u][c] = load_at(F.P + (int64_t)min(k0 + c, w - 1) * f, off);
+        }
+    }
+    __syncthreads();
+    int k = k0;
+    if constexpr (NBP > 24) lu_panel_pivots<T, NT, R, NBP, 32>(X, F, k0, k, kend, prm, D, lp, kind, dd, st);
+    if constexpr (NBP > 16) lu_panel_pivots<T, NT, R, NBP, 24>(X, F, k0, k, kend, prm, D, lp, kind, dd, st);
+    if constexpr (NBP > 8) lu_panel_pivots<T, NT, R, NBP, 16>(X, F, k0, k, kend, prm, D, lp, kind, dd, st);
+    lu_panel_pivots<T, NT, R, NBP, (NBP < 8 ? NBP : 8)>(X, F, k0, k, kend, prm, D, lp, kind, dd, st);
+}
+
+// the U rows of a panel's pivots k0 .. k0 + np - 1 in the 64 columns from J0 (after the panel): u = a -
+// L u in pivot order, eight rows at a time, a thread per column; the unscaled rows go to the front's
+// scratch (U[q f + j], read by k_lu_trail), u / d to Q. task: (s, J0, 0, scratch offset)
+constexpr int LU_PANEL_MAX = 32;  // most columns of a panel
+
+template <typename T>
+__global__ void __launch_bounds__(64) k_lu_urows(DevSym S, const Task* __restrict__ tasks, int k0, int cols,
+                                                 const T* __restrict__ factor, T* __restrict__ ufactor,
+                                                 const T* __restrict__ dvec, T* __restrict__ scratch) {
+    __shared__ T Ls[LU_PANEL_MAX][LU_PANEL_MAX + 1];  // Ls[r][q] = L(k0 + r, k0 + q)
+    const Task t = tasks[blockIdx.x];
+    const int s = t.s, f = S.fnrows[s], w = S.fncols[s];
+    if (k0 >= w) return;
+    const int np = min(cols, w - k0), j = t.a + threadIdx.x;
+    if (t.a + 64 <= k0 + np) return;
+    const T* P = factor + S.panel_off[s];
+    T* Q = ufactor + S.panel_off[s];
+    const T* dd = dvec + S.super_ptr[s] + k0;
+    T* U = scratch + t.c;
+    const bool on = j >= k0 + np && j < f;
+    const int jc = min(max(j, k0 + np), f - 1);  // (np < f - k0 in a front with columns after the panel)
+    for (int q = threadIdx.x; q < np * np; q += 64) {
+        const int c = q / np, r = q - c * np;
+        Ls[r][c] = P[(int64_t)(k0 + c) * f + k0 + r];
+    }
+    __syncthreads();
+    for (int b0 = 0; b0 < np; b0 += 8) {
+        T a[8];
+#pragma unroll
+        for (int r = 0; r < 8; ++r) {
+            const int i = k0 + min(b0 + r, np - 1);
+            a[r] = jc < w ? P[(int64_t)jc * f + i] : Q[(int64_t)i * f + jc];
+        }
+        for (int q0 = 0; q0 < b0; q0 += 8) {  // (whole blocks of eight: b0 is a multiple of eight)
+            T uv[8];
+#pragma unroll
+            for (int q = 0; q < 8; ++q) uv[q] = U[(int64_t)(q0 + q) * f + jc];
+#pragma unroll
+            for (int q = 0; q < 8; ++q)
+#pragma unroll
+                for (int r = 0; r < 8; ++r) a[r] = a[r] - Ls[min(b0 + r, np - 1)][q0 + q] * uv[q];
+        }
+#pragma unroll
+        for (int r = 0; r < 8; ++r) {
+#pragma unroll
+            for (int r2 = r + 1; r2 < 8; ++r2) a[r2] = a[r2] - Ls[min(b0 + r2, np - 1)][min(b0 + r, np - 1)] * a[r];
+        }
+#pragma unroll
+        for (int r = 0; r < 8; ++r)
+            if (on && b0 + r < np) {
+                U[(int64_t)(b0 + r) * f + j] = a[r];
+                Q[(int64_t)(k0 + b0 + r) * f + j] = a[r] / dd[b0 + r];
+            }
+    }
+}
+
+// a panel's update of the entries after it: tile (s, I0, J0, scratch offset) of 64 x 64 entries, J0 < w: the
+// fully summed columns (every row), J0 >= w: U12 (the fully summed rows, stored transposed), each
+// entry a - L u in pivot order. Lanes along the contiguous direction, sixteen entries a thread loaded
+// together; the panel's factor along the lanes in registers, the other from LDS by broadcast.
+// Bound: HBM / L2 (two accesses per entry and panel).
+template <typename T>
+__global__ void __launch_bounds__(256) k_lu_trail(DevSym S, const Task* __restrict__ tasks, int k0, int cols,
+                                                  T* __restrict__ factor, T* __restrict__ ufactor,
+                                                  const T* __restrict__ scratch) {
+    __shared__ __align__(16) T Bs[LU_PANEL_MAX][TILE];
+    const Task t = tasks[blockIdx.x];
+    const int s = t.s, f = S.fnrows[s], w = S.fncols[s];
+    if (k0 >= w) return;
+    const int np = min(cols, w - k0), kend = k0 + np;
+    const int I0 = t.a, J0 = t.b;
+    if (I0 + TILE <= kend || J0 + TILE <= kend) return;
+    T* P = factor + S.panel_off[s];
+    T* Q = ufactor + S.panel_off[s];
+    const T* U = scratch + t.c;
+    const int tid = threadIdx.x, lane = tid & 63, cb = (tid >> 6) * 16;
+    const bool u12 = J0 >= w;
+    // element c of the thread: row `lane`, column cb + c (P), or column `lane`, row cb + c (Q); A: the
+    // panel's factor along the lanes, B along c
+    const T* A = u12 ? U + min(J0 + lane, f - 1) : P + (int64_t)k0 * f + min(I0 + lane, f - 1);
+    const T* B = u12 ? P + (int64_t)k0 * f + I0 : U + J0;
+    const int nb = (u12 ? w - I0 : w - J0);  // rows / columns of the tile that exist
+    for (int q = tid; q < np * TILE; q += 256) {
+        const int pp = q / TILE, c = q - pp * TILE;
+        Bs[pp][c] = B[(int64_t)pp * f + min(c, nb - 1)];
+    }
+    T* X = u12 ? Q + (int64_t)I0 * f + min(J0 + lane, f - 1) : P + (int64_t)J0 * f + min(I0 + lane, f - 1);
+    T x[16];
+#pragma unroll
+    for (int c = 0; c < 16; ++c) x[c] = X[(int64_t)min(cb + c, nb - 1) * f];
+    __syncthreads();
+    for (int q0 = 0; q0 < np; q0 += 8) {
+        T a[8];
+#pragma unroll
+        for (int q = 0; q < 8; ++q) a[q] = A[(int64_t)min(q0 + q, np - 1) * f];
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int q = 0; q < 8; ++q) {
+            if (q0 + q >= np) break;
+#pragma unroll
+            for (int c = 0; c < 16; ++c) x[c] = x[c] - a[q] * Bs[q0 + q][cb + c];
+        }
+    }
+    const int il = (u12 ? J0 : I0) + lane, ic = (u12 ? I0 : J0) + cb;
+    if (il >= f || il < kend) return;
+#pragma unroll
+    for (int c = 0; c < 16; ++c)
+        if (ic + c >= kend && cb + c < nb) X[(int64_t)(cb + c) * f] = x[c];
+}
+
+// after the last panel: unit diagonals and empty upper triangles of both panels, the global pivot
+// order. task: (s, I0, J0), a 64 x 64 tile of the fully summed square with I0 <= J0
+template <typename T>
+__global__ void __launch_bounds__(256) k_lu_unit(DevSym S, const Task* __restrict__ tasks, T* __restrict__ factor,
+                                                 T* __restrict__ ufactor, int32_t* __restrict__ piv) {
+    const Task t = tasks[blockIdx.x];
+    const int s = t.s, f = S.fnrows[s], w = S.fncols[s], c0 = S.super_ptr[s];
+    const int i = t.a + (threadIdx.x & 63);
+    T* P = factor + S.panel_off[s];
+    T* Q = ufactor + S.panel_off[s];
+    for (int j = t.b + (threadIdx.x >> 6); j < min(t.b + 64, w); j += 4)
+        if (i <= j) {
+            P[(int64_t)j * f + i] = i == j ? T(1) : T(0);
+            Q[(int64_t)j * f + i] = i == j ? T(1) : T(0);
+        }
+    if (t.a == t.b && threadIdx.x < 64 && i < w) piv[c0 + i] = c0 + piv[c0 + i];
+}
+
 // F22 <- F22 - (L21 D) U12 by 64 x 64 tiles (I0, J0 front rows/columns >= w), each entry's
 // sum over k = 0, 1, ..., w - 1 in order. L21 D and U12 in chunks of 16 columns in LDS.
 template <typename T>
@@ -732,6 +1079,50 @@ void launch_lu_finish(hipStream_t st, const DevSym& S, const Task* tasks, int n,
 }
 
 template <typename T>
+void launch_lu_panel(hipStream_t st, const DevSym& S, const Task* tasks, int n, int k0, int cols, T* factor,
+                     T* ufactor, T* dvec, int32_t* piv, int8_t* kind, int64_t* stats, int pivoting, double u,
+                     double eps, int scaled, const double* aux) {
+    const LuPrm p{pivoting, u, eps};
+#define PANEL(R, C)                                                                                                  \
+    hipLaunchKernelGGL((k_lu_panel<T, R, C>), dim3(n), dim3(512), 0, st, S, tasks, k0, factor, ufactor, dvec, piv,   \
+                       kind, stats, p, scaled, aux)
+    switch (cols) {
+        case 32: PANEL(3, 32); break;
+        case 16: PANEL(6, 16); break;
+        case 8: PANEL(10, 8); break;
+        default: PANEL(20, 4); break;
+    }
+#undef PANEL
+}
+
+// columns of the next panel of fronts with at most `rows` rows and `cols` columns left (0: too tall
+// for the registers of one workgroup). The widest panel whose rows fit: a panel pays three launches
+// and its loads and stores once, whatever its columns; no wider than the columns left need.
+int lu_panel_cols(int rows, int cols) {
+    if (rows <= 3 * 512 && cols > 16) return 32;
+    if (rows <= 6 * 512 && cols > 8) return 16;
+    if (rows <= 10 * 512) return 8;
+    return rows <= 20 * 512 ? 4 : 0;
+}
+
+template <typename T>
+void launch_lu_urows(hipStream_t st, const DevSym& S, const Task* tasks, int n, int k0, int cols, const T* factor,
+                     T* ufactor, const T* dvec, T* scratch) {
+    hipLaunchKernelGGL(k_lu_urows<T>, dim3(n), dim3(64), 0, st, S, tasks, k0, cols, factor, ufactor, dvec, scratch);
+}
+
+template <typename T>
+void launch_lu_trail(hipStream_t st, const DevSym& S, const Task* tasks, int n, int k0, int cols, T* factor,
+                     T* ufactor, const T* scratch) {
+    hipLaunchKernelGGL(k_lu_trail<T>, dim3(n), dim3(256), 0, st, S, tasks, k0, cols, factor, ufactor, scratch);
+}
+
+template <typename T>
+void launch_lu_unit(hipStream_t st, const DevSym& S, const Task* tasks, int n, T* factor, T* ufactor, int32_t* piv) {
+    hipLaunchKernelGGL(k_lu_unit<T>, dim3(n), dim3(256), 0, st, S, tasks, factor, ufactor, piv);
+}
+
+template <typename T>
 void launch_lu_cb(hipStream_t st, const DevSym& S, const Task* tasks, int n, const T* factor, const T* ufactor,
                   T* cbpool, const T* dvec) {
     hipLaunchKernelGGL(k_lu_cb<T>, dim3(n), dim3(256), 0, st, S, tasks, factor, ufactor, cbpool, dvec);
@@ -748,6 +1139,12 @@ void launch_lu_cb(hipStream_t st, const DevSym& S, const Task* tasks, int n, con
     template void launch_lu_pivot<T>(hipStream_t, const DevSym&, const Task*, int, int, T*, T*, T*, int32_t*,      \
                                      int8_t*, int64_t*, int, double, double, int, const double*);                   \
     template void launch_lu_update<T>(hipStream_t, const DevSym&, const Task*, int, int, T*, T*, const T*);         \
+    template void launch_lu_panel<T>(hipStream_t, const DevSym&, const Task*, int, int, int, T*, T*, T*, int32_t*, \
+                                     int8_t*, int64_t*, int, double, double, int, const double*);                   \
+    template void launch_lu_urows<T>(hipStream_t, const DevSym&, const Task*, int, int, int, const T*, T*,          \
+                                     const T*, T*);                                                                 \
+    template void launch_lu_trail<T>(hipStream_t, const DevSym&, const Task*, int, int, int, T*, T*, const T*);     \
+    template void launch_lu_unit<T>(hipStream_t, const DevSym&, const Task*, int, T*, T*, int32_t*);                \
     template void launch_lu_finish<T>(hipStream_t, const DevSym&, const Task*, int, T*, T*, const T*, int32_t*);
 INST(double)
 INST(float)

@@ -63,6 +63,10 @@ enum LaunchKind {
     L_LDLT_FINISH,   // k_ldlt_finish: unit diagonals and the pivot order
     L_LDLT_PANEL,    // k_ldlt_panel: a panel of pivots of every large front of the level
     L_LDLT_TRAIL,    // k_ldlt_trail: that panel's update of the columns after it
+    L_LU_PANEL,      // k_lu_panel: the pivots of columns [k, k + nstep) of every large front of the level
+    L_LU_UROWS,      // k_lu_urows: those pivots' U rows in the columns after
+    L_LU_TRAIL,      // k_lu_trail: their update of the entries after
+    L_LU_UNIT,       // k_lu_unit: unit diagonals and the pivot order
     L_LU_PIVOT,      // k_lu_pivot: step k's pivot of every large front of the level
     L_LU_UPDATE,     // k_lu_update: step k's rank-1 update tiles
     L_LU_FINISH,     // k_lu_finish: the last deferred scaling, U^T and unit diagonals
@@ -133,6 +137,10 @@ int prof_kind(int kind) {
         case L_LDLT_PANEL: return SDS_K_PIVOT_PANEL;
         case L_LDLT_TRAIL: return SDS_K_UPDATE_PANEL;
         case L_LU_UPDATE: return SDS_K_PIVOT_PANEL;
+        case L_LU_PANEL: return SDS_K_PIVOT_PANEL;
+        case L_LU_UROWS: return SDS_K_PIVOT_PANEL;
+        case L_LU_TRAIL: return SDS_K_UPDATE_PANEL;
+        case L_LU_UNIT: return SDS_K_PIVOT_PANEL;
         case L_LU_FINISH: return SDS_K_PIVOT_PANEL;
         case L_LU_ZERO: return SDS_K_ZERO_SCATTER;
         case L_LU_SCATTER: return SDS_K_ZERO_SCATTER;
@@ -247,8 +255,8 @@ struct sds_handle {
     int small_kind = 0;  // small-front kernels (Cholesky): 0 one wave per tiny front + blocked,
                          // 1 one wave per tiny front + column by column, 2 column by column
     int panel_block = 0;  // Cholesky large fronts: panel block width (a multiple of NB; 0 = one block)
-    int pivot_panels = 0;  // LDL^T large fronts: 0 panels of pivot columns, 1 one pivot per launch pair
-    int64_t ldlt_scr = 0;  // ... the panels' scratch (elements)
+    int pivot_panels = 0;  // LDL^T and LU large fronts: 0 panels of pivot columns, 1 one pivot per launch pair
+    int64_t ldlt_scr = 0;  // LDL^T and LU panels' scratch (elements)
     void* lscratch = nullptr;
     int32_t* status = nullptr;
     void* dvec = nullptr;        // D: 2n entries of the factor type (diagonal, 2x2 subdiagonals)
@@ -812,8 +820,88 @@ int build_schedule(sds_handle* h, int dtype) {
         push_extend(L, false, lu ? L_LU_EXTEND : L_EXTEND_ADD);
         int wmax = 0;
         for (int32_t s : L.big) wmax = std::max(wmax, h->fncols[s]);
-        if (lu) {
-            // pivoted LU of the large fronts, one step at a time over all of them: the pivot
+        int fmax = 0;
+        for (int32_t s : L.big) fmax = std::max(fmax, h->fnrows[s]);
+        if (lu && !h->pivot_panels && lu_panel_cols(fmax, wmax) > 0) {
+            // pivoted LU of the large fronts in panels: the panel's pivots (one workgroup per front), the
+            // U rows of those pivots in the columns after it (64 columns a task), its update of the
+            // fully summed columns and of U12 (64 x 64 tiles; the lists start anew every 64 columns)
+            std::vector<Task> tp, td;
+            std::vector<int32_t> off;
+            int64_t o = 0;
+            int maxcols = 0;
+            for (int k = 0; k < wmax;) {
+                int rows = 0;
+                for (int32_t s : L.big)
+                    if (h->fncols[s] > k) rows = std::max(rows, h->fnrows[s] - k);
+                const int cols = lu_panel_cols(rows, wmax - k);
+                maxcols = std::max(maxcols, cols);
+                k += cols;
+            }
+            for (int32_t s : L.big) {
+                tp.push_back({s, 0, 0, 0});
+                off.push_back((int32_t)o);
+                o += (int64_t)maxcols * h->fnrows[s];
+                for (int J0 = 0; J0 < h->fncols[s]; J0 += 64)
+                    for (int I0 = 0; I0 <= J0; I0 += 64) td.push_back({s, I0, J0, 0});
+            }
+            if (o >= ((int64_t)1 << 31)) return fail(h, SDS_NOT_SUPPORTED, "panel scratch beyond 2^31 entries");
+            h->ldlt_scr = std::max(h->ldlt_scr, o);
+            const int64_t off_p = (int64_t)tasks.size();
+            tasks.insert(tasks.end(), tp.begin(), tp.end());
+            int64_t off_r = 0, off_u = 0;
+            int n_r = 0, n_u = 0, e_u = -1;
+            for (int k = 0; k < wmax;) {
+                int rows = 0;
+                for (int32_t s : L.big)
+                    if (h->fncols[s] > k) rows = std::max(rows, h->fnrows[s] - k);
+                const int cols = lu_panel_cols(rows, wmax - k);
+                if (k / 64 != e_u) {
+                    e_u = k / 64;
+                    const int e0 = 64 * e_u;
+                    off_r = (int64_t)tasks.size();
+                    for (size_t q = 0; q < L.big.size(); ++q) {
+                        const int32_t s = L.big[q];
+                        if (e0 < h->fncols[s])
+                            for (int J0 = e0; J0 < h->fnrows[s]; J0 += 64) tasks.push_back({s, J0, 0, off[q]});
+                    }
+                    n_r = (int)((int64_t)tasks.size() - off_r);
+                    off_u = (int64_t)tasks.size();
+                    for (size_t q = 0; q < L.big.size(); ++q) {
+                        const int32_t s = L.big[q];
+                        const int f = h->fnrows[s], w = h->fncols[s];
+                        if (e0 >= w) continue;
+                        for (int J0 = e0; J0 < w; J0 += 64)
+                            for (int I0 = e0; I0 < f; I0 += 64) tasks.push_back({s, I0, J0, off[q]});
+                        for (int J0 = w; J0 < f; J0 += 64)
+                            for (int I0 = e0; I0 < w; I0 += 64) tasks.push_back({s, I0, J0, off[q]});
+                    }
+                    n_u = (int)((int64_t)tasks.size() - off_u);
+                }
+                double fl1 = 0, by1 = 0;
+                bool after = false;
+                for (int32_t s : L.big) {
+                    const double f = h->fnrows[s], w = h->fncols[s];
+                    if (k >= w) continue;
+                    after = after || k + cols < f;
+                    const double c = std::max(w - k - cols, 0.0), ent = std::max(f - k - cols, 0.0) * c + c * (f - w);
+                    fl1 += 2.0 * cols * ent;
+                    by1 += 2.0 * dbl_es * ent;
+                }
+                auto put1 = [&](int kind, int64_t off1, int n1, double fl2, double by2) {
+                    L.plan.push_back({kind, off1, n1, fl2, by2});
+                    L.plan.back().k = k;
+                    L.plan.back().nstep = cols;
+                };
+                put1(L_LU_PANEL, off_p, (int)tp.size(), 0.0, 0.0);
+                if (after) put1(L_LU_UROWS, off_r, n_r, 0.0, 0.0);
+                if (k + cols < wmax) put1(L_LU_TRAIL, off_u, n_u, fl1, by1);
+                k += cols;
+            }
+            push_launch(L, L_LU_UNIT, td, 0.0, 0.0);
+            wmax = 0;
+        } else if (lu) {
+            // fronts too tall for a panel's registers (or pivot_panels = 1): pivoted LU one step at a time over all of them: the pivot
             // (one workgroup per front) and the rank-1 update tiles (every front's remaining
             // fully summed columns and U12, 64 x 64 tiles; one tile list per 64 steps)
             std::vector<Task> tp;
@@ -1508,6 +1596,19 @@ int factorize_lu(sds_handle* h, const double* nz, int pivoting, double u, double
                     case L_LU_ZERO: launch_big_lu_zero<T>(st, h->dsym, t, ln.n, factor, uf, cb); break;
                     case L_LU_SCATTER: launch_big_lu_scatter<T>(st, h->dsym, t, ln.n, nz, factor, uf); break;
                     case L_LU_EXTEND: launch_big_lu_extend_add<T>(st, h->dsym, t, ln.n, factor, uf, cb); break;
+                    case L_LU_PANEL:
+                        launch_lu_panel<T>(st, h->dsym, t, ln.n, ln.k, ln.nstep, factor, uf, dv, h->piv, h->pkind,
+                                           h->stats, pivoting, u, eps, scaled, h->aux);
+                        break;
+                    case L_LU_UROWS:
+                        launch_lu_urows<T>(st, h->dsym, t, ln.n, ln.k, ln.nstep, factor, uf, dv,
+                                           static_cast<T*>(h->lscratch));
+                        break;
+                    case L_LU_TRAIL:
+                        launch_lu_trail<T>(st, h->dsym, t, ln.n, ln.k, ln.nstep, factor, uf,
+                                           static_cast<const T*>(h->lscratch));
+                        break;
+                    case L_LU_UNIT: launch_lu_unit<T>(st, h->dsym, t, ln.n, factor, uf, h->piv); break;
                     case L_LU_PIVOT:
                         launch_lu_pivot<T>(st, h->dsym, t, ln.n, ln.k, factor, uf, dv, h->piv, h->pkind, h->stats,
                                            pivoting, u, eps, scaled, h->aux);

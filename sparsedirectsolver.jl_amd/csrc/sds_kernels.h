@@ -111,6 +111,23 @@ void launch_lu_pivot(hipStream_t st, const DevSym& S, const Task* tasks, int n, 
 template <typename T>
 void launch_lu_update(hipStream_t st, const DevSym& S, const Task* tasks, int n, int k, T* factor, T* ufactor,
                       const T* dvec);
+// panels of the large fronts: the pivot columns [k0, k0 + cols) of every front that has them (task
+// (s)), the U rows of those pivots in the columns after (task (s, J0, 0, scratch offset), 64 columns;
+// scratch: lu_panel_cols' largest answer times f entries a front), their update of the entries after
+// (task (s, I0, J0, scratch offset)); after the last one the unit diagonals (task (s, I0, J0))
+template <typename T>
+void launch_lu_panel(hipStream_t st, const DevSym& S, const Task* tasks, int n, int k0, int cols, T* factor,
+                     T* ufactor, T* dvec, int32_t* piv, int8_t* kind, int64_t* stats, int pivoting, double u,
+                     double eps, int scaled, const double* aux);
+int lu_panel_cols(int rows, int cols);  // 0: one pivot per launch pair
+template <typename T>
+void launch_lu_urows(hipStream_t st, const DevSym& S, const Task* tasks, int n, int k0, int cols, const T* factor,
+                     T* ufactor, const T* dvec, T* scratch);
+template <typename T>
+void launch_lu_trail(hipStream_t st, const DevSym& S, const Task* tasks, int n, int k0, int cols, T* factor,
+                     T* ufactor, const T* scratch);
+template <typename T>
+void launch_lu_unit(hipStream_t st, const DevSym& S, const Task* tasks, int n, T* factor, T* ufactor, int32_t* piv);
 template <typename T>
 void launch_lu_finish(hipStream_t st, const DevSym& S, const Task* tasks, int n, T* factor, T* ufactor,
                       const T* dvec, int32_t* piv);
