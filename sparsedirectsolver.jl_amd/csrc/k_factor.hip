@@ -14,6 +14,8 @@
 // Reference counterparts: regime B fused kernel src/numeric/front.jl:154-206,
 // assembly src/numeric/assembly.jl:18-252, regime C panel src/numeric/factorize.jl:240-269,
 // statistics src/numeric/factorize.jl:13-48.
+#include <algorithm>
+
 #include "k_dense.h"
 #include "k_front.h"
 #include "sds_common.h"
@@ -41,9 +43,12 @@ __device__ inline double rsqrt_nr(double a) {
 }
 
 // ---------------------------------------------------------------------------
-// small fronts: fused assembly + dense Cholesky of the whole front in LDS
+// small fronts: fused assembly + dense Cholesky of the whole front in LDS. RPL: rows a lane holds, 1
+// for fronts of at most 64 rows. A launch of a 64 x 64 x 64 Laplacian's level takes 48 us on average
+// in FP64 (157 us with unrolled pivots at one workgroup a CU), of 160 merged 2-D members 98 us in
+// FP32 (171 us); bounded by the serial chain of assembly loads and pivots, not by the LDS.
 
-template <typename T>
+template <typename T, int RPL>
 __global__ void __launch_bounds__(256) k_front_small_chol(DevSym S, const int32_t* __restrict__ fronts,
                                                          const double* __restrict__ nz, T* __restrict__ factor,
                                                          T* __restrict__ cbpool, T* __restrict__ DB,
@@ -55,8 +60,8 @@ __global__ void __launch_bounds__(256) k_front_small_chol(DevSym S, const int32_
     const int f = S.fnrows[s], w = S.fncols[s], m = f - w;
     const int tid = threadIdx.x;
     assemble_dense<T>(S, s, nz, cbpool, F, f, 0);
-    // blocked Cholesky of the w pivot columns over the whole front (f <= 128)
-    const int st = front_chol_lds<T, 2>(F, f, w, eps, &sh);
+    // blocked Cholesky of the w pivot columns over the whole front (f <= 64 RPL)
+    const int st = front_chol_lds<T, RPL>(F, f, w, eps, &sh);
     // the panel (strict upper triangle zero) and the contribution block's lower triangle, a wave
     // per column, lanes along the rows
     const int lane = tid & 63, wv = tid >> 6;
@@ -226,7 +231,9 @@ __global__ void __launch_bounds__(256) k_subtree_chol(DevSym S, const int32_t* _
 // entry's updates come in column order as separate products and differences, the arithmetic of
 // the blocked kernel. The panel and contribution block are written from the registers, and for
 // fronts of at most FUSED_INV_MAX columns the diagonal block's inverse (column c by lane c, the
-// arithmetic of the per-block inverse kernel).
+// arithmetic of the per-block inverse kernel). Bounded by its chain of dependent loads and the first
+// fetch of its code: 14 us a launch for a few dozen fronts (22 us unrolled over the pivots, child by
+// child), 45 us for thousands in FP32 (70 us).
 template <typename T>
 __global__ void __launch_bounds__(256) k_front_tiny_chol(DevSym S, const int32_t* __restrict__ fronts, int nfronts,
                                                         const double* __restrict__ nz, T* __restrict__ factor,
@@ -239,97 +246,98 @@ __global__ void __launch_bounds__(256) k_front_tiny_chol(DevSym S, const int32_t
     T* F = Fs[wv];
     const int s = fronts[id];
     const int f = S.fnrows[s], w = S.fncols[s], m = f - w;
+    const int k0 = S.child_ptr[s], k1 = S.child_ptr[s + 1];
+    const int64_t a0 = S.asm_ptr[s], a1 = S.asm_ptr[s + 1];
+    Children ch;
+    ch.load(S, k0, k1, lane);
     for (int q = lane; q < f * f; q += 64) F[q] = T(0);
     wave_sync();
     // A: one lane sums each run of entries with one destination, in nzval order (distinct runs
     // have distinct destinations)
-    const int64_t a0 = S.asm_ptr[s], a1 = S.asm_ptr[s + 1];
     for (int64_t k = a0 + lane; k < a1; k += 64) {
-        const int64_t d = S.asm_dst[k];
-        if (k > a0 && S.asm_dst[k - 1] == d) continue;
-        double v = 0.0;
-        for (int64_t q = k; q < a1 && S.asm_dst[q] == d; ++q) v += nz[S.asm_src[q]];
+        int64_t d;
+        double v;
+        if (!asm_run(S, nz, a0, a1, k, d, v)) continue;
         F[d >= 0 ? d : -(d + 1)] += T(v);
     }
     wave_sync();
-    for (int k = S.child_ptr[s]; k < S.child_ptr[s + 1]; ++k) {
-        const int c = S.child_list[k];
-        const int64_t co = S.cb_off[c];
-        if (co < 0) continue;
-        const int mc = S.fnrows[c] - S.fncols[c];
-        const T* C = cbpool + co;
-        const int32_t* ri = S.relind + S.relind_ptr[c];
-        const int rl = lane < mc ? ri[lane] : 0;
-        for (int jj = 0; jj < mc; ++jj) {
-            const int pj = __builtin_amdgcn_readlane(rl, jj);
-            if (lane >= jj && lane < mc) F[pj * f + rl] += C[(int64_t)jj * mc + lane];
+    // the children's blocks, eight columns in flight
+    for (int kb = k0; kb < k1; kb += 64) {
+        if (kb > k0) ch.load(S, kb, k1, lane);
+        for (int kc = 0; kc < min(64, k1 - kb); ++kc) {
+            const int64_t co = lane_int64(ch.cb, kc), rp = lane_int64(ch.rel, kc);
+            const int mc = __builtin_amdgcn_readlane(ch.m, kc);
+            if (co < 0 || mc == 0) continue;
+            const T* C = cbpool + co + min(lane, mc - 1);
+            const int rl = S.relind[rp + min(lane, mc - 1)];
+            for (int j0 = 0; j0 < mc; j0 += 8) {
+                T v[8];
+#pragma unroll
+                for (int u = 0; u < 8; ++u) v[u] = C[(int64_t)min(j0 + u, mc - 1) * mc];
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int u = 0; u < 8; ++u) {
+                    const int jj = j0 + u;
+                    if (jj >= mc) break;
+                    const int pj = __builtin_amdgcn_readlane(rl, jj);
+                    if (lane >= jj && lane < mc) F[pj * f + rl] += v[u];
+                }
+            }
+            wave_sync();
         }
-        wave_sync();
     }
-    // row `lane` into registers
-    T r[TINY_F];
+    // row `lane` into registers: r[k] is column j + k at pivot j, the columns move one register left per
+    // pivot. One rolled loop body serves every pivot (unrolled over the pivots the code, fetched once
+    // per launch, cost more than the arithmetic: 22 us a launch). x: column `lane` of L11^-1, whose
+    // substitution step j reads the same broadcasts (fronts of at most FUSED_INV_MAX columns).
+    T r[TINY_F], x[FUSED_INV_MAX];
 #pragma unroll
     for (int k = 0; k < TINY_F; ++k) r[k] = (k < f && lane < f) ? F[k * f + lane] : T(0);
+#pragma unroll
+    for (int q = 0; q < FUSED_INV_MAX; ++q) x[q] = q == lane ? T(1) : T(0);
+    T* P = factor + S.panel_off[s];
+    T* o = DB + (int64_t)(S.super_ptr[s] + min(lane, w - 1)) * NB;
+    const bool inv = w <= FUSED_INV_MAX;
     int st = 0;
+#pragma unroll 1
+    for (int j = 0; j < w; ++j) {
+        const double a = (double)lane_value(r[0], j);
+        if (!st && !chol_accept(a, eps)) st = j + 1;
+        if (st) {  // the columns from a failed pivot on are left as they stand
+            if (lane < f) P[(int64_t)j * f + lane] = lane >= j ? r[0] : T(0);
+            if (inv && lane < w) o[j] = T(0);
 #pragma unroll
-    for (int j = 0; j < TINY_F; ++j) {
-        if (j < w && !st) {
-            const double a = (double)lane_value(r[j], j);
-            if (!chol_accept(a, eps)) {
-                st = j + 1;
-            } else {
-                const T d = T(sqrt(fmax(a, eps)));
-                const T rd = T(1) / d;
-                if (lane == j) r[j] = d;
-                else if (lane > j) r[j] = r[j] * rd;
+            for (int k = 1; k < TINY_F; ++k) r[k - 1] = r[k];
+            continue;
+        }
+        const T d = T(sqrt(fmax(a, eps)));
+        const T rd = T(1) / d;
+        const T l = lane == j ? d : r[0] * rd;
+        if (lane < f) P[(int64_t)j * f + lane] = lane >= j ? l : T(0);
+        const T xm = x[0] * rd;
+        if (inv && lane < w) o[j] = xm;
 #pragma unroll
-                for (int k = j + 1; k < TINY_F; ++k) {
-                    if (k < f) {
-                        const T lk = lane_value(r[j], k);
-                        if (lane >= k) {
-                            const T prod = r[j] * lk;
-                            r[k] = r[k] - prod;
-                        }
-                    }
+        for (int kb = 0; kb < TINY_F; kb += 8) {
+            if (kb < f - j) {
+#pragma unroll
+                for (int k = kb == 0 ? 1 : kb; k < kb + 8; ++k) {
+                    const T lk = lane_value(l, j + k);  // (entries above the diagonal: never stored)
+                    const T prod = l * lk;
+                    r[k - 1] = r[k] - prod;
+                    if (k < FUSED_INV_MAX) x[k - 1] = fma(-lk, xm, x[k]);
                 }
             }
         }
     }
-    T* P = factor + S.panel_off[s];
-#pragma unroll
-    for (int j = 0; j < TINY_F; ++j)
-        if (j < w && lane < f) P[(int64_t)j * f + lane] = lane >= j ? r[j] : T(0);
     const int64_t co = S.cb_off[s];
     if (co >= 0) {
         T* C = cbpool + co;
 #pragma unroll
         for (int k = 0; k < TINY_F; ++k)
-            if (k >= w && k < f && lane >= k && lane < f) C[(int64_t)(k - w) * m + lane - w] = r[k];
+            if (k < m && lane >= w + k && lane < f) C[(int64_t)k * m + lane - w] = r[k];
     }
-    if (w <= FUSED_INV_MAX) {
-        // column `lane` of L11^-1: L(rr, mm) is row rr's register mm
-        T x[FUSED_INV_MAX];
-#pragma unroll
-        for (int q = 0; q < FUSED_INV_MAX; ++q) x[q] = q == lane ? T(1) : T(0);
-#pragma unroll
-        for (int mm = 0; mm < FUSED_INV_MAX; ++mm) {
-            if (mm < w) {
-                const T rinv = T(1) / lane_value(r[mm], mm);
-                x[mm] = x[mm] * rinv;
-                const T xm = x[mm];
-#pragma unroll
-                for (int rr = mm + 1; rr < FUSED_INV_MAX; ++rr)
-                    if (rr < w) x[rr] = fma(-lane_value(r[mm], rr), xm, x[rr]);
-            }
-        }
-        if (lane < w) {
-            T* o = DB + (int64_t)(S.super_ptr[s] + lane) * NB;
-#pragma unroll
-            for (int q = 0; q < FUSED_INV_MAX; ++q) o[q] = q < w ? x[q] : T(0);
-#pragma unroll
-            for (int q = FUSED_INV_MAX; q < NB; ++q) o[q] = T(0);
-        }
-    }
+    if (inv && lane < w)
+        for (int q = w; q < NB; ++q) o[q] = T(0);
     if (lane == 0) status[s] = st;
 }
 
@@ -1286,12 +1294,22 @@ __global__ void k_schur_export(DevSym S, int s, const T* __restrict__ factor, in
 // ---------------------------------------------------------------------------
 // launchers
 
+// A level's fronts of at most 64 rows (nlow of them, listed first) get a launch of their own, half the
+// registers and LDS of the larger ones and so twice the workgroups on a CU, where the level has only
+// those or they alone are more than the chip holds at two a CU; else one launch takes all. (Levels of
+// 2,114 and 5,308 such fronts in FP32: 67 us a launch instead of 105 among the larger ones; a level
+// of few gains nothing from the split and would pay a launch.)
+constexpr int LOW_SPLIT = 512;
 template <typename T>
-void launch_front_small_chol(hipStream_t st, const DevSym& S, const int32_t* fronts, int nfronts, int fmax,
+void launch_front_small_chol(hipStream_t st, const DevSym& S, const int32_t* fronts, int nfronts, int nlow, int fmax,
                              const double* nz, T* factor, T* cbpool, T* DB, int32_t* status, double eps) {
-    size_t lds = (size_t)fmax * fmax * sizeof(T);
-    hipLaunchKernelGGL(k_front_small_chol<T>, dim3(nfronts), dim3(256), lds, st, S, fronts, nz, factor, cbpool, DB,
-                       status, eps);
+    const int n1 = nlow == nfronts || nlow > LOW_SPLIT ? nlow : 0, fl = std::min(fmax, 64);
+    if (n1)
+        hipLaunchKernelGGL((k_front_small_chol<T, 1>), dim3(n1), dim3(256), (size_t)fl * fl * sizeof(T), st, S, fronts,
+                           nz, factor, cbpool, DB, status, eps);
+    if (n1 < nfronts)
+        hipLaunchKernelGGL((k_front_small_chol<T, 2>), dim3(nfronts - n1), dim3(256), (size_t)fmax * fmax * sizeof(T),
+                           st, S, fronts + n1, nz, factor, cbpool, DB, status, eps);
 }
 
 template <typename T>
@@ -1405,7 +1423,7 @@ void launch_fill_i32(hipStream_t st, int32_t* p, int64_t n, int32_t v) {
 }
 
 #define INST(T)                                                                                                   \
-    template void launch_front_small_chol<T>(hipStream_t, const DevSym&, const int32_t*, int, int, const double*, \
+    template void launch_front_small_chol<T>(hipStream_t, const DevSym&, const int32_t*, int, int, int, const double*, \
                                              T*, T*, T*, int32_t*, double);                                       \
     template void launch_subtree_chol<T>(hipStream_t, const DevSym&, const int32_t*, const int32_t*, int, int, int, \
                                          const int32_t*, const int32_t*, const double*, T*, T*, T*, int32_t*,     \

@@ -100,7 +100,7 @@ struct Level {
     // Cholesky: the small fronts of at most TINY_F rows (one wave each) and the others
     std::vector<int32_t> tiny, mid;
     int64_t off_tiny = 0, off_mid = 0;
-    int fmax_mid = 0;
+    int fmax_mid = 0, nlow_mid = 0;  // nlow_mid: the first of mid, of at most 64 rows
     double tiny_flops = 0, tiny_bytes = 0;
     std::vector<Launch> plan;           // large-front launches of this level
     std::vector<Launch> fwd_plan, bwd_plan;  // large-front solve launches (per right-hand side work)
@@ -640,6 +640,8 @@ int build_schedule(sds_handle* h, int dtype) {
         L.off_tiny = (int64_t)flist.size();
         flist.insert(flist.end(), L.tiny.begin(), L.tiny.end());
         L.off_mid = (int64_t)flist.size();
+        L.nlow_mid = (int)(std::stable_partition(L.mid.begin(), L.mid.end(), [&](int32_t s) { return h->fnrows[s] <= 64; }) -
+                           L.mid.begin());
         flist.insert(flist.end(), L.mid.begin(), L.mid.end());
     }
     for (auto& L : h->levels) {
@@ -1454,7 +1456,7 @@ int factorize_cholesky(sds_handle* h, const double* nz, double eps, const volati
                 timed(h, SDS_K_FRONT_SMALL, tiny ? L.small_flops - L.tiny_flops : L.small_flops,
                       tiny ? L.small_bytes - L.tiny_bytes : L.small_bytes, [&] {
                           if (h->small_kind == 0)
-                              launch_front_small_chol<T>(st, h->dsym, fl, nf, fm, nz, factor, cb, DB, h->status, eps);
+                              launch_front_small_chol<T>(st, h->dsym, fl, nf, L.nlow_mid, fm, nz, factor, cb, DB, h->status, eps);
                           else
                               launch_front_col_chol<T>(st, h->dsym, fl, nf, fm, nz, factor, cb, DB, h->status, eps);
                       });

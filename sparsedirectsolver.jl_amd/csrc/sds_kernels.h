@@ -25,7 +25,7 @@ template <typename T>
 void launch_front_tiny_chol(hipStream_t st, const DevSym& S, const int32_t* fronts, int nfronts, const double* nz,
                             T* factor, T* cbpool, T* DB, int32_t* status, double eps);
 template <typename T>
-void launch_front_small_chol(hipStream_t st, const DevSym& S, const int32_t* fronts, int nfronts, int fmax,
+void launch_front_small_chol(hipStream_t st, const DevSym& S, const int32_t* fronts, int nfronts, int nlow, int fmax,
                              const double* nz, T* factor, T* cbpool, T* DB, int32_t* status, double eps);
 template <typename T>
 void launch_big_zero_scatter(hipStream_t st, const DevSym& S, const Task* tasks, int n, const double* nz, T* factor,
