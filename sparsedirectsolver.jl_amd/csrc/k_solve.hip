@@ -12,6 +12,7 @@
 //
 // Reference counterparts: src/solve/permute.jl:68-90, src/solve/sweeps.jl:438-570,
 // src/solve/refinement.jl:136-200.
+#include "k_dense.h"
 #include "sds_common.h"
 #include "sds_kernels.h"
 
@@ -100,48 +101,109 @@ __device__ inline void load_block(T (*B)[NB + 1], const T* __restrict__ P, int f
     }
 }
 
-// solve a diagonal block held in LDS: xs[i * nrhs + r] <- L_bb^-1 xs (lower = 1) or
-// L_bb^-T xs (lower = 0); Lb[j][i] = L(k + i, k + j). One wave per right-hand side group,
-// lane i holds row i in a register; the solved value moves between lanes by shuffles.
+// solve a unit triangular diagonal block held in LDS: xs[i * nrhs + r] <- L_bb^-1 xs (LOWER) or
+// L_bb^-T xs; Lb[j][i] = L(k + i, k + j). One wave per right-hand side group, lane i holds row i in a
+// register; the solved value of step j is read from its lane (v_readlane: a shuffle through the LDS
+// and a divergent update per step took most of 12 us a launch of k_bwd_step, 7.5 now) and eight steps' entries are
+// loaded together. Steps past nb and lanes whose row is done take no part (selects).
 // xs is read before and written after the solve only (callers put barriers around it).
-template <typename T>
-__device__ void block_solve(const T (*Lb)[NB + 1], T* xs, int nb, int nrhs, int unit, int lower) {
-    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, nw = blockDim.x >> 6;
+template <typename T, bool LOWER>
+__device__ __forceinline__ void block_solve(const T (*Lb)[NB + 1], T* xs, int nb, int nrhs) {
+    const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), nw = blockDim.x >> 6;
     for (int r = wv; r < nrhs; r += nw) {
-        T v = lane < nb ? xs[lane * nrhs + r] : T(0);
-        if (lower) {
-            for (int j = 0; j < nb; ++j) {
-                T xj = __shfl(v, j);
-                if (!unit) xj /= Lb[j][j];
-                if (lane == j) v = xj;
-                if (lane > j && lane < nb) v -= Lb[j][lane] * xj;
+        T v = xs[min(lane, nb - 1) * nrhs + r];
+#pragma unroll 1
+        for (int q0 = 0; q0 < nb; q0 += 8) {
+            T l[8];
+#pragma unroll
+            for (int q = 0; q < 8; ++q) {
+                const int j = LOWER ? min(q0 + q, nb - 1) : max(nb - 1 - q0 - q, 0);
+                l[q] = LOWER ? Lb[j][lane] : Lb[lane][j];
             }
-        } else {
-            for (int j = nb - 1; j >= 0; --j) {
-                T xj = __shfl(v, j);
-                if (!unit) xj /= Lb[j][j];
-                if (lane == j) v = xj;
-                if (lane < j) v -= Lb[lane][j] * xj;
+#pragma unroll
+            for (int q = 0; q < 8; ++q) {
+                const int j = LOWER ? q0 + q : nb - 1 - q0 - q;
+                const T xj = lane_value(v, max(j, 0));
+                const T t = v - l[q] * xj;
+                v = (LOWER ? lane > j : lane < j) ? t : v;
             }
         }
         if (lane < nb) xs[lane * nrhs + r] = v;
     }
 }
 
-// forward sweep over the fronts of one level, one workgroup per front.
-// unit: unit diagonal (LDL^T, LU); piv (nullable): local pivot order of each
-// supernode (global factor columns), applied to its slice first through the
-// scratch Z (same shape as Y; a front only touches its own columns there).
+// up to 64 panel entries of row i in the columns k..k + nb - 1 (registers, all in flight together)
+template <typename T>
+__device__ __forceinline__ void load_row(const T* __restrict__ P, int f, int k, int nb, int i, T (&l)[NB]) {
+#pragma unroll
+    for (int g = 0; g < NB; g += 16) {
+        int n = __builtin_amdgcn_readfirstlane(nb);
+        asm volatile("" : "+s"(n));  // (the columns' addresses stay inside the callers' loops)
+        if (g < n) {
+#pragma unroll
+            for (int jj = 0; jj < 16; ++jj) l[g + jj] = P[(int64_t)(k + min(g + jj, n - 1)) * f + i];
+        }
+    }
+    __builtin_amdgcn_sched_barrier(0);
+}
+// row[r] (-= or +=) sum_j l[j] xs[j nrhs + r] over the nb columns, for NR right-hand sides
+template <int NR, typename T>
+__device__ __forceinline__ void row_dot(T* row, const T (&l)[NB], int nb, const T* xs, int nrhs, bool sub) {
+    T acc[NR];
+#pragma unroll
+    for (int r = 0; r < NR; ++r) acc[r] = T(0);
+#pragma unroll
+    for (int j0 = 0; j0 < NB; j0 += 8) {
+        int n = __builtin_amdgcn_readfirstlane(nb);
+        asm volatile("" : "+s"(n));  // (64 comparisons moved ahead of the sums would take two registers each)
+        if (j0 < n) {
+#pragma unroll
+            for (int j = j0; j < j0 + 8; ++j) {
+                if (j < n) {
+#pragma unroll
+                    for (int r = 0; r < NR; ++r) acc[r] += l[j] * xs[j * nrhs + r];
+                }
+            }
+        }
+    }
+    T o[NR];
+#pragma unroll
+    for (int r = 0; r < NR; ++r) o[r] = row[r];
+#pragma unroll
+    for (int r = 0; r < NR; ++r) row[r] = sub ? o[r] - acc[r] : o[r] + acc[r];
+}
+// the same for nr <= 4 right-hand sides
+template <typename T>
+__device__ __forceinline__ void row_dots(T* row, const T (&l)[NB], int nb, const T* xs, int nrhs, int nr, bool sub) {
+    if (nr == 1)
+        row_dot<1>(row, l, nb, xs, nrhs, sub);
+    else if (nr == 2)
+        row_dot<2>(row, l, nb, xs, nrhs, sub);
+    else if (nr == 3)
+        row_dot<3>(row, l, nb, xs, nrhs, sub);
+    else
+        row_dot<4>(row, l, nb, xs, nrhs, sub);
+}
+
+// forward sweep over the small fronts (w <= NB) of one level, one workgroup per front; unit
+// diagonal (LDL^T, LU). piv (nullable): local pivot order of each supernode (global factor columns),
+// applied as its slice is read. Bound: latency (a chain of dependent loads, then the 64 steps of
+// the block): the block's entries are asked for before the children's updates are added, a thread's
+// row of the panel before the block is solved (18 -> 14 us a launch of a 32 x 32 x 32 LU level, FP64).
 template <typename T>
 __global__ void __launch_bounds__(256) k_fwd(DevSym S, const int32_t* __restrict__ fronts,
                                             const T* __restrict__ factor, T* __restrict__ Y, T* __restrict__ U,
-                                            T* __restrict__ Z, int nrhs, int unit, const int32_t* __restrict__ piv) {
+                                            int nrhs, const int32_t* __restrict__ piv) {
+    extern __shared__ __align__(16) unsigned char smem_raw[];
+    T* xs = reinterpret_cast<T*>(smem_raw);  // 64 * nrhs
+    __shared__ T Lb[NB][NB + 1];
     const int s = fronts[blockIdx.x];
     const int f = S.fnrows[s], w = S.fncols[s], m = f - w;
     const int c0 = S.super_ptr[s];
     const int tid = threadIdx.x, nt = blockDim.x;
     const T* P = factor + S.panel_off[s];
     T* us = S.uv_off[s] >= 0 ? U + S.uv_off[s] * nrhs : nullptr;
+    load_block<T>(Lb, P, f, 0, 0, w, w);
     if (us)
         for (int q = tid; q < m * nrhs; q += nt) us[q] = T(0);
     __syncthreads();
@@ -162,100 +224,127 @@ __global__ void __launch_bounds__(256) k_fwd(DevSym S, const int32_t* __restrict
         __syncthreads();
     }
     T* y = Y + (int64_t)c0 * nrhs;
-    if (piv) {
-        T* z = Z + (int64_t)c0 * nrhs;
-        for (int q = tid; q < w * nrhs; q += nt) {
-            const int kk = q / nrhs, r = q - kk * nrhs;
-            z[q] = Y[(int64_t)piv[c0 + kk] * nrhs + r];
-        }
-        __syncthreads();
-        for (int q = tid; q < w * nrhs; q += nt) y[q] = z[q];
-        __syncthreads();
+    for (int q = tid; q < w * nrhs; q += nt) {
+        const int kk = q / nrhs, r = q - kk * nrhs;
+        xs[q] = piv ? Y[(int64_t)piv[c0 + kk] * nrhs + r] : y[q];
     }
-    __shared__ T Lb[NB][NB + 1];
-    __shared__ T xs[NB * MAX_NRHS];
-    for (int j0 = 0; j0 < w; j0 += NB) {
-        const int nb = min(NB, w - j0), j1 = j0 + nb;
-        load_block<T>(Lb, P, f, j0, j0, nb, nb);
-        for (int q = tid; q < nb * nrhs; q += nt) xs[q] = y[j0 * nrhs + q];
-        __syncthreads();
-        block_solve<T>(Lb, xs, nb, nrhs, unit, 1);
-        __syncthreads();
-        for (int q = tid; q < nb * nrhs; q += nt) y[j0 * nrhs + q] = xs[q];
-        // rows below the chunk: in L11 (subtract now) or below the supernode (update vector)
-        for (int q = tid; q < (f - j1) * nrhs; q += nt) {
-            const int i = j1 + q / nrhs, r = q % nrhs;
-            T t = T(0);
-#pragma unroll 16
-            for (int j = 0; j < nb; ++j) t += P[(int64_t)(j0 + j) * f + i] * xs[j * nrhs + r];
-            if (i < w)
-                y[i * nrhs + r] -= t;
-            else if (us)
-                us[(i - w) * nrhs + r] += t;
-        }
-        __syncthreads();
+    // the rows below: item q is row w + q % m, the right-hand sides 4 (q / m)...
+    const int items = us ? m * ((nrhs + 3) >> 2) : 0;
+    T l[NB];
+    if (tid < items) load_row<T>(P, f, 0, w, w + tid % m, l);
+    __syncthreads();
+    block_solve<T, true>(Lb, xs, w, nrhs);
+    __syncthreads();
+    for (int q = tid; q < w * nrhs; q += nt) y[q] = xs[q];
+#pragma unroll 1
+    for (int q = tid; q < items; q += nt) {
+        const int i = q % m, rb = 4 * (q / m);
+        if (q != tid) load_row<T>(P, f, 0, w, w + i, l);
+        T* row = us + (int64_t)i * nrhs + rb;
+        row_dots<T>(row, l, w, xs + rb, nrhs, min(4, nrhs - rb), false);
     }
 }
 
-// backward sweep over the fronts of one level, one workgroup (4 waves) per front:
-// x_j = (y_j - sum_{i > j} L[i, j] x_i) / L[j, j], columns in chunks of 64 from the
-// last; the dot products over the rows past the chunk one wave per column, the
-// substitution inside the chunk on LDS copies. piv (nullable): undo the local pivot
-// order afterwards through the scratch Z.
+// the sum of v over the wave in every lane: lanes 32, 16, 8, 4, 2, 1 apart in that order (a row's
+// rotations pair the same lanes as exclusive-or shuffles once the larger distances are summed)
+template <int CTRL>
+__device__ inline double row_rotate(double v) {
+    int2 x = __builtin_bit_cast(int2, v);
+    x.x = __builtin_amdgcn_update_dpp(0, x.x, CTRL, 0xf, 0xf, false);
+    x.y = __builtin_amdgcn_update_dpp(0, x.y, CTRL, 0xf, 0xf, false);
+    return __builtin_bit_cast(double, x);
+}
+template <int CTRL>
+__device__ inline float row_rotate(float v) {
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xf, 0xf, false));
+}
+template <typename T>
+__device__ inline T wave_sum(T v) {
+    v += __shfl_xor(v, 32);
+    v += __shfl_xor(v, 16);
+    v += row_rotate<0x128>(v);
+    v += row_rotate<0x124>(v);
+    v += row_rotate<0x122>(v);
+    return v + row_rotate<0x121>(v);
+}
+
+// backward sweep over the small fronts (w <= NB) of one level, one workgroup (4 waves) per front:
+// x_j = y_j - sum_{i > j} L[i, j] x_i (unit diagonal). The values of the rows below are gathered
+// once, 256 rows and RB right-hand sides at a time, into LDS; a wave takes sixteen columns together,
+// lanes along the rows, so that sixteen loads a lane are in flight; then the block is solved from
+// LDS. piv (nullable): the local pivot order is undone as the solved values are written. Bound:
+// latency (gathering the rows anew for each column and 96 shuffles per column took 37 us a launch of
+// a 32 x 32 x 32 LU level in FP64 instead of 12).
 template <typename T, int RB>
 __global__ void __launch_bounds__(256) k_bwd(DevSym S, const int32_t* __restrict__ fronts,
-                                            const T* __restrict__ factor, T* __restrict__ Y, T* __restrict__ Z,
-                                            int nrhs, int unit, const int32_t* __restrict__ piv) {
+                                            const T* __restrict__ factor, T* __restrict__ Y, int nrhs,
+                                            const int32_t* __restrict__ piv) {
     extern __shared__ __align__(16) unsigned char smem_raw[];
-    T* xs = reinterpret_cast<T*>(smem_raw);  // 64 * nrhs: the chunk's values
-    T* ts = xs + 64 * nrhs;                  // 64 * nrhs: dot products past the chunk
-    __shared__ T Lb[NB][NB + 1];             // the chunk's diagonal block
+    T* xs = reinterpret_cast<T*>(smem_raw);  // 64 * nrhs: the block's values
+    T* ts = xs + 64 * nrhs;                  // 64 * nrhs: dot products with the rows below
+    __shared__ T Lb[NB][NB + 1];             // the diagonal block
+    __shared__ T Yc[RB][256];
     const int s = fronts[blockIdx.x];
     const int f = S.fnrows[s], w = S.fncols[s];
     const int c0 = S.super_ptr[s];
-    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+    const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
     const T* P = factor + S.panel_off[s];
     const int32_t* rows = S.rowval + S.rowptr[s];
     T* y = Y + (int64_t)c0 * nrhs;
-    for (int j1 = w; j1 > 0; j1 -= 64) {
-        const int j0 = max(j1 - 64, 0);
-        for (int j = j0 + wv; j < j1; j += 4) {
-            for (int rb = 0; rb < nrhs; rb += RB) {
-                T acc[RB];
+    load_block<T>(Lb, P, f, 0, 0, w, w);
+    for (int rb = 0; rb < nrhs; rb += RB) {
+        T acc[16][RB];
 #pragma unroll
-                for (int r = 0; r < RB; ++r) acc[r] = T(0);
-                for (int i = j1 + lane; i < f; i += 64) {
-                    const T l = P[(int64_t)j * f + i];
-                    const T* yr = Y + (int64_t)rows[i] * nrhs + rb;
+        for (int c = 0; c < 16; ++c)
 #pragma unroll
-                    for (int r = 0; r < RB; ++r)
-                        if (rb + r < nrhs) acc[r] += l * yr[r];
-                }
+            for (int r = 0; r < RB; ++r) acc[c][r] = T(0);
+        for (int i0 = w; i0 < f; i0 += 256) {
+            const int64_t row = rows[min(i0 + tid, f - 1)];
+#pragma unroll
+            for (int r = 0; r < RB; ++r) Yc[r][tid] = Y[row * nrhs + min(rb + r, nrhs - 1)];
+            __syncthreads();
+#pragma unroll 1
+            for (int u = 0; u < 256 && i0 + u < f; u += 64) {
+                const int i = i0 + u + lane;
+                T l[16];
+#pragma unroll
+                for (int c = 0; c < 16; ++c) l[c] = P[(int64_t)min(wv + 4 * c, w - 1) * f + min(i, f - 1)];
+                __builtin_amdgcn_sched_barrier(0);
+                T yv[RB];
+#pragma unroll
+                for (int r = 0; r < RB; ++r) yv[r] = Yc[r][u + lane];
+#pragma unroll
+                for (int c = 0; c < 16; ++c)
+#pragma unroll
+                    for (int r = 0; r < RB; ++r) {
+                        const T t = acc[c][r] + l[c] * yv[r];
+                        acc[c][r] = i < f ? t : acc[c][r];
+                    }
+            }
+            __syncthreads();
+        }
+#pragma unroll
+        for (int c = 0; c < 16; ++c) {
+            if (wv + 4 * c < w) {
 #pragma unroll
                 for (int r = 0; r < RB; ++r) {
-                    T v = acc[r];
-                    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
-                    if (lane == 0 && rb + r < nrhs) ts[(j - j0) * nrhs + rb + r] = v;
+                    const T v = wave_sum<T>(acc[c][r]);
+                    if (lane == 0 && rb + r < nrhs) ts[(wv + 4 * c) * nrhs + rb + r] = v;
                 }
             }
         }
-        load_block<T>(Lb, P, f, j0, j0, j1 - j0, j1 - j0);
-        __syncthreads();
-        for (int q = tid; q < (j1 - j0) * nrhs; q += 256) xs[q] = y[j0 * nrhs + q] - ts[q];
-        __syncthreads();
-        block_solve<T>(Lb, xs, j1 - j0, nrhs, unit, 0);
-        __syncthreads();
-        for (int q = tid; q < (j1 - j0) * nrhs; q += 256) y[j0 * nrhs + q] = xs[q];
-        __syncthreads();
     }
-    if (piv) {
-        T* z = Z + (int64_t)c0 * nrhs;
-        for (int q = tid; q < w * nrhs; q += 256) z[q] = y[q];
-        __syncthreads();
-        for (int q = tid; q < w * nrhs; q += 256) {
-            const int kk = q / nrhs, r = q - kk * nrhs;
-            Y[(int64_t)piv[c0 + kk] * nrhs + r] = z[q];
-        }
+    __syncthreads();
+    for (int q = tid; q < w * nrhs; q += 256) xs[q] = y[q] - ts[q];
+    __syncthreads();
+    block_solve<T, false>(Lb, xs, w, nrhs);
+    __syncthreads();
+    for (int q = tid; q < w * nrhs; q += 256) {
+        const int kk = q / nrhs, r = q - kk * nrhs;
+        if (piv)
+            Y[(int64_t)piv[c0 + kk] * nrhs + r] = xs[q];
+        else
+            y[q] = xs[q];
     }
 }
 
@@ -307,51 +396,39 @@ __global__ void __launch_bounds__(256) k_fwd_pull(DevSym S, const Task* __restri
 
 // forward block step: every workgroup solves the diagonal block [k, k + nb) (from Y) and
 // applies it to its tile of 256 rows below: rows < w of Y, rows >= w of the update vector.
-// The solved block goes to Z (written by the task with c = 1). task: (s, k, row0, c)
+// The solved block goes to Z (written by the task with c = 1). task: (s, k, row0, c). Bound: latency
+// (the block's entries, its 64 steps, the row): 17.6 -> 9.4 us a launch of a 32 x 32 x 32 LU with the
+// row's entries asked for before the block is solved and the steps' values read from their lanes.
 template <typename T>
 __global__ void __launch_bounds__(256) k_fwd_step(DevSym S, const Task* __restrict__ tasks,
                                                  const T* __restrict__ factor, T* __restrict__ Y, T* __restrict__ U,
-                                                 T* __restrict__ Z, int nrhs, int unit) {
+                                                 T* __restrict__ Z, int nrhs) {
+    extern __shared__ __align__(16) unsigned char smem_raw[];
+    T* xs = reinterpret_cast<T*>(smem_raw);  // 64 * nrhs
     __shared__ T Lb[NB][NB + 1];
-    __shared__ T xs[NB * MAX_NRHS];
     const Task t = tasks[blockIdx.x];
     const int s = t.s, f = S.fnrows[s], w = S.fncols[s], k = t.a, row0 = t.b;
     const int nb = min(NB, w - k);
     const int c0 = S.super_ptr[s];
     const int tid = threadIdx.x;
     const T* P = factor + S.panel_off[s];
+    T* us = S.uv_off[s] >= 0 ? U + S.uv_off[s] * nrhs : nullptr;
+    const int i = row0 + tid;
+    const bool on = i < min(row0 + 256, f) && (i < w || us);
     load_block<T>(Lb, P, f, k, k, nb, nb);
     for (int q = tid; q < nb * nrhs; q += 256) xs[q] = Y[(int64_t)(c0 + k) * nrhs + q];
+    T l[NB];  // the row's panel entries, on their way while the block is solved
+    load_row<T>(P, f, k, nb, min(i, f - 1), l);
     __syncthreads();
-    block_solve<T>(Lb, xs, nb, nrhs, unit, 1);
+    block_solve<T, true>(Lb, xs, nb, nrhs);
     __syncthreads();
     if (t.c)
         for (int q = tid; q < nb * nrhs; q += 256) Z[(int64_t)(c0 + k) * nrhs + q] = xs[q];
-    const int i = row0 + tid;
-    T* us = S.uv_off[s] >= 0 ? U + S.uv_off[s] * nrhs : nullptr;
-    if (i < min(row0 + 256, f) && (i < w || us)) {
-        for (int rb = 0; rb < nrhs; rb += 8) {
-            const int nr = min(8, nrhs - rb);
-            T acc[8];
-#pragma unroll
-            for (int r = 0; r < 8; ++r) acc[r] = T(0);
-            for (int j0 = 0; j0 < nb; j0 += 16) {
-                // sixteen panel entries of the row in flight together (clamped to the block)
-                T l[16];
-#pragma unroll
-                for (int jj = 0; jj < 16; ++jj) l[jj] = P[(int64_t)(k + min(j0 + jj, nb - 1)) * f + i];
-                __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-                for (int jj = 0; jj < 16; ++jj) {
-                    if (j0 + jj >= nb) break;
-#pragma unroll
-                    for (int r = 0; r < 8; ++r)
-                        if (r < nr) acc[r] += l[jj] * xs[(j0 + jj) * nrhs + rb + r];
-                }
-            }
-            rmw8<T>(i < w ? Y + (int64_t)(c0 + i) * nrhs + rb : us + (int64_t)(i - w) * nrhs + rb, acc, nr, i < w);
-        }
-    }
+    if (!on) return;
+    T* row = i < w ? Y + (int64_t)(c0 + i) * nrhs : us + (int64_t)(i - w) * nrhs;
+#pragma unroll 1
+    for (int rb = 0; rb < nrhs; rb += 4)
+        row_dots<T>(row + rb, l, nb, xs + rb, nrhs, min(4, nrhs - rb), i < w);
 }
 
 // after the block steps of a level: the solved values of the fronts' own columns from Z
@@ -463,10 +540,11 @@ __global__ void __launch_bounds__(256) k_bwd_l21_sum(DevSym S, const Task* __res
 template <typename T>
 __global__ void __launch_bounds__(256) k_bwd_step(DevSym S, const Task* __restrict__ tasks,
                                                  const T* __restrict__ factor, T* __restrict__ Y, T* __restrict__ Z,
-                                                 int nrhs, int unit) {
+                                                 int nrhs) {
+    extern __shared__ __align__(16) unsigned char smem_raw[];
+    T* xs = reinterpret_cast<T*>(smem_raw);  // 64 * nrhs
     __shared__ T Lb[NB][NB + 1];
     __shared__ T Lt[NB][NB + 1];  // Lt[jj][i] = L(k + i, col0 + jj)
-    __shared__ T xs[NB * MAX_NRHS];
     const Task t = tasks[blockIdx.x];
     const int s = t.s, f = S.fnrows[s], w = S.fncols[s], k = t.a, col0 = t.b;
     const int nb = min(NB, w - k);
@@ -478,7 +556,7 @@ __global__ void __launch_bounds__(256) k_bwd_step(DevSym S, const Task* __restri
     load_block<T>(Lt, P, f, k, col0, nb, ncol);
     for (int q = tid; q < nb * nrhs; q += 256) xs[q] = Y[(int64_t)(c0 + k) * nrhs + q];
     __syncthreads();
-    block_solve<T>(Lb, xs, nb, nrhs, unit, 0);
+    block_solve<T, false>(Lb, xs, nb, nrhs);
     __syncthreads();
     if (t.c)
         for (int q = tid; q < nb * nrhs; q += 256) Z[(int64_t)(c0 + k) * nrhs + q] = xs[q];
@@ -639,16 +717,20 @@ void launch_permute_out(hipStream_t st, int n, int nrhs, const int32_t* perm, co
 }
 
 template <typename T>
-void launch_fwd(hipStream_t st, const DevSym& S, const int32_t* fronts, int nfronts, const T* factor, T* Y, T* U, T* Z,
-                int nrhs, int unit, const int32_t* piv) {
-    hipLaunchKernelGGL(k_fwd<T>, dim3(nfronts), dim3(256), 0, st, S, fronts, factor, Y, U, Z, nrhs, unit, piv);
+void launch_fwd(hipStream_t st, const DevSym& S, const int32_t* fronts, int nfronts, const T* factor, T* Y, T* U,
+                int nrhs, const int32_t* piv) {
+    hipLaunchKernelGGL(k_fwd<T>, dim3(nfronts), dim3(256), (size_t)64 * nrhs * sizeof(T), st, S, fronts, factor, Y, U,
+                       nrhs, piv);
 }
 
+// right-hand sides taken together: as many as there are, up to the four whose sums (16 columns each)
+// fit the registers
 template <typename T>
-void launch_bwd(hipStream_t st, const DevSym& S, const int32_t* fronts, int nfronts, const T* factor, T* Y, T* Z,
-                int nrhs, int unit, const int32_t* piv) {
-    size_t lds = (size_t)128 * nrhs * sizeof(T);
-    hipLaunchKernelGGL((k_bwd<T, 8>), dim3(nfronts), dim3(256), lds, st, S, fronts, factor, Y, Z, nrhs, unit, piv);
+void launch_bwd(hipStream_t st, const DevSym& S, const int32_t* fronts, int nfronts, const T* factor, T* Y, int nrhs,
+                const int32_t* piv) {
+    const size_t lds = (size_t)128 * nrhs * sizeof(T);
+    auto kernel = nrhs == 1 ? k_bwd<T, 1> : nrhs == 2 ? k_bwd<T, 2> : k_bwd<T, 4>;
+    hipLaunchKernelGGL(kernel, dim3(nfronts), dim3(256), lds, st, S, fronts, factor, Y, nrhs, piv);
 }
 
 template <typename T>
@@ -659,8 +741,9 @@ void launch_fwd_pull(hipStream_t st, const DevSym& S, const Task* tasks, int n, 
 
 template <typename T>
 void launch_fwd_step(hipStream_t st, const DevSym& S, const Task* tasks, int n, const T* factor, T* Y, T* U, T* Z,
-                     int nrhs, int unit) {
-    hipLaunchKernelGGL(k_fwd_step<T>, dim3(n), dim3(256), 0, st, S, tasks, factor, Y, U, Z, nrhs, unit);
+                     int nrhs) {
+    hipLaunchKernelGGL(k_fwd_step<T>, dim3(n), dim3(256), (size_t)64 * nrhs * sizeof(T), st, S, tasks, factor, Y, U, Z,
+                       nrhs);
 }
 
 template <typename T>
@@ -683,9 +766,9 @@ void launch_bwd_l21_sum(hipStream_t st, const DevSym& S, const Task* tasks, int 
 int bwd_l21_chunk() { return L21_CHUNK; }
 
 template <typename T>
-void launch_bwd_step(hipStream_t st, const DevSym& S, const Task* tasks, int n, const T* factor, T* Y, T* Z, int nrhs,
-                     int unit) {
-    hipLaunchKernelGGL(k_bwd_step<T>, dim3(n), dim3(256), 0, st, S, tasks, factor, Y, Z, nrhs, unit);
+void launch_bwd_step(hipStream_t st, const DevSym& S, const Task* tasks, int n, const T* factor, T* Y, T* Z, int nrhs) {
+    hipLaunchKernelGGL(k_bwd_step<T>, dim3(n), dim3(256), (size_t)64 * nrhs * sizeof(T), st, S, tasks, factor, Y, Z,
+                       nrhs);
 }
 
 template <typename T>
@@ -731,17 +814,17 @@ void launch_residual(hipStream_t st, int n, int nrhs, const int64_t* rowptr, con
     template void launch_schur_pull<T>(hipStream_t, const DevSym&, int, T*, const T*, int);                        \
     template void launch_permute_out<T>(hipStream_t, int, int, const int32_t*, const T*, double*, int64_t, int,     \
                                         const int32_t*, const double*);                                             \
-    template void launch_fwd<T>(hipStream_t, const DevSym&, const int32_t*, int, const T*, T*, T*, T*, int, int,    \
+    template void launch_fwd<T>(hipStream_t, const DevSym&, const int32_t*, int, const T*, T*, T*, int,               \
                                 const int32_t*);                                                                    \
-    template void launch_bwd<T>(hipStream_t, const DevSym&, const int32_t*, int, const T*, T*, T*, int, int,        \
+    template void launch_bwd<T>(hipStream_t, const DevSym&, const int32_t*, int, const T*, T*, int,                  \
                                 const int32_t*);                                                                    \
     template void launch_diag<T>(hipStream_t, int, int, const T*, const int8_t*, T*);                              \
     template void launch_fwd_pull<T>(hipStream_t, const DevSym&, const Task*, int, T*, T*, T*, int, const int32_t*); \
-    template void launch_fwd_step<T>(hipStream_t, const DevSym&, const Task*, int, const T*, T*, T*, T*, int, int);  \
+    template void launch_fwd_step<T>(hipStream_t, const DevSym&, const Task*, int, const T*, T*, T*, T*, int);       \
     template void launch_finish<T>(hipStream_t, const DevSym&, const Task*, int, T*, const T*, int, const int32_t*); \
     template void launch_bwd_l21<T>(hipStream_t, const DevSym&, const Task*, int, const T*, const T*, T*, int);     \
     template void launch_bwd_l21_sum<T>(hipStream_t, const DevSym&, const Task*, int, T*, const T*, int);          \
-    template void launch_bwd_step<T>(hipStream_t, const DevSym&, const Task*, int, const T*, T*, T*, int, int);
+    template void launch_bwd_step<T>(hipStream_t, const DevSym&, const Task*, int, const T*, T*, T*, int);
 INST(double)
 INST(float)
 #undef INST

@@ -1727,7 +1727,6 @@ void sweeps(sds_handle* h, const SolveWork& W, int nrhs, int fwd, int diag, int 
     T* Y = static_cast<T*>(W.Y);
     T* Z = static_cast<T*>(W.Z);
     T* U = static_cast<T*>(W.U);
-    const int unit = h->method == M_CHOLESKY ? 0 : 1;
     const int32_t* pv = h->method == M_CHOLESKY ? nullptr : h->piv;
     const bool lu = h->method == M_LU;
     const T* ffac = lu && transposed ? Ut : L;
@@ -1810,7 +1809,7 @@ void sweeps(sds_handle* h, const SolveWork& W, int nrhs, int fwd, int diag, int 
         timed(h, kind, ln.flops * nrhs, ln.bytes + (ln.flops > 0 ? es * nrhs * ln.flops / 16 : 0), [&] {
             switch (ln.kind) {
                 case S_FWD_PULL: launch_fwd_pull<T>(st, h->dsym, t, ln.n, Y, U, Z, nrhs, fpiv); break;
-                case S_FWD_STEP: launch_fwd_step<T>(st, h->dsym, t, ln.n, ffac, Y, U, Z, nrhs, unit); break;
+                case S_FWD_STEP: launch_fwd_step<T>(st, h->dsym, t, ln.n, ffac, Y, U, Z, nrhs); break;
                 case S_FWD_FINISH: launch_finish<T>(st, h->dsym, t, ln.n, Y, Z, nrhs, nullptr); break;
                 case S_BWD_L21:
                     launch_bwd_l21<T>(st, h->dsym, t, ln.n, bfac, Y, static_cast<T*>(W.part), nrhs);
@@ -1818,7 +1817,7 @@ void sweeps(sds_handle* h, const SolveWork& W, int nrhs, int fwd, int diag, int 
                 case S_BWD_L21_SUM:
                     launch_bwd_l21_sum<T>(st, h->dsym, t, ln.n, Y, static_cast<const T*>(W.part), nrhs);
                     break;
-                case S_BWD_STEP: launch_bwd_step<T>(st, h->dsym, t, ln.n, bfac, Y, Z, nrhs, unit); break;
+                case S_BWD_STEP: launch_bwd_step<T>(st, h->dsym, t, ln.n, bfac, Y, Z, nrhs); break;
                 case S_BWD_FINISH: launch_finish<T>(st, h->dsym, t, ln.n, Y, Z, nrhs, bpiv); break;
             }
         });
@@ -1827,8 +1826,8 @@ void sweeps(sds_handle* h, const SolveWork& W, int nrhs, int fwd, int diag, int 
         for (auto& L : h->levels) {
             if (!L.ssmall.empty())
                 timed(h, SDS_K_FWD, L.fwd_flops * nrhs, L.fwd_bytes + es * nrhs * L.rhs_rows, [&] {
-                    launch_fwd<T>(st, h->dsym, h->d_fronts + L.off_ssmall, (int)L.ssmall.size(), ffac, Y, U, Z,
-                                  nrhs, unit, fpiv);
+                    launch_fwd<T>(st, h->dsym, h->d_fronts + L.off_ssmall, (int)L.ssmall.size(), ffac, Y, U, nrhs,
+                                  fpiv);
                 });
             for (const Launch& ln : L.fwd_plan) run(ln, SDS_K_FWD);
         }
@@ -1842,8 +1841,8 @@ void sweeps(sds_handle* h, const SolveWork& W, int nrhs, int fwd, int diag, int 
         for (auto it = h->levels.rbegin(); it != h->levels.rend(); ++it) {
             if (!it->ssmall.empty())
                 timed(h, SDS_K_BWD, it->fwd_flops * nrhs, it->fwd_bytes + es * nrhs * it->rhs_rows, [&] {
-                    launch_bwd<T>(st, h->dsym, h->d_fronts + it->off_ssmall, (int)it->ssmall.size(), bfac, Y, Z,
-                                  nrhs, unit, bpiv);
+                    launch_bwd<T>(st, h->dsym, h->d_fronts + it->off_ssmall, (int)it->ssmall.size(), bfac, Y, nrhs,
+                                  bpiv);
                 });
             for (const Launch& ln : it->bwd_plan) run(ln, SDS_K_BWD);
         }

@@ -142,11 +142,11 @@ void launch_permute_out(hipStream_t st, int n, int nrhs, const int32_t* perm, co
 // out = w .* nz (the matching's scaled values)
 void launch_scale_values(hipStream_t st, int64_t nnz, const double* w, const double* nz, double* out);
 template <typename T>
-void launch_fwd(hipStream_t st, const DevSym& S, const int32_t* fronts, int nfronts, const T* factor, T* Y, T* U, T* Z,
-                int nrhs, int unit, const int32_t* piv);
+void launch_fwd(hipStream_t st, const DevSym& S, const int32_t* fronts, int nfronts, const T* factor, T* Y, T* U,
+                int nrhs, const int32_t* piv);
 template <typename T>
-void launch_bwd(hipStream_t st, const DevSym& S, const int32_t* fronts, int nfronts, const T* factor, T* Y, T* Z,
-                int nrhs, int unit, const int32_t* piv);
+void launch_bwd(hipStream_t st, const DevSym& S, const int32_t* fronts, int nfronts, const T* factor, T* Y, int nrhs,
+                const int32_t* piv);
 template <typename T>
 void launch_diag(hipStream_t st, int n, int nrhs, const T* d, const int8_t* kind, T* Y);
 template <typename T>
@@ -154,7 +154,7 @@ void launch_fwd_pull(hipStream_t st, const DevSym& S, const Task* tasks, int n, 
                      const int32_t* piv);
 template <typename T>
 void launch_fwd_step(hipStream_t st, const DevSym& S, const Task* tasks, int n, const T* factor, T* Y, T* U, T* Z,
-                     int nrhs, int unit);
+                     int nrhs);
 template <typename T>
 void launch_finish(hipStream_t st, const DevSym& S, const Task* tasks, int n, T* Y, const T* Z, int nrhs,
                    const int32_t* piv);
@@ -165,8 +165,7 @@ template <typename T>
 void launch_bwd_l21_sum(hipStream_t st, const DevSym& S, const Task* tasks, int n, T* Y, const T* part, int nrhs);
 int bwd_l21_chunk();  // rows per partial sum of launch_bwd_l21
 template <typename T>
-void launch_bwd_step(hipStream_t st, const DevSym& S, const Task* tasks, int n, const T* factor, T* Y, T* Z, int nrhs,
-                     int unit);
+void launch_bwd_step(hipStream_t st, const DevSym& S, const Task* tasks, int n, const T* factor, T* Y, T* Z, int nrhs);
 // Cholesky sweeps with inverted diagonal blocks (k_solve_inv.hip)
 template <typename T>
 void launch_block_inverse(hipStream_t st, const DevSym& S, const Task* tasks, int n, T* factor, T* DB, int bs);
