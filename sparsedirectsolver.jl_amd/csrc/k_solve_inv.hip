@@ -27,6 +27,9 @@
 //             across the lanes at the end); then x_step = inverse^T (y_step - partials):
 //             k_bwd_diag (narrow) or k_sub_partials (y_step less the partials, into Z) +
 //             k_bwd_inv (wide, one wave per 8 columns, from Z into y).
+#include <algorithm>
+#include <type_traits>
+
 #include "sds_common.h"
 #include "sds_kernels.h"
 
@@ -106,31 +109,53 @@ extern __shared__ __align__(16) unsigned char sweep_lds[];
 
 
 
-// one recursive-halving exchange at lane distance D: the lanes with bit D set keep the upper
-// halves a[D, 2D), the others the lower, each adding its partner's copy
-template <int D, typename T>
-__device__ __attribute__((always_inline)) inline void halving_step(T (&a)[64], int lane) {
-    const bool up = (lane & D) != 0;
+// one exchange at lane distance D of N sums: while more than one is left the lanes with bit D set
+// keep the upper half, the others the lower, each adding its partner's copy; then both keep the one
+template <int N, int D, typename T, int M>
+__device__ __attribute__((always_inline)) inline void halving_step(T (&a)[M], int lane) {
+    if constexpr (D > 0) {
+        if constexpr (N > 1) {
+            const bool up = (lane & D) != 0;
 #pragma unroll
-    for (int v = 0; v < D; ++v) {
-        const T send = up ? a[v] : a[v + D];
-        const T keep = up ? a[v + D] : a[v];
-        a[v] = keep + __shfl_xor(send, D);
+            for (int v = 0; v < N / 2; ++v) {
+                const T send = up ? a[v] : a[v + N / 2];
+                const T keep = up ? a[v + N / 2] : a[v];
+                a[v] = keep + __shfl_xor(send, D);
+            }
+        } else {
+            a[0] = a[0] + __shfl_xor(a[0], D);
+        }
+        halving_step<(N > 1 ? N / 2 : 1), D / 2>(a, lane);
     }
 }
 
-// sum over the 64 lanes of a[v] for v < 64, reduce-scattered: lane l returns the sum of a[l]
-// (recursive halving, 63 exchanges; a fixed summation order)
-template <typename T>
-__device__ __attribute__((always_inline)) inline T wave_reduce_scatter64(T (&a)[64]) {
-    const int lane = threadIdx.x & 63;
-    halving_step<32>(a, lane);
-    halving_step<16>(a, lane);
-    halving_step<8>(a, lane);
-    halving_step<4>(a, lane);
-    halving_step<2>(a, lane);
-    halving_step<1>(a, lane);
+// sum over the 64 lanes of a[v] for v < N (a power of two), reduce-scattered: lane l returns the sum
+// of a[l N / 64] (recursive halving; the same summation order for every N)
+template <typename T, int N>
+__device__ __attribute__((always_inline)) inline T wave_reduce_scatter(T (&a)[N]) {
+    halving_step<N, 32>(a, threadIdx.x & 63);
     return a[0];
+}
+
+// Right-hand sides: the sweeps' kernels take RB of them (1, 2, 4 or 8: launch_rb) in one workgroup,
+// the grid's second dimension covers them all. One at a time a launch sums and exchanges an eighth
+// of what eight need, and more than eight are done side by side, not one group after another: with
+// 24 on a 40 x 40 x 40 Laplacian a solve takes 1.9 ms (3.4 ms in three passes per workgroup), with one
+// on 47 x 47 x 47 in FP32 a launch of k_fwd_rows 7.6 us and of k_bwd_inv 6.0 (10.9 and 11.3). A group
+// of RB gives each right-hand side the same operations in the same order.
+template <int RB, typename T>
+__device__ __attribute__((always_inline)) inline void rmw_row(T* row, const T (&a)[RB], int nr, bool sub) {
+    T o[RB];
+#pragma unroll
+    for (int r = 0; r < RB; ++r) o[r] = row[min(r, nr - 1)];
+#pragma unroll
+    for (int r = 0; r < RB; ++r) {
+        o[r] = sub ? o[r] - a[r] : o[r] + a[r];
+        asm volatile("" : "+v"(o[r]));
+    }
+#pragma unroll
+    for (int r = 0; r < RB; ++r)
+        if (r < nr) row[r] = o[r];
 }
 
 // ---------------------------------------------------------------------------
@@ -140,18 +165,19 @@ __device__ __attribute__((always_inline)) inline T wave_reduce_scatter64(T (&a)[
 // [c0, c1) of a wide front): task (step, fused). At c0 = 0 pull the children's update vectors;
 // y = Linv t over the step's columns (entry (j, r) per thread, Linv rows read
 // coalesced, t in LDS); a fused front (at most FUSE_ROWS rows below) also forms its update
-// vector u_i = L(i, front) y, one row per thread. LDS: 2 NB 8 entries.
-template <typename T>
+// vector u_i = L(i, front) y, one row per thread. LDS: 2 NB RB entries.
+template <typename T, int RB>
 __device__ __attribute__((always_inline)) inline void fwd_diag_body(const DevSym& S,
                                                                     const SolveStep* __restrict__ steps, const Task tk,
                                                                     const T* __restrict__ factor,
                                                                     const T* __restrict__ DB, T* __restrict__ Y,
                                                                     T* __restrict__ U, int nrhs) {
-    T* tb = reinterpret_cast<T*>(sweep_lds);  // NB x 8: t
-    T* yx = tb + NB * 8;                       // NB x 8: y
+    T* tb = reinterpret_cast<T*>(sweep_lds);  // NB x RB: t
+    T* yx = tb + NB * RB;                      // NB x RB: y
     const int tid = threadIdx.x, nt = blockDim.x;
     const SolveStep st = steps[tk.s];
     const int s = st.s, c0 = st.c0, nw = st.c1 - c0;
+    const int rb = RB * blockIdx.y, nr = min(RB, nrhs - rb);
     const int f = S.fnrows[s], w = S.fncols[s], m = f - w;
     const int cg = S.super_ptr[s];
     const T* P = factor + S.panel_off[s];
@@ -164,8 +190,8 @@ __device__ __attribute__((always_inline)) inline void fwd_diag_body(const DevSym
     if (c0 == 0) {
         const int32_t* pp = S.pm_ptr + S.pm_row[s];
         const int rows = us ? f : w;
-        for (int q = tid; q < rows * nrhs; q += nt) {
-            const int i = q / nrhs, r = q - i * nrhs;
+        for (int q = tid; q < rows * nr; q += nt) {
+            const int i = q / nr, r = rb + q - i * nr;
             const int e0 = pp[i], e1 = pp[i + 1];
             if (i < w) {
                 if (e0 == e1) continue;
@@ -183,42 +209,38 @@ __device__ __attribute__((always_inline)) inline void fwd_diag_body(const DevSym
     __syncthreads();
     T* y = Y + (int64_t)(cg + c0) * nrhs;
     const T* Li = DB + (int64_t)(cg + c0) * NB;
-    for (int rb = 0; rb < nrhs; rb += 8) {
-        const int nr = min(8, nrhs - rb);
-        for (int q = tid; q < nw * 8; q += nt) tb[q] = (q & 7) < nr ? y[(q >> 3) * nrhs + rb + (q & 7)] : T(0);
-        __syncthreads();
-        for (int q = tid; q < nw * 8; q += nt) {
-            const int j = q >> 3, r = q & 7;
-            T acc = T(0);
+    for (int q = tid; q < nw * RB; q += nt) tb[q] = q % RB < nr ? y[(q / RB) * nrhs + rb + q % RB] : T(0);
+    __syncthreads();
+    for (int q = tid; q < nw * RB; q += nt) {
+        const int j = q / RB, r = q % RB;
+        T acc = T(0);
 #pragma unroll 8
-            for (int i = 0; i <= j; ++i) acc += Li[(int64_t)i * NB + j] * tb[i * 8 + r];
-            yx[q] = acc;
-            if (r < nr) y[j * nrhs + rb + r] = acc;
-        }
-        __syncthreads();
-        if (us)
-            for (int i = w + tid; i < f; i += nt) {
-                T a[8];
-#pragma unroll
-                for (int r = 0; r < 8; ++r) a[r] = T(0);
-#pragma unroll 8
-                for (int j = 0; j < nw; ++j) {
-                    const T lv = P[(int64_t)j * f + i];
-#pragma unroll
-                    for (int r = 0; r < 8; ++r) a[r] += lv * yx[j * 8 + r];
-                }
-                rmw8<T>(us + (i - w) * nrhs + rb, a, nr, false);
-            }
-        __syncthreads();
+        for (int i = 0; i <= j; ++i) acc += Li[(int64_t)i * NB + j] * tb[i * RB + r];
+        yx[q] = acc;
+        if (r < nr) y[j * nrhs + rb + r] = acc;
     }
+    __syncthreads();
+    if (us)
+        for (int i = w + tid; i < f; i += nt) {
+            T a[RB];
+#pragma unroll
+            for (int r = 0; r < RB; ++r) a[r] = T(0);
+#pragma unroll 8
+            for (int j = 0; j < nw; ++j) {
+                const T lv = P[(int64_t)j * f + i];
+#pragma unroll
+                for (int r = 0; r < RB; ++r) a[r] += lv * yx[j * RB + r];
+            }
+            rmw_row<RB>(us + (i - w) * nrhs + rb, a, nr, false);
+        }
 }
 
-template <typename T>
+template <typename T, int RB>
 __global__ void __launch_bounds__(256) k_fwd_diag(DevSym S, const SolveStep* __restrict__ steps,
                                                  const Task* __restrict__ tasks, const T* __restrict__ factor,
                                                  const T* __restrict__ DB, T* __restrict__ Y, T* __restrict__ U,
                                                  int nrhs) {
-    fwd_diag_body<T>(S, steps, tasks[blockIdx.x], factor, DB, Y, U, nrhs);
+    fwd_diag_body<T, RB>(S, steps, tasks[blockIdx.x], factor, DB, Y, U, nrhs);
 }
 
 // rows [r0, r1) below a front step (64 per workgroup of 8 waves, within L11 or within the update
@@ -228,15 +250,15 @@ __global__ void __launch_bounds__(256) k_fwd_diag(DevSym S, const SolveStep* __r
 // LDS; the eight partial sums are added in wave order. task: (step, r0, copy, wide): a wide
 // step's y_step is read from Z, where k_fwd_inv left it, and the task with copy = 1 also copies it
 // to Y (no task of the launch reads those rows of Y).
-// LDS: SOLVE_STEP 8 + 8 64 8 entries.
-template <typename T>
+// LDS: SOLVE_STEP RB + 8 64 RB entries.
+template <typename T, int RB>
 __global__ void __launch_bounds__(512) k_fwd_rows(DevSym S, const SolveStep* __restrict__ steps,
                                                  const Task* __restrict__ tasks, const T* __restrict__ factor,
                                                  T* __restrict__ Y, const T* __restrict__ Z, T* __restrict__ U,
                                                  int nrhs) {
     constexpr int NWV = 8;
-    T* ys = reinterpret_cast<T*>(sweep_lds);  // step columns x 8
-    T* red = ys + SOLVE_STEP * 8;              // NWV waves x 64 rows x 8
+    T* ys = reinterpret_cast<T*>(sweep_lds);  // step columns x RB
+    T* red = ys + SOLVE_STEP * RB;             // NWV waves x 64 rows x RB
     const Task tk = tasks[blockIdx.x];
     const SolveStep st = steps[tk.s];
     const int s = st.s, c0 = st.c0, c1 = st.c1;
@@ -244,6 +266,7 @@ __global__ void __launch_bounds__(512) k_fwd_rows(DevSym S, const SolveStep* __r
     const int cg = S.super_ptr[s];
     const int r0 = tk.a, r1 = min(r0 + 64, r0 < w ? w : f);
     const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6, nt = NWV * 64;
+    const int rb = RB * blockIdx.y, nr = min(RB, nrhs - rb);
     const T* P = factor + S.panel_off[s];
     const bool below = r0 >= w;
     T* us = below ? U + S.uv_off[s] * nrhs : nullptr;
@@ -251,8 +274,8 @@ __global__ void __launch_bounds__(512) k_fwd_rows(DevSym S, const SolveStep* __r
         // the rows' entries of the children's update vectors, row by row from the pull map
         // (child_list order; update vector rows start from zero)
         const int32_t* pp = S.pm_ptr + S.pm_row[s];
-        for (int q = tid; q < (r1 - r0) * nrhs; q += nt) {
-            const int di = q / nrhs, i = r0 + di, r = q - di * nrhs;
+        for (int q = tid; q < (r1 - r0) * nr; q += nt) {
+            const int di = q / nr, i = r0 + di, r = rb + q - di * nr;
             const int e0 = pp[i], e1 = pp[i + 1];
             if (below) {
                 T v = T(0);
@@ -272,44 +295,43 @@ __global__ void __launch_bounds__(512) k_fwd_rows(DevSym S, const SolveStep* __r
     const T* pi = P + i;
     const T* ysrc = tk.c ? Z : Y;
     if (tk.b)
-        for (int q = tid; q < nw * nrhs; q += nt) Y[(int64_t)(cg + c0) * nrhs + q] = Z[(int64_t)(cg + c0) * nrhs + q];
-    for (int rb = 0; rb < nrhs; rb += 8) {
-        const int nr = min(8, nrhs - rb);
-        for (int q = tid; q < nw * 8; q += nt) {
-            const int j = q >> 3, r = q & 7;
-            ys[q] = r < nr ? ysrc[(int64_t)(cg + c0 + j) * nrhs + rb + r] : T(0);
+        for (int q = tid; q < nw * nr; q += nt) {
+            const int64_t o = (int64_t)(cg + c0 + q / nr) * nrhs + rb + q % nr;
+            Y[o] = Z[o];
         }
-        __syncthreads();
-        T acc[8];
+    for (int q = tid; q < nw * RB; q += nt) {
+        const int j = q / RB, r = q % RB;
+        ys[q] = r < nr ? ysrc[(int64_t)(cg + c0 + j) * nrhs + rb + r] : T(0);
+    }
+    __syncthreads();
+    T acc[RB];
 #pragma unroll
-        for (int r = 0; r < 8; ++r) acc[r] = T(0);
-        for (int jb = 16 * wv; jb < nw; jb += 16 * NWV) {
-            T l[16];
+    for (int r = 0; r < RB; ++r) acc[r] = T(0);
+    for (int jb = 16 * wv; jb < nw; jb += 16 * NWV) {
+        T l[16];
 #pragma unroll
-            for (int jj = 0; jj < 16; ++jj)  // the factor streams through once per sweep
-                l[jj] = __builtin_nontemporal_load(pi + (int64_t)(c0 + min(jb + jj, nw - 1)) * f);
+        for (int jj = 0; jj < 16; ++jj)  // the factor streams through once per sweep
+            l[jj] = __builtin_nontemporal_load(pi + (int64_t)(c0 + min(jb + jj, nw - 1)) * f);
 #pragma unroll
-            for (int jj = 0; jj < 16; ++jj) {
-                const T lv = jb + jj < nw ? l[jj] : T(0);
-                const T* yj = ys + min(jb + jj, nw - 1) * 8;
+        for (int jj = 0; jj < 16; ++jj) {
+            const T lv = jb + jj < nw ? l[jj] : T(0);
+            const T* yj = ys + min(jb + jj, nw - 1) * RB;
 #pragma unroll
-                for (int r = 0; r < 8; ++r) acc[r] += lv * yj[r];
-            }
+            for (int r = 0; r < RB; ++r) acc[r] += lv * yj[r];
         }
+    }
 #pragma unroll
-        for (int r = 0; r < 8; ++r) red[(wv * 64 + lane) * 8 + r] = acc[r];
-        __syncthreads();
-        if (wv == 0 && r0 + lane < r1) {
-            T v[8];
+    for (int r = 0; r < RB; ++r) red[(wv * 64 + lane) * RB + r] = acc[r];
+    __syncthreads();
+    if (wv == 0 && r0 + lane < r1) {
+        T v[RB];
 #pragma unroll
-            for (int r = 0; r < 8; ++r) {
-                v[r] = red[lane * 8 + r];
+        for (int r = 0; r < RB; ++r) {
+            v[r] = red[lane * RB + r];
 #pragma unroll
-                for (int u = 1; u < NWV; ++u) v[r] += red[(u * 64 + lane) * 8 + r];
-            }
-            rmw8<T>(below ? us + (int64_t)(i - w) * nrhs + rb : Y + (int64_t)(cg + i) * nrhs + rb, v, nr, !below);
+            for (int u = 1; u < NWV; ++u) v[r] += red[(u * 64 + lane) * RB + r];
         }
-        __syncthreads();
+        rmw_row<RB>(below ? us + (int64_t)(i - w) * nrhs + rb : Y + (int64_t)(cg + i) * nrhs + rb, v, nr, !below);
     }
 }
 
@@ -317,10 +339,10 @@ __global__ void __launch_bounds__(512) k_fwd_rows(DevSym S, const SolveStep* __r
 // backward
 
 // partial sums of L(rows below the step, step)^T x over the chunk of L21T_CHUNK rows of a task
-// (step, col0, chunk): one wave for the 8 columns from col0; lanes along the rows; 8
-// right-hand sides per pass. The 64 sums are reduce-scattered across the lanes (lane l: column
-// l / 8, right-hand side l % 8). part[(poff + chunk nw + j - c0) nrhs + r], nw = c1 - c0.
-template <typename T>
+// (step, col0, chunk): one wave for the 8 columns from col0; lanes along the rows; RB
+// right-hand sides. The 8 RB sums are reduce-scattered across the lanes.
+// part[(poff + chunk nw + j - c0) nrhs + r], nw = c1 - c0.
+template <typename T, int RB>
 __global__ void __launch_bounds__(64) k_bwd_l21t(DevSym S, const SolveStep* __restrict__ steps,
                                                 const Task* __restrict__ tasks, const T* __restrict__ factor,
                                                 const T* __restrict__ Y, T* __restrict__ part, int nrhs) {
@@ -334,45 +356,45 @@ __global__ void __launch_bounds__(64) k_bwd_l21t(DevSym S, const SolveStep* __re
     const int32_t* rows = S.rowval + S.rowptr[s];
     const int r0 = c1 + chunk * L21T_CHUNK, r1 = min(f, r0 + L21T_CHUNK);
     T* out = part + (st.poff + (int64_t)chunk * (c1 - c0)) * nrhs;
-    for (int rb = 0; rb < nrhs; rb += 8) {
-        T a[64];
+    const int rb = RB * blockIdx.y;
+    T a[8 * RB];
 #pragma unroll
-        for (int v = 0; v < 64; ++v) a[v] = T(0);
+    for (int v = 0; v < 8 * RB; ++v) a[v] = T(0);
 #pragma unroll 2
-        for (int i = r0 + lane; i < r1; i += 64) {
-            const T* yr = Y + (int64_t)rows[i] * nrhs;
-            T x[8];
+    for (int i = r0 + lane; i < r1; i += 64) {
+        const T* yr = Y + (int64_t)rows[i] * nrhs;
+        T x[RB];
 #pragma unroll
-            for (int r = 0; r < 8; ++r) x[r] = yr[min(rb + r, nrhs - 1)];
-            const T* pc = P + (int64_t)col0 * f + i;  // column col0 + c; columns past c1 read c1 - 1
-            T l[8];  // the row's eight loads issued together (the FP32 build otherwise waits per load)
+        for (int r = 0; r < RB; ++r) x[r] = yr[min(rb + r, nrhs - 1)];
+        const T* pc = P + (int64_t)col0 * f + i;  // column col0 + c; columns past c1 read c1 - 1
+        T l[8];  // the row's eight loads issued together (the FP32 build otherwise waits per load)
 #pragma unroll
-            for (int c = 0; c < 8; ++c) {
-                l[c] = __builtin_nontemporal_load(pc);  // the factor streams through once per sweep
-                pc += col0 + c + 1 < c1 ? f : 0;
-            }
-            __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-            for (int c = 0; c < 8; ++c)
-#pragma unroll
-                for (int r = 0; r < 8; ++r) a[c * 8 + r] += l[c] * x[r];
+        for (int c = 0; c < 8; ++c) {
+            l[c] = __builtin_nontemporal_load(pc);  // the factor streams through once per sweep
+            pc += col0 + c + 1 < c1 ? f : 0;
         }
-        const T v = wave_reduce_scatter64<T>(a);
-        const int c = lane >> 3, r = lane & 7;
-        if (col0 + c < c1 && rb + r < nrhs) out[(int64_t)(col0 + c - c0) * nrhs + rb + r] = v;
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int c = 0; c < 8; ++c)
+#pragma unroll
+            for (int r = 0; r < RB; ++r) a[c * RB + r] += l[c] * x[r];
     }
+    const T v = wave_reduce_scatter(a);
+    constexpr int LPV = 8 / RB;  // lanes with the same sum
+    const int q = lane / LPV, c = q / RB, r = q % RB;
+    if (lane % LPV == 0 && col0 + c < c1 && rb + r < nrhs) out[(int64_t)(col0 + c - c0) * nrhs + rb + r] = v;
 }
 
 // one workgroup per narrow step (a whole narrow front, or the last columns [c0, c1) of a wide
 // front): task (step, 0). t = y - the L21^T x partial sums (chunk order), x = Linv^T t over the
-// step's columns (entry (j, r) per thread). LDS: NB 8 entries.
-template <typename T>
+// step's columns (entry (j, r) per thread). LDS: NB RB entries.
+template <typename T, int RB>
 __device__ __attribute__((always_inline)) inline void bwd_diag_body(const DevSym& S,
                                                                     const SolveStep* __restrict__ steps, const Task tk,
                                                                     const T* __restrict__ factor,
                                                                     const T* __restrict__ DB, T* __restrict__ Y,
                                                                     const T* __restrict__ part, int nrhs) {
-    T* tb = reinterpret_cast<T*>(sweep_lds);  // NB x 8
+    T* tb = reinterpret_cast<T*>(sweep_lds);  // NB x RB
     const int tid = threadIdx.x, nt = blockDim.x;
     const SolveStep st = steps[tk.s];
     const int s = st.s, c0 = st.c0, nw = st.c1 - c0;
@@ -380,35 +402,32 @@ __device__ __attribute__((always_inline)) inline void bwd_diag_body(const DevSym
     T* y = Y + (int64_t)(cg + c0) * nrhs;
     const T* pp = part + st.poff * nrhs;
     const T* Li = DB + (int64_t)(cg + c0) * NB;
-    for (int rb = 0; rb < nrhs; rb += 8) {
-        const int nr = min(8, nrhs - rb);
-        for (int q = tid; q < nw * 8; q += nt) {
-            const int j = q >> 3, r = q & 7;
-            T v = T(0);
-            if (r < nr) {
-                v = y[j * nrhs + rb + r];
-                for (int ch = 0; ch < st.nch; ++ch) v -= pp[((int64_t)ch * nw + j) * nrhs + rb + r];
-            }
-            tb[q] = v;
+    const int rb = RB * blockIdx.y, nr = min(RB, nrhs - rb);
+    for (int q = tid; q < nw * RB; q += nt) {
+        const int j = q / RB, r = q % RB;
+        T v = T(0);
+        if (r < nr) {
+            v = y[j * nrhs + rb + r];
+            for (int ch = 0; ch < st.nch; ++ch) v -= pp[((int64_t)ch * nw + j) * nrhs + rb + r];
         }
-        __syncthreads();
-        for (int q = tid; q < nw * 8; q += nt) {
-            const int j = q >> 3, r = q & 7;
-            T acc = T(0);
+        tb[q] = v;
+    }
+    __syncthreads();
+    for (int q = tid; q < nw * RB; q += nt) {
+        const int j = q / RB, r = q % RB;
+        T acc = T(0);
 #pragma unroll 8
-            for (int i = j; i < nw; ++i) acc += Li[(int64_t)j * NB + i] * tb[i * 8 + r];
-            if (r < nr) y[j * nrhs + rb + r] = acc;
-        }
-        __syncthreads();
+        for (int i = j; i < nw; ++i) acc += Li[(int64_t)j * NB + i] * tb[i * RB + r];
+        if (r < nr) y[j * nrhs + rb + r] = acc;
     }
 }
 
-template <typename T>
+template <typename T, int RB>
 __global__ void __launch_bounds__(256) k_bwd_diag(DevSym S, const SolveStep* __restrict__ steps,
                                                  const Task* __restrict__ tasks, const T* __restrict__ factor,
                                                  const T* __restrict__ DB, T* __restrict__ Y,
                                                  const T* __restrict__ part, int nrhs) {
-    bwd_diag_body<T>(S, steps, tasks[blockIdx.x], factor, DB, Y, part, nrhs);
+    bwd_diag_body<T, RB>(S, steps, tasks[blockIdx.x], factor, DB, Y, part, nrhs);
 }
 
 // ---------------------------------------------------------------------------
@@ -547,14 +566,14 @@ __global__ void __launch_bounds__(256) k_step_inverse(DevSym S, const SolveStep*
 // partial sums of a row are added in group order. t = the step's rows of y, less the children's
 // update entries at the first step of a front (applied here to an LDS copy). The result goes
 // to Z (the other workgroups still read y); k_copy_rows moves it to y. task: (step, ri0).
-// LDS: SOLVE_STEP 8 + 16 16 8 entries.
-template <typename T>
+// LDS: SOLVE_STEP RB + 16 16 RB entries.
+template <typename T, int RB>
 __device__ __attribute__((always_inline)) inline void fwd_inv_body(const DevSym& S, const SolveStep* __restrict__ steps,
                                                                    const Task tk, const T* __restrict__ XB,
                                                                    const T* __restrict__ Y, T* __restrict__ Z,
                                                                    const T* __restrict__ U, int nrhs) {
-    T* t = reinterpret_cast<T*>(sweep_lds);  // step rows x 8
-    T* red = t + SOLVE_STEP * 8;              // 16 groups x 16 rows x 8
+    T* t = reinterpret_cast<T*>(sweep_lds);  // step rows x RB
+    T* red = t + SOLVE_STEP * RB;             // 16 groups x 16 rows x RB
     const SolveStep st = steps[tk.s];
     const int s = st.s, c0 = st.c0, c1 = st.c1, nw = c1 - c0;
     const int cg = S.super_ptr[s];
@@ -562,75 +581,72 @@ __device__ __attribute__((always_inline)) inline void fwd_inv_body(const DevSym&
     const int ri0 = tk.a, nbi = min(16, nw - ri0), ncols = ri0 + nbi;
     const int tid = threadIdx.x, rl = tid & 15, g = tid >> 4;
     const int r = ri0 + min(rl, nbi - 1);
-    for (int rb = 0; rb < nrhs; rb += 8) {
-        const int nr = min(8, nrhs - rb);
-        // t = the step's rows of y, less (at the front's first step) the children's update entries
-        // of those rows, row by row from the pull map in child_list order
-        const int32_t* pp = S.pm_ptr + S.pm_row[s];
-        for (int q = tid; q < ncols * 8; q += 256) {
-            const int i = q >> 3, rr = q & 7;
-            T v = T(0);
-            if (rr < nr) {
-                v = Y[(int64_t)(cg + c0 + i) * nrhs + rb + rr];
-                if (c0 == 0) {
-                    const int e1 = pp[i + 1];
-                    for (int e = pp[i]; e < e1; ++e) v -= U[(int64_t)S.pm_src[e] * nrhs + rb + rr];
-                }
-            }
-            t[q] = v;
-        }
-        __syncthreads();
-        T acc[8];
-#pragma unroll
-        for (int rr = 0; rr < 8; ++rr) acc[rr] = T(0);
-        const T* xr = X + r;
-        for (int cb = 16 * g; cb < ncols; cb += 256) {
-            T l[16];
-#pragma unroll
-            for (int jj = 0; jj < 16; ++jj) l[jj] = xr[(int64_t)min(cb + jj, ncols - 1) * nw];
-#pragma unroll
-            for (int jj = 0; jj < 16; ++jj) {
-                const T lv = cb + jj < ncols ? l[jj] : T(0);
-                const T* tj = t + min(cb + jj, ncols - 1) * 8;
-#pragma unroll
-                for (int rr = 0; rr < 8; ++rr) acc[rr] += lv * tj[rr];
+    const int rb = RB * blockIdx.y, nr = min(RB, nrhs - rb);
+    // t = the step's rows of y, less (at the front's first step) the children's update entries
+    // of those rows, row by row from the pull map in child_list order
+    const int32_t* pp = S.pm_ptr + S.pm_row[s];
+    for (int q = tid; q < ncols * RB; q += 256) {
+        const int i = q / RB, rr = q % RB;
+        T v = T(0);
+        if (rr < nr) {
+            v = Y[(int64_t)(cg + c0 + i) * nrhs + rb + rr];
+            if (c0 == 0) {
+                const int e1 = pp[i + 1];
+                for (int e = pp[i]; e < e1; ++e) v -= U[(int64_t)S.pm_src[e] * nrhs + rb + rr];
             }
         }
+        t[q] = v;
+    }
+    __syncthreads();
+    T acc[RB];
 #pragma unroll
-        for (int rr = 0; rr < 8; ++rr) red[(g * 16 + rl) * 8 + rr] = acc[rr];
-        __syncthreads();
-        if (tid < 16 * 8) {
-            const int row = tid >> 3, rr = tid & 7;
-            if (row < nbi && rr < nr) {
-                T v = red[row * 8 + rr];
+    for (int rr = 0; rr < RB; ++rr) acc[rr] = T(0);
+    const T* xr = X + r;
+    for (int cb = 16 * g; cb < ncols; cb += 256) {
+        T l[16];
 #pragma unroll
-                for (int u = 1; u < 16; ++u) v += red[(u * 16 + row) * 8 + rr];
-                Z[(int64_t)(cg + c0 + ri0 + row) * nrhs + rb + rr] = v;
-            }
+        for (int jj = 0; jj < 16; ++jj) l[jj] = xr[(int64_t)min(cb + jj, ncols - 1) * nw];
+#pragma unroll
+        for (int jj = 0; jj < 16; ++jj) {
+            const T lv = cb + jj < ncols ? l[jj] : T(0);
+            const T* tj = t + min(cb + jj, ncols - 1) * RB;
+#pragma unroll
+            for (int rr = 0; rr < RB; ++rr) acc[rr] += lv * tj[rr];
         }
-        __syncthreads();
+    }
+#pragma unroll
+    for (int rr = 0; rr < RB; ++rr) red[(g * 16 + rl) * RB + rr] = acc[rr];
+    __syncthreads();
+    if (tid < 16 * RB) {
+        const int row = tid / RB, rr = tid % RB;
+        if (row < nbi && rr < nr) {
+            T v = red[row * RB + rr];
+#pragma unroll
+            for (int u = 1; u < 16; ++u) v += red[(u * 16 + row) * RB + rr];
+            Z[(int64_t)(cg + c0 + ri0 + row) * nrhs + rb + rr] = v;
+        }
     }
 }
 
-template <typename T>
+template <typename T, int RB>
 __global__ void __launch_bounds__(256) k_fwd_inv(DevSym S, const SolveStep* __restrict__ steps,
                                                 const Task* __restrict__ tasks, const T* __restrict__ XB,
                                                 const T* __restrict__ Y, T* __restrict__ Z, const T* __restrict__ U,
                                                 int nrhs) {
-    fwd_inv_body<T>(S, steps, tasks[blockIdx.x], XB, Y, Z, U, nrhs);
+    fwd_inv_body<T, RB>(S, steps, tasks[blockIdx.x], XB, Y, Z, U, nrhs);
 }
 
 // backward, wide steps: x_j = sum_{i >= j} X_ij t_i for 8 columns [col0, col0 + 8) of a step,
 // one wave per (step, col0); t = the step's rows of y (k_sub_partials has subtracted the
-// L21^T x partial sums), rows >= col0 staged in LDS. Lanes along the rows of X (coalesced); the 64 sums are
+// L21^T x partial sums), rows >= col0 staged in LDS. Lanes along the rows of X (coalesced); the 8 RB sums are
 // reduce-scattered across the lanes. t (y_step less the partial sums) comes from Z, where
 // k_sub_partials formed it, and x goes to y directly (no task of the launch reads those rows of y).
-// task: (step, col0). LDS: SOLVE_STEP 8 entries.
-template <typename T>
+// task: (step, col0). LDS: SOLVE_STEP RB entries.
+template <typename T, int RB>
 __global__ void __launch_bounds__(64) k_bwd_inv(DevSym S, const SolveStep* __restrict__ steps,
                                                const Task* __restrict__ tasks, const T* __restrict__ XB,
                                                T* __restrict__ Y, const T* __restrict__ Z, int nrhs) {
-    T* t = reinterpret_cast<T*>(sweep_lds);  // rows [col0, nw) of the step x 8
+    T* t = reinterpret_cast<T*>(sweep_lds);  // rows [col0, nw) of the step x RB
     const Task tk = tasks[blockIdx.x];
     const SolveStep st = steps[tk.s];
     const int s = st.s, c0 = st.c0, c1 = st.c1, nw = c1 - c0;
@@ -638,40 +654,38 @@ __global__ void __launch_bounds__(64) k_bwd_inv(DevSym S, const SolveStep* __res
     const T* X = XB + st.xoff;
     const int col0 = tk.a, cend = min(nw, col0 + 8);
     const int lane = threadIdx.x;
-    for (int rb = 0; rb < nrhs; rb += 8) {
-        const int nr = min(8, nrhs - rb);
-        for (int q = lane; q < (nw - col0) * 8; q += 64) {
-            const int i = col0 + (q >> 3), rr = q & 7;
-            t[q] = rr < nr ? Z[(int64_t)(cg + c0 + i) * nrhs + rb + rr] : T(0);
-        }
-        __syncthreads();
-        T a[64];
-#pragma unroll
-        for (int v = 0; v < 64; ++v) a[v] = T(0);
-#pragma unroll 2
-        for (int i = col0 + lane; i < nw; i += 64) {
-            const T* ti = t + (i - col0) * 8;
-            T x[8];
-#pragma unroll
-            for (int rr = 0; rr < 8; ++rr) x[rr] = ti[rr];
-            const T* pc = X + (int64_t)col0 * nw + i;  // column col0 + c; columns past cend read cend - 1
-            T l[8];  // the row's eight loads issued together (the FP32 build otherwise waits per load)
-#pragma unroll
-            for (int c = 0; c < 8; ++c) {
-                l[c] = *pc;
-                pc += col0 + c + 1 < cend ? nw : 0;
-            }
-            __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-            for (int c = 0; c < 8; ++c)
-#pragma unroll
-                for (int rr = 0; rr < 8; ++rr) a[c * 8 + rr] += l[c] * x[rr];
-        }
-        const T v = wave_reduce_scatter64<T>(a);
-        const int col = col0 + (lane >> 3), rr = lane & 7;
-        if (col < cend && rr < nr) Y[(int64_t)(cg + c0 + col) * nrhs + rb + rr] = v;
-        __syncthreads();
+    const int rb = RB * blockIdx.y, nr = min(RB, nrhs - rb);
+    for (int q = lane; q < (nw - col0) * RB; q += 64) {
+        const int i = col0 + q / RB, rr = q % RB;
+        t[q] = rr < nr ? Z[(int64_t)(cg + c0 + i) * nrhs + rb + rr] : T(0);
     }
+    __syncthreads();
+    T a[8 * RB];
+#pragma unroll
+    for (int v = 0; v < 8 * RB; ++v) a[v] = T(0);
+#pragma unroll 2
+    for (int i = col0 + lane; i < nw; i += 64) {
+        const T* ti = t + (i - col0) * RB;
+        T x[RB];
+#pragma unroll
+        for (int rr = 0; rr < RB; ++rr) x[rr] = ti[rr];
+        const T* pc = X + (int64_t)col0 * nw + i;  // column col0 + c; columns past cend read cend - 1
+        T l[8];  // the row's eight loads issued together (the FP32 build otherwise waits per load)
+#pragma unroll
+        for (int c = 0; c < 8; ++c) {
+            l[c] = *pc;
+            pc += col0 + c + 1 < cend ? nw : 0;
+        }
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int c = 0; c < 8; ++c)
+#pragma unroll
+            for (int rr = 0; rr < RB; ++rr) a[c * RB + rr] += l[c] * x[rr];
+    }
+    const T v = wave_reduce_scatter(a);
+    constexpr int LPV = 8 / RB;  // lanes with the same sum
+    const int q = lane / LPV, col = col0 + q / RB, rr = q % RB;
+    if (lane % LPV == 0 && col < cend && rr < nr) Y[(int64_t)(cg + c0 + col) * nrhs + rb + rr] = v;
 }
 
 // rows [r0, r0 + nr) of a wide step: Z = y less the L21^T x partial sums of those rows, in chunk
@@ -718,31 +732,44 @@ __global__ void __launch_bounds__(256) k_copy_rows(DevSym S, const SolveStep* __
 // forward, the narrow steps (the first ndiag workgroups, tasks of k_fwd_diag) and the wide steps'
 // inverse products (tasks of k_fwd_inv); backward, the narrow steps (k_bwd_diag) and the wide
 // steps' t = y less the partial sums (k_sub_partials). Each workgroup runs its kernel's body.
-template <typename T>
+template <typename T, int RB>
 __global__ void __launch_bounds__(256) k_fwd_group(DevSym S, const SolveStep* __restrict__ steps,
                                                   const Task* __restrict__ tdiag, int ndiag,
                                                   const Task* __restrict__ tinv, const T* __restrict__ factor,
                                                   const T* __restrict__ DB, const T* __restrict__ XB,
                                                   T* __restrict__ Y, T* __restrict__ Z, T* __restrict__ U, int nrhs) {
     if ((int)blockIdx.x < ndiag)
-        fwd_diag_body<T>(S, steps, tdiag[blockIdx.x], factor, DB, Y, U, nrhs);
+        fwd_diag_body<T, RB>(S, steps, tdiag[blockIdx.x], factor, DB, Y, U, nrhs);
     else
-        fwd_inv_body<T>(S, steps, tinv[blockIdx.x - ndiag], XB, Y, Z, U, nrhs);
+        fwd_inv_body<T, RB>(S, steps, tinv[blockIdx.x - ndiag], XB, Y, Z, U, nrhs);
 }
 
-template <typename T>
+template <typename T, int RB>
 __global__ void __launch_bounds__(256) k_bwd_group(DevSym S, const SolveStep* __restrict__ steps,
                                                   const Task* __restrict__ tdiag, int ndiag,
                                                   const Task* __restrict__ tsub, const T* __restrict__ factor,
                                                   const T* __restrict__ DB, T* __restrict__ Y, T* __restrict__ Z,
                                                   const T* __restrict__ part, int nrhs) {
     if ((int)blockIdx.x < ndiag)
-        bwd_diag_body<T>(S, steps, tdiag[blockIdx.x], factor, DB, Y, part, nrhs);
-    else
+        bwd_diag_body<T, RB>(S, steps, tdiag[blockIdx.x], factor, DB, Y, part, nrhs);
+    else if (blockIdx.y == 0)  // all the right-hand sides
         sub_partials_body<T>(S, steps, tsub[blockIdx.x - ndiag], Y, Z, part, nrhs);
 }
 
 // ---------------------------------------------------------------------------
+
+// right-hand sides per workgroup: all up to four (three as four), else eight
+template <typename F>
+inline void launch_rb(int nrhs, F launch) {
+    if (nrhs == 1)
+        launch(std::integral_constant<int, 1>{}, 1);
+    else if (nrhs == 2)
+        launch(std::integral_constant<int, 2>{}, 1);
+    else if (nrhs <= 4)
+        launch(std::integral_constant<int, 4>{}, 1);
+    else
+        launch(std::integral_constant<int, 8>{}, (nrhs + 7) / 8);
+}
 
 template <typename T>
 void launch_block_inverse(hipStream_t st, const DevSym& S, const Task* tasks, int n, T* factor, T* DB, int bs) {
@@ -757,46 +784,68 @@ void launch_block_inverse(hipStream_t st, const DevSym& S, const Task* tasks, in
 template <typename T>
 void launch_fwd_diag(hipStream_t st, const DevSym& S, const SolveStep* steps, const Task* tasks, int n, int threads,
                      const T* factor, const T* DB, T* Y, T* U, int nrhs) {
-    const size_t lds = 2 * NB * 8 * sizeof(T);
-    hipLaunchKernelGGL(k_fwd_diag<T>, dim3(n), dim3(threads), lds, st, S, steps, tasks, factor, DB, Y, U, nrhs);
+    launch_rb(nrhs, [&](auto rb, int ny) {
+        constexpr int RB = decltype(rb)::value;
+        const size_t lds = 2 * NB * RB * sizeof(T);
+        hipLaunchKernelGGL((k_fwd_diag<T, RB>), dim3(n, ny), dim3(threads), lds, st, S, steps, tasks, factor, DB,
+                           Y, U, nrhs);
+    });
 }
 
 template <typename T>
 void launch_fwd_group(hipStream_t st, const DevSym& S, const SolveStep* steps, const Task* tdiag, int ndiag,
                       const Task* tinv, int ninv, const T* factor, const T* DB, const T* XB, T* Y, T* Z, T* U,
                       int nrhs) {
-    const size_t lds = std::max(2 * NB * 8, SOLVE_STEP * 8 + 16 * 16 * 8) * sizeof(T);
-    hipLaunchKernelGGL(k_fwd_group<T>, dim3(ndiag + ninv), dim3(256), lds, st, S, steps, tdiag, ndiag, tinv, factor,
-                       DB, XB, Y, Z, U, nrhs);
+    launch_rb(nrhs, [&](auto rb, int ny) {
+        constexpr int RB = decltype(rb)::value;
+        const size_t lds = std::max(2 * NB * RB, SOLVE_STEP * RB + 16 * 16 * RB) * sizeof(T);
+        hipLaunchKernelGGL((k_fwd_group<T, RB>), dim3(ndiag + ninv, ny), dim3(256), lds, st, S, steps, tdiag,
+                           ndiag, tinv, factor, DB, XB, Y, Z, U, nrhs);
+    });
 }
 
 template <typename T>
 void launch_bwd_group(hipStream_t st, const DevSym& S, const SolveStep* steps, const Task* tdiag, int ndiag,
                       const Task* tsub, int nsub, const T* factor, const T* DB, T* Y, T* Z, const T* part,
                       int nrhs) {
-    const size_t lds = NB * 8 * sizeof(T);
-    hipLaunchKernelGGL(k_bwd_group<T>, dim3(ndiag + nsub), dim3(256), lds, st, S, steps, tdiag, ndiag, tsub, factor,
-                       DB, Y, Z, part, nrhs);
+    launch_rb(nrhs, [&](auto rb, int ny) {
+        constexpr int RB = decltype(rb)::value;
+        const size_t lds = NB * RB * sizeof(T);
+        hipLaunchKernelGGL((k_bwd_group<T, RB>), dim3(ndiag + nsub, ny), dim3(256), lds, st, S, steps, tdiag,
+                           ndiag, tsub, factor, DB, Y, Z, part, nrhs);
+    });
 }
 
 template <typename T>
 void launch_fwd_rows(hipStream_t st, const DevSym& S, const SolveStep* steps, const Task* tasks, int n,
                      const T* factor, T* Y, const T* Z, T* U, int nrhs) {
-    const size_t lds = (SOLVE_STEP * 8 + 8 * 64 * 8) * sizeof(T);
-    hipLaunchKernelGGL(k_fwd_rows<T>, dim3(n), dim3(512), lds, st, S, steps, tasks, factor, Y, Z, U, nrhs);
+    launch_rb(nrhs, [&](auto rb, int ny) {
+        constexpr int RB = decltype(rb)::value;
+        const size_t lds = (SOLVE_STEP * RB + 8 * 64 * RB) * sizeof(T);
+        hipLaunchKernelGGL((k_fwd_rows<T, RB>), dim3(n, ny), dim3(512), lds, st, S, steps, tasks, factor, Y,
+                           Z, U, nrhs);
+    });
 }
 
 template <typename T>
 void launch_bwd_l21t(hipStream_t st, const DevSym& S, const SolveStep* steps, const Task* tasks, int n,
                      const T* factor, const T* Y, T* part, int nrhs) {
-    hipLaunchKernelGGL(k_bwd_l21t<T>, dim3(n), dim3(64), 0, st, S, steps, tasks, factor, Y, part, nrhs);
+    launch_rb(nrhs, [&](auto rb, int ny) {
+        constexpr int RB = decltype(rb)::value;
+        hipLaunchKernelGGL((k_bwd_l21t<T, RB>), dim3(n, ny), dim3(64), 0, st, S, steps, tasks, factor, Y,
+                           part, nrhs);
+    });
 }
 
 template <typename T>
 void launch_bwd_diag(hipStream_t st, const DevSym& S, const SolveStep* steps, const Task* tasks, int n, int threads,
                      const T* factor, const T* DB, T* Y, const T* part, int nrhs) {
-    const size_t lds = NB * 8 * sizeof(T);
-    hipLaunchKernelGGL(k_bwd_diag<T>, dim3(n), dim3(threads), lds, st, S, steps, tasks, factor, DB, Y, part, nrhs);
+    launch_rb(nrhs, [&](auto rb, int ny) {
+        constexpr int RB = decltype(rb)::value;
+        const size_t lds = NB * RB * sizeof(T);
+        hipLaunchKernelGGL((k_bwd_diag<T, RB>), dim3(n, ny), dim3(threads), lds, st, S, steps, tasks, factor, DB,
+                           Y, part, nrhs);
+    });
 }
 
 template <typename T>
@@ -808,15 +857,21 @@ void launch_step_inverse(hipStream_t st, const DevSym& S, const SolveStep* steps
 template <typename T>
 void launch_fwd_inv(hipStream_t st, const DevSym& S, const SolveStep* steps, const Task* tasks, int n, const T* XB,
                     const T* Y, T* Z, const T* U, int nrhs) {
-    const size_t lds = (SOLVE_STEP * 8 + 16 * 16 * 8) * sizeof(T);
-    hipLaunchKernelGGL(k_fwd_inv<T>, dim3(n), dim3(256), lds, st, S, steps, tasks, XB, Y, Z, U, nrhs);
+    launch_rb(nrhs, [&](auto rb, int ny) {
+        constexpr int RB = decltype(rb)::value;
+        const size_t lds = (SOLVE_STEP * RB + 16 * 16 * RB) * sizeof(T);
+        hipLaunchKernelGGL((k_fwd_inv<T, RB>), dim3(n, ny), dim3(256), lds, st, S, steps, tasks, XB, Y, Z, U, nrhs);
+    });
 }
 
 template <typename T>
 void launch_bwd_inv(hipStream_t st, const DevSym& S, const SolveStep* steps, const Task* tasks, int n, const T* XB,
                     T* Y, const T* Z, int nrhs) {
-    const size_t lds = SOLVE_STEP * 8 * sizeof(T);
-    hipLaunchKernelGGL(k_bwd_inv<T>, dim3(n), dim3(64), lds, st, S, steps, tasks, XB, Y, Z, nrhs);
+    launch_rb(nrhs, [&](auto rb, int ny) {
+        constexpr int RB = decltype(rb)::value;
+        const size_t lds = SOLVE_STEP * RB * sizeof(T);
+        hipLaunchKernelGGL((k_bwd_inv<T, RB>), dim3(n, ny), dim3(64), lds, st, S, steps, tasks, XB, Y, Z, nrhs);
+    });
 }
 
 template <typename T>

@@ -640,8 +640,9 @@ int build_schedule(sds_handle* h, int dtype) {
         L.off_tiny = (int64_t)flist.size();
         flist.insert(flist.end(), L.tiny.begin(), L.tiny.end());
         L.off_mid = (int64_t)flist.size();
-        L.nlow_mid = (int)(std::stable_partition(L.mid.begin(), L.mid.end(), [&](int32_t s) { return h->fnrows[s] <= 64; }) -
-                           L.mid.begin());
+        const auto high =
+            std::stable_partition(L.mid.begin(), L.mid.end(), [&](int32_t s) { return h->fnrows[s] <= 64; });
+        L.nlow_mid = (int)(high - L.mid.begin());
         flist.insert(flist.end(), L.mid.begin(), L.mid.end());
     }
     for (auto& L : h->levels) {
