@@ -824,15 +824,18 @@ __global__ void __launch_bounds__(512) k_lu_panel(DevSym S, const Task* __restri
 }
 
 // the U rows of a panel's pivots k0 .. k0 + np - 1 in the 64 columns from J0 (after the panel): u = a -
-// L u in pivot order, eight rows at a time, a thread per column; the unscaled rows go to the front's
-// scratch (U[q f + j], read by k_lu_trail), u / d to Q. task: (s, J0, 0, scratch offset)
+// L u in pivot order, a thread per column with all its np entries in registers, loaded together; the
+// unscaled rows go to the front's scratch (U[q f + j], read by k_lu_trail), u / d to Q. task: (s, J0,
+// 0, scratch offset). Bound: latency, one wave per 64 columns: the chain of 32 pivots after one
+// round of loads (eight rows at a time, each block read the rows before it back from the scratch:
+// 16.8 us a launch of a 32 x 32 x 32 LU in FP64, 10.7 now).
 constexpr int LU_PANEL_MAX = 32;  // most columns of a panel
 
 template <typename T>
 __global__ void __launch_bounds__(64) k_lu_urows(DevSym S, const Task* __restrict__ tasks, int k0, int cols,
                                                  const T* __restrict__ factor, T* __restrict__ ufactor,
                                                  const T* __restrict__ dvec, T* __restrict__ scratch) {
-    __shared__ T Ls[LU_PANEL_MAX][LU_PANEL_MAX + 1];  // Ls[r][q] = L(k0 + r, k0 + q)
+    __shared__ __align__(16) T Lc[LU_PANEL_MAX][LU_PANEL_MAX];  // Lc[q][r] = L(k0 + r, k0 + q)
     const Task t = tasks[blockIdx.x];
     const int s = t.s, f = S.fnrows[s], w = S.fncols[s];
     if (k0 >= w) return;
@@ -844,39 +847,52 @@ __global__ void __launch_bounds__(64) k_lu_urows(DevSym S, const Task* __restric
     T* U = scratch + t.c;
     const bool on = j >= k0 + np && j < f;
     const int jc = min(max(j, k0 + np), f - 1);  // (np < f - k0 in a front with columns after the panel)
-    for (int q = threadIdx.x; q < np * np; q += 64) {
-        const int c = q / np, r = q - c * np;
-        Ls[r][c] = P[(int64_t)(k0 + c) * f + k0 + r];
+    // row r of the column in P (fully summed) or of U12, stored by rows, in Q; blocks of eight rows up to
+    // np: rows past np in the last block repeat row np - 1 and are neither stored nor read by others
+    const T* col = jc < w ? P + (int64_t)jc * f + k0 : Q + (int64_t)k0 * f + jc;
+    const int64_t step = jc < w ? 1 : f;
+    T a[LU_PANEL_MAX];
+#pragma unroll
+    for (int g = 0; g < LU_PANEL_MAX; g += 8)
+        if (g < np) {
+#pragma unroll
+            for (int r = 0; r < 8; ++r) a[g + r] = col[min(g + r, np - 1) * step];
+        }
+    const int lane = threadIdx.x;
+    T lv[LU_PANEL_MAX / 2];
+#pragma unroll
+    for (int u = 0; u < LU_PANEL_MAX / 2; ++u) {
+        const int c = 2 * u + (lane >> 5), r = lane & 31;
+        lv[u] = P[(int64_t)(k0 + min(c, np - 1)) * f + k0 + min(r, np - 1)];
     }
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int u = 0; u < LU_PANEL_MAX / 2; ++u) Lc[2 * u + (lane >> 5)][lane & 31] = lv[u];
     __syncthreads();
-    for (int b0 = 0; b0 < np; b0 += 8) {
-        T a[8];
 #pragma unroll
-        for (int r = 0; r < 8; ++r) {
-            const int i = k0 + min(b0 + r, np - 1);
-            a[r] = jc < w ? P[(int64_t)jc * f + i] : Q[(int64_t)i * f + jc];
-        }
-        for (int q0 = 0; q0 < b0; q0 += 8) {  // (whole blocks of eight: b0 is a multiple of eight)
-            T uv[8];
+    for (int g = 0; g < LU_PANEL_MAX; g += 8)
+        if (g < np) {
 #pragma unroll
-            for (int q = 0; q < 8; ++q) uv[q] = U[(int64_t)(q0 + q) * f + jc];
+            for (int r = g; r < g + 8; ++r) {
 #pragma unroll
-            for (int q = 0; q < 8; ++q)
-#pragma unroll
-                for (int r = 0; r < 8; ++r) a[r] = a[r] - Ls[min(b0 + r, np - 1)][q0 + q] * uv[q];
-        }
-#pragma unroll
-        for (int r = 0; r < 8; ++r) {
-#pragma unroll
-            for (int r2 = r + 1; r2 < 8; ++r2) a[r2] = a[r2] - Ls[min(b0 + r2, np - 1)][min(b0 + r, np - 1)] * a[r];
-        }
-#pragma unroll
-        for (int r = 0; r < 8; ++r)
-            if (on && b0 + r < np) {
-                U[(int64_t)(b0 + r) * f + j] = a[r];
-                Q[(int64_t)(k0 + b0 + r) * f + j] = a[r] / dd[b0 + r];
+                for (int r2 = r + 1; r2 < g + 8; ++r2) a[r2] = a[r2] - Lc[r][r2] * a[r];
             }
-    }
+            // the block's rows in the rows after it
+#pragma unroll
+            for (int h = g + 8; h < LU_PANEL_MAX; h += 8)
+                if (h < np) {
+#pragma unroll
+                    for (int r = g; r < g + 8; ++r)
+#pragma unroll
+                        for (int r2 = h; r2 < h + 8; ++r2) a[r2] = a[r2] - Lc[r][r2] * a[r];
+                }
+#pragma unroll
+            for (int r = g; r < g + 8; ++r)
+                if (on && r < np) {
+                    U[(int64_t)r * f + j] = a[r];
+                    Q[(int64_t)(k0 + r) * f + j] = a[r] / dd[r];
+                }
+        }
 }
 
 // a panel's update of the entries after it: tile (s, I0, J0, scratch offset) of 64 x 64 entries, J0 < w: the
