@@ -863,15 +863,15 @@ inline int64_t lp_scratch(int f, int w, int cols) { return (int64_t)(LP_MAXP + 1
 // a front during a panel, as its NT threads see it
 template <typename T, int NT, int R, int MAXP>
 struct PanelFront {
-    T* P;
+    Global<T>* P;
     int f, w, k0;
-    int* lp;
+    Global<int>* lp;
     RedBuf<NT>* rb;
-    T *U, *DG;
-    T* V;  // the panel's columns kv, kv + 1, ... (MAXP - 1 of them, ld f) as they were before the pivot kv
-    // LDS: per column q of the panel (k0 + q) the kind of its pivot step: 0 none yet, 1 a 1x1,
-    // 2 the first and 3 the second column of a 2x2
-    int* ctype;
+    Global<T>*U, *DG;
+    Global<T>* V;  // the panel's columns kv, kv + 1, ... (MAXP - 1 of them, ld f) as they were before the pivot kv
+    // the panel's pivot steps, bit q for column k0 + q: the 1x1 pivots, the first columns of 2x2 ones
+    uint32_t one, two;
+    // LDS
     T* Uc;          // U(., j) of the column being formed
     T* Lr;          // L(r, .) of the pivot row whose U row is being formed
     T (*Ls)[MAXP];  // Ls[r][q] = L(k0 + r, k0 + q), q < r, of the panel's pivots
@@ -892,10 +892,9 @@ struct PanelFront {
             }
 #pragma unroll
             for (int q = 0; q < 8; ++q) {
-                const int ct = q0 + q < np ? uni(ctype[q0 + q]) : 0;
-                if (ct == 1)
+                if (one >> (q0 + q) & 1)
                     x = x - lv[q] * uv[q];
-                else if (ct == 2)
+                else if (two >> (q0 + q) & 1)
                     x = x - (lv[q] * uv[q] + lv[q + 1] * uv[q + 1]);
             }
         }
@@ -909,12 +908,12 @@ struct PanelFront {
         t = o - u * NT;
     }
     // the thread's rows of a column
-    __device__ __attribute__((always_inline)) void load_rows(const T* col, T (&y)[R]) const {
+    __device__ __attribute__((always_inline)) void load_rows(const Global<T>* col, T (&y)[R]) const {
         const auto rw = rows();
 #pragma unroll
         for (int u = 0; u < R; ++u) y[u] = load_at(col, rw.clamped(u));
     }
-    __device__ __attribute__((always_inline)) void store_rows(T* col, const T (&y)[R]) const {
+    __device__ __attribute__((always_inline)) void store_rows(Global<T>* col, const T (&y)[R]) const {
         const auto rw = rows();
         const int nf = rw.count(f);
 #pragma unroll
@@ -929,30 +928,30 @@ struct PanelFront {
             __syncthreads();
             return;
         }
-        constexpr int G = R <= 6 ? 8 : R <= 12 ? 4 : 2;
+        constexpr int G = R <= 3 ? 8 : R <= 6 ? 4 : 2;
         for (int q = threadIdx.x; q < np; q += NT) Uc[q] = U[(int64_t)q * w + j];
         __syncthreads();
         load_rows(P + (int64_t)j * f, y);
+#pragma unroll 1
         for (int q0 = 0; q0 < np; q0 += G) {
             const auto rw = rows();
             T l[G][R];
 #pragma unroll
             for (int g = 0; g < G; ++g) {
-                const T* cq = P + (int64_t)(k0 + min(q0 + g, np - 1)) * f;
+                const Global<T>* cq = P + (int64_t)(k0 + min(q0 + g, np - 1)) * f;
 #pragma unroll
                 for (int u = 0; u < R; ++u) l[g][u] = load_at(cq, rw.clamped(u));
             }
             __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
             for (int g = 0; g < G; ++g) {
-                const int ct = q0 + g < np ? uni(ctype[q0 + g]) : 0;
-                if (ct == 1) {
+                if (one >> (q0 + g) & 1) {
                     const T v = Uc[q0 + g];
 #pragma unroll
                     for (int u = 0; u < R; ++u) y[u] = y[u] - l[g][u] * v;
-                } else if (ct == 2) {
+                } else if (two >> (q0 + g) & 1) {
                     const T v = Uc[q0 + g], v2 = Uc[q0 + g + 1];
-                    const T* c2 = P + (int64_t)(k0 + q0 + g + 1) * f;
+                    const Global<T>* c2 = P + (int64_t)(k0 + q0 + g + 1) * f;
 #pragma unroll
                     for (int u = 0; u < R; ++u) y[u] = y[u] - (l[g][u] * v + load_at(c2, rw.clamped(u)) * v2);
                 }
@@ -964,9 +963,15 @@ struct PanelFront {
     __device__ __attribute__((always_inline)) void pick(const T (&y)[R], int i, int slot) const {
         int t, us;
         owner(i, t, us);
+        // (each entry hidden from the optimizer: as plain selects they become one load by a variable index,
+        // and the column a scratch array)
         T v = y[0];
 #pragma unroll
-        for (int u = 1; u < R; ++u) v = u == us ? y[u] : v;
+        for (int u = 1; u < R; ++u) {
+            T z = y[u];
+            asm("" : "+v"(z));
+            v = u == us ? z : v;
+        }
         if ((int)threadIdx.x == t) pk[slot] = (double)v;
     }
     // rows a and b of a column in registers exchanged (pk[sa], pk[sb]: its entries there)
@@ -1014,7 +1019,7 @@ struct PanelFront {
         const int np = r - k0;
         for (int q = threadIdx.x; q < np; q += NT) Lr[q] = P[(int64_t)(k0 + q) * f + r];
         __syncthreads();
-        T* ur = U + (int64_t)np * w;
+        Global<T>* ur = U + (int64_t)np * w;
         for (int j = j0 + threadIdx.x; j < w; j += NT)
             ur[j] = apply(P[(int64_t)j * f + r], np, [&](int q) { return Lr[q]; },
                           [&](int q) { return U[(int64_t)q * w + j]; });
@@ -1024,7 +1029,7 @@ struct PanelFront {
     // there: a thread per column, eight rows at a time (all threads; ends with a barrier)
     __device__ __attribute__((always_inline)) void form_urows(int n0, int n1) const {
         for (int j = k0 + n1 + threadIdx.x; j < w; j += NT) {
-            const T* cj = P + (int64_t)j * f + k0;
+            const Global<T>* cj = P + (int64_t)j * f + k0;
 #pragma unroll 1
             for (int b0 = n0; b0 < n1; b0 += 8) {
                 T a[8];
@@ -1037,11 +1042,11 @@ struct PanelFront {
                     for (int q = 0; q < 9; ++q) uv[q] = U[(int64_t)min(q0 + q, b0 - 1) * w + j];
 #pragma unroll
                     for (int q = 0; q < 8; ++q) {
-                        const int ct = q0 + q < b0 ? uni(ctype[q0 + q]) : 0;
-                        if (ct == 1) {
+                        if (q0 + q >= b0) break;
+                        if (one >> (q0 + q) & 1) {
 #pragma unroll
                             for (int r = 0; r < 8; ++r) a[r] = a[r] - Ls[min(b0 + r, n1 - 1)][q0 + q] * uv[q];
-                        } else if (ct == 2) {
+                        } else if (two >> (q0 + q) & 1) {
 #pragma unroll
                             for (int r = 0; r < 8; ++r)
                                 a[r] = a[r] - (Ls[min(b0 + r, n1 - 1)][q0 + q] * uv[q] +
@@ -1066,7 +1071,8 @@ struct PanelFront {
     __device__ __attribute__((always_inline)) void update_v(int q, const T (&la)[R], const T (&lb)[R]) const {
         constexpr int G = R <= 3 ? 8 : R <= 6 ? 4 : R <= 12 ? 2 : 1;
         const int n = min(MAXP - 1, w - k0) - q;  // V's columns inside the panel
-        const T* u0 = U + (int64_t)q * w + k0 + q;
+        const Global<T>* u0 = U + (int64_t)q * w + k0 + q;
+#pragma unroll 1
         for (int c0 = TWO ? 2 : 1; c0 < n; c0 += G) {
             const auto rw = rows();
             const int nf = rw.count(f);
@@ -1130,13 +1136,64 @@ struct PanelFront {
         c = k;
         if (p.pivot == PV_NONE) return;
         pick(xa, k, 0);
-        T y[R];
+        const double mk = colmax(xa, k, f, k, k);
+        const double akk = fabs(pk[0]);
+        bool ok, two2 = false;
+        double det = 0.0, mx = 0.0;
+        int rr = -1;
         if (p.pivot == PV_DIAG) {
-            const double m = colmax(xa, k, f, k, k);
-            const double akk = fabs(pk[0]);
-            if (uni(akk >= p.eps && akk >= p.u * m)) return;
+            ok = akk >= p.eps && akk >= p.u * mk;
+        } else {
+            const double alpha = (1.0 + sqrt(17.0)) / 8.0;  // Bunch-Kaufman constant (ldlt.jl:22)
+            double lambda = 0.0;
+            {
+                const int n = rows().count(w);
+                const bool up = (int)threadIdx.x > k - k0;
+#pragma unroll
+                for (int u = 0; u < R; ++u) {
+                    const double a = fabs((double)xa[u]);
+                    if (u < n && (u > 0 || up) && a > lambda) {
+                        lambda = a;
+                        rr = u;
+                    }
+                }
+                if (rr >= 0) rr = k0 + (int)threadIdx.x + NT * rr;
+            }
+            block_argmax<NT>(lambda, rr, *rb);
+            rr = uni(rr);
+            if (rr < 0) lambda = 0.0;
+            if (rr < 0 || uni(akk >= alpha * lambda)) {
+                ok = akk >= p.eps && akk >= p.u * mk;
+            } else {
+                form_col(rr, np, xb);
+                pick(xa, rr, 1);
+                pick(xb, k, 2);
+                pick(xb, rr, 3);
+                const double sigma = colmax(xb, k, w, rr, rr);
+                const double arr = pk[3], ark = pk[1], akr = pk[2];
+                if (uni(akk * sigma >= alpha * lambda * lambda)) {
+                    ok = akk >= p.eps && akk >= p.u * mk;
+                } else if (uni(fabs(arr) >= alpha * sigma)) {
+                    c = rr;
+                    ok = fabs(arr) >= p.eps && fabs(arr) >= p.u * colmax(xb, k, f, rr, rr);
+                } else {
+                    two2 = true;
+                    det = pk[0] * arr - akr * ark;
+                    mx = jmax(jmax(akk, fabs(ark)), fabs(arr));
+                    ok = det != 0.0 && isfinite(det) && mx >= p.eps;
+                    if (uni(ok)) {
+                        const double e11 = fabs(arr / det), e12 = fabs(akr / det), e21 = fabs(ark / det),
+                                     e22 = fabs(pk[0] / det);
+                        const double m1 = colmax(xa, k, f, k, rr), m2 = colmax(xb, k, f, rr, k);
+                        ok = p.u * (e11 * m1 + e21 * m2) <= 1.0 && p.u * (e12 * m1 + e22 * m2) <= 1.0;
+                    }
+                }
+            }
+        }
+        if (!uni(ok)) {
+            T y[R];
             int best = best_1x1(k, p, y);
-            if (best < 0) {
+            if (best < 0 && p.pivot == PV_DIAG) {
                 // the largest diagonal entry, first on ties; a NaN |a_kk| keeps k (DG was formed by
                 // best_1x1)
                 double v = akk;
@@ -1153,72 +1210,15 @@ struct PanelFront {
                 if (best == k) return;
                 form_col(best, np, y);
             }
-            c = best;
-#pragma unroll
-            for (int u = 0; u < R; ++u) xa[u] = y[u];
-            return;
-        }
-        const double alpha = (1.0 + sqrt(17.0)) / 8.0;  // Bunch-Kaufman constant (ldlt.jl:22)
-        double lambda = 0.0;
-        int rr = -1;
-        {
-            const int n = rows().count(w);
-            const bool up = (int)threadIdx.x > k - k0;
-#pragma unroll
-            for (int u = 0; u < R; ++u) {
-                const double a = fabs((double)xa[u]);
-                if (u < n && (u > 0 || up) && a > lambda) {
-                    lambda = a;
-                    rr = u;
-                }
-            }
-            if (rr >= 0) rr = k0 + (int)threadIdx.x + NT * rr;
-        }
-        block_argmax<NT>(lambda, rr, *rb);
-        rr = uni(rr);
-        if (rr < 0) lambda = 0.0;
-        const double akk = fabs(pk[0]);
-        const double mk = colmax(xa, k, f, k, k);
-        bool ok, two = false;
-        double det = 0.0, mx = 0.0;
-        if (rr < 0 || uni(akk >= alpha * lambda)) {
-            ok = akk >= p.eps && akk >= p.u * mk;
-        } else {
-            form_col(rr, np, xb);
-            pick(xa, rr, 1);
-            pick(xb, k, 2);
-            pick(xb, rr, 3);
-            const double sigma = colmax(xb, k, w, rr, rr);
-            const double arr = pk[3], ark = pk[1], akr = pk[2];
-            if (uni(akk * sigma >= alpha * lambda * lambda)) {
-                ok = akk >= p.eps && akk >= p.u * mk;
-            } else if (uni(fabs(arr) >= alpha * sigma)) {
-                c = rr;
-                ok = fabs(arr) >= p.eps && fabs(arr) >= p.u * colmax(xb, k, f, rr, rr);
-            } else {
-                two = true;
-                det = pk[0] * arr - akr * ark;
-                mx = jmax(jmax(akk, fabs(ark)), fabs(arr));
-                ok = det != 0.0 && isfinite(det) && mx >= p.eps;
-                if (uni(ok)) {
-                    const double e11 = fabs(arr / det), e12 = fabs(akr / det), e21 = fabs(ark / det),
-                                 e22 = fabs(pk[0] / det);
-                    const double m1 = colmax(xa, k, f, k, rr), m2 = colmax(xb, k, f, rr, k);
-                    ok = p.u * (e11 * m1 + e21 * m2) <= 1.0 && p.u * (e12 * m1 + e22 * m2) <= 1.0;
-                }
-            }
-        }
-        if (!uni(ok)) {
-            const int best = best_1x1(k, p, y);
             if (best >= 0) {
                 c = best;
 #pragma unroll
                 for (int u = 0; u < R; ++u) xa[u] = y[u];
                 return;
             }
-            two = uni(two && det != 0.0 && isfinite(det) && mx >= p.eps);  // (a singular 2x2: k as a 1x1)
+            two2 = uni(two2 && det != 0.0 && isfinite(det) && mx >= p.eps);  // (a singular 2x2: k as a 1x1)
         }
-        if (two) {
+        if (two2) {
             r = rr;
         } else if (c != k) {
 #pragma unroll
@@ -1288,7 +1288,8 @@ struct PanelRegs {
 template <typename T, int NT, int R, int NBP, int W, class Z>
 __device__ __attribute__((always_inline)) inline bool panel_pivots(PanelRegs<T, R, NBP>& X, const Z& F, int& k, int kend,
                                                                    const LdltPrm& p, double (*red)[NT / 64][2],
-                                                                   T (*urow)[NBP], int8_t* kind, T* dd) {
+                                                                   T (*urow)[NBP], int* ctype, Global<int8_t>* kind,
+                                                                   Global<T>* dd) {
     const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6, f = F.f, w = F.w, k0 = F.k0;
     const double alpha = (1.0 + sqrt(17.0)) / 8.0;  // Bunch-Kaufman constant (ldlt.jl:22)
     const int kstop = min(kend, k0 + NBP - (W > 8 ? W - 8 : 0));
@@ -1339,7 +1340,7 @@ __device__ __attribute__((always_inline)) inline bool panel_pivots(PanelRegs<T, 
         if (p.pivot != PV_NONE) fast = fast && !nan && akk >= p.u * mx;
         if (p.pivot == PV_BK) fast = fast && akk >= alpha * lam;
         if (!uni(fast)) return false;
-        T* col = F.P + (int64_t)k * f;
+        Global<T>* col = F.P + (int64_t)k * f;
         // the scaling of three row slots at a time (independent divisions), then their updates
 #pragma unroll
         for (int u0 = 0; u0 < R; u0 += 3) {
@@ -1359,7 +1360,7 @@ __device__ __attribute__((always_inline)) inline bool panel_pivots(PanelRegs<T, 
         if (tid == 0) {
             kind[k] = KIND_1X1;
             dd[k] = d;
-            F.ctype[k - k0] = 1;
+            ctype[k - k0] = 1;
         }
         if (d > T(0))
             X.npos++;
@@ -1368,23 +1369,6 @@ __device__ __attribute__((always_inline)) inline bool panel_pivots(PanelRegs<T, 
         ++k;
     }
     return true;
-}
-
-// the LDS words of a panel
-template <typename T, int NBP>
-struct PanelLds {
-    RedBuf<512> rb;
-    double pk[4];
-    int ctype[NBP + 1];
-    T Uc[NBP + 1], Lr[NBP + 1];
-    T Ls[NBP + 1][NBP + 1];
-    __align__(16) double red[2][512 / 64][2];
-    __align__(16) T urow[2][NBP];
-};
-template <typename T, int NBP>
-__device__ inline PanelLds<T, NBP>& panel_lds() {
-    __shared__ PanelLds<T, NBP> lds;
-    return lds;
 }
 
 // a front's arrays during a panel
@@ -1399,39 +1383,62 @@ struct PanelArgs {
     const int32_t* perm_c0;
     LdltPrm prm;
 };
+// the LDS words of a panel. The front's arrays are kept here too: panel_general reads them back, so that they
+// take no scalar registers during the usual pivots. ctype: per column q of the panel (k0 + q) the kind
+// of its pivot step: 0 none yet, 1 a 1x1, 2 the first and 3 the second column of a 2x2
+template <typename T, int NBP>
+struct PanelLds {
+    PanelArgs<T> args;
+    RedBuf<512> rb;
+    double pk[4];
+    int ctype[NBP + 1];
+    T Uc[NBP + 1], Lr[NBP + 1];
+    T Ls[NBP + 1][NBP + 1];
+    __align__(16) double red[2][512 / 64][2];
+    __align__(16) T urow[2][NBP];
+};
+template <typename T, int NBP>
+__device__ inline PanelLds<T, NBP>& panel_lds() {
+    __shared__ PanelLds<T, NBP> lds;
+    return lds;
+}
 template <typename T, int R, int NBP>
-__device__ __attribute__((always_inline)) inline PanelFront<T, 512, R, NBP + 1> panel_front(const PanelArgs<T>& A) {
+__device__ __attribute__((always_inline)) inline PanelFront<T, 512, R, NBP + 1> panel_front() {
     PanelLds<T, NBP>& S = panel_lds<T, NBP>();
-    T* DG = A.U + (int64_t)LP_MAXP * A.w;
-    return PanelFront<T, 512, R, NBP + 1>{A.P,     A.f,     A.w,  A.k0, A.lp, &S.rb, A.U, DG, DG + A.w,
-                                          S.ctype, S.Uc, S.Lr, S.Ls, S.pk};
+    const PanelArgs<T>& A = S.args;
+    const int w = uni(A.w), lane = threadIdx.x & 63, ct = S.ctype[min(lane, NBP)];
+    Global<T>*U = uni_ptr(A.U), *DG = U + (int64_t)LP_MAXP * w;
+    return PanelFront<T, 512, R, NBP + 1>{uni_ptr(A.P), uni(A.f), w, uni(A.k0), uni_ptr(A.lp), &S.rb, U, DG, DG + w,
+                                          (uint32_t)__ballot(lane <= NBP && ct == 1),
+                                          (uint32_t)__ballot(lane <= NBP && ct == 2), S.Uc, S.Lr, S.Ls, S.pk};
 }
 
 // any pivot but the usual one, at column k, from the panel memory (V holds the panel's columns from k
-// on, nu pivot rows are formed); returns the next column. A function of its own: the panel's
-// registers are free while it runs.
+// on, nu pivot rows are formed); returns the next column. Part of the kernel: the panel's registers are free
+// meanwhile. As a function of its own, its pointers in a struct, it had its columns and the caller's
+// registers in scratch memory and every access a flat one (36 us a pivot instead of 23).
 template <typename T, int R, int NBP>
-__device__ __attribute__((noinline)) int panel_general(const PanelArgs<T> A,
-                                                                                             int k, int nu) {
-    const auto Z = panel_front<T, R, NBP>(A);
-    const int tid = threadIdx.x, f = uni(A.f), k0 = uni(A.k0);
-    const LdltPrm& prm = A.prm;
-    T* P = A.P;
-    T *dd = A.dd, *ee = A.ee;
-    int* lp = A.lp;
-    int* ctype = Z.ctype;
-    double* pk = Z.pk;
-    int8_t* kind = A.kind;
-    int64_t* st = A.st;
-    const int8_t* sreq_row = A.sreq_row;
-    const int32_t* perm_c0 = A.perm_c0;
+__device__ __attribute__((always_inline)) inline int panel_general(int k, int nu) {
+    const auto Z = panel_front<T, R, NBP>();
+    PanelLds<T, NBP>& S = panel_lds<T, NBP>();
+    const PanelArgs<T>& A = S.args;
+    const LdltPrm prm = {uni(A.prm.pivot), A.prm.u, A.prm.eps};
+    const int tid = threadIdx.x, f = Z.f, k0 = Z.k0;
+    k = uni(k);
+    nu = uni(nu);
+    Global<T>*P = Z.P, *dd = uni_ptr(A.dd), *ee = uni_ptr(A.ee);
+    Global<int>* lp = Z.lp;
+    int* ctype = S.ctype;
+    double* pk = S.pk;
+    Global<int8_t>* kind = uni_ptr(A.kind);
+    Global<int64_t>* st = uni_ptr(A.st);
     T xa[R], xb[R];
     Z.load_rows(Z.V, xa);
     if (nu < k - k0) Z.form_urows(nu, k - k0);
     int c, r;
     Z.choose(k, prm, c, r, xa, xb);
     __syncthreads();
-    T* ck = P + (int64_t)k * f;
+    Global<T>* ck = P + (int64_t)k * f;
     if (r < 0) {
         Z.template swap<false>(k, c, k - k0, xa, xb);
         Z.pick(xa, k, 0);
@@ -1441,7 +1448,7 @@ __device__ __attribute__((noinline)) int panel_general(const PanelArgs<T> A,
             int8_t kd = KIND_1X1;
             if (!(fabs(d) >= prm.eps) || d == 0.0) {
                 if (d == 0.0) st[ST_NZERO]++;
-                const int req = sreq_row ? (int)sreq_row[perm_c0[lp[k]]] : 0;
+                const int req = A.sreq_row ? (int)A.sreq_row[A.perm_c0[lp[k]]] : 0;
                 const double sg = req != 0 ? (double)req : (d < 0.0 ? -1.0 : 1.0);
                 d = sg * prm.eps;
                 kd = KIND_PERTURBED;
@@ -1542,6 +1549,7 @@ __global__ void __launch_bounds__(512) k_ldlt_panel(DevSym S, const Task* __rest
                                                     const double* __restrict__ aux, const int8_t* __restrict__ psign) {
     constexpr int NT = 512;
     constexpr int MAXP = NBP + 1;
+    static_assert(NBP == 4 || NBP == 8 || NBP == 16, "the usual pivots come in two runs: of NBP columns, then of 8");
     const Task tk = tasks[blockIdx.x];
     const int s = tk.s;
     const int f = S.fnrows[s], w = S.fncols[s];
@@ -1574,17 +1582,15 @@ __global__ void __launch_bounds__(512) k_ldlt_panel(DevSym S, const Task* __rest
     }
     const int k0 = k, kend = min(w, k0 + NBP);
     PanelLds<T, NBP>& D = panel_lds<T, NBP>();
-    auto& Ls = D.Ls;
     for (int q = tid; q < MAXP; q += NT) D.ctype[q] = 0;
-    T* base = scratch + tk.a;
-    const PanelArgs<T> A{P, base, dd, ee, f, w, k0, lp, kind, st, psign, S.perm + c0, prm};
-    const auto Z = panel_front<T, R, NBP>(A);
+    if (tid == 0) D.args = {P, scratch + tk.a, dd, ee, f, w, k0, lp, kind, st, psign, S.perm + c0, prm};
     const int nr = (f - k0 + NT - 1) / NT;
     int nu = 0;  // U rows formed
     int kv = k0;  // the last general pivot
     int npos = 0, nneg = 0;
     while (k < kend) {
         __syncthreads();
+        const auto Z = panel_front<T, R, NBP>();
         PanelRegs<T, R, NBP> X;
         X.nr = nr;
         X.buf = 0;
@@ -1593,9 +1599,9 @@ __global__ void __launch_bounds__(512) k_ldlt_panel(DevSym S, const Task* __rest
         const int np = k - k0, last = k - kv;  // (last: columns of that pivot, 0 at the panel's start)
         for (int q = tid; q < MAXP * np; q += NT) {
             const int pp = q / MAXP, r = q - pp * MAXP;
-            if (r > pp && k0 + r < f) Ls[r][pp] = P[(int64_t)(k0 + pp) * f + k0 + r];
+            if (r > pp && k0 + r < f) D.Ls[r][pp] = Z.P[(int64_t)(k0 + pp) * f + k0 + r];
         }
-        const T* src = last ? Z.V + (int64_t)last * f : P + (int64_t)k * f;
+        const Global<T>* src = last ? Z.V + (int64_t)last * f : Z.P + (int64_t)k * f;
         const int cmax = last ? NBP - 1 - last : w - 1 - k;
         {
             const auto rw = Z.rows();
@@ -1609,8 +1615,10 @@ __global__ void __launch_bounds__(512) k_ldlt_panel(DevSym S, const Task* __rest
         }
         __syncthreads();
         bool go = true;
-        if constexpr (NBP > 8) go = panel_pivots<T, NT, R, NBP, NBP>(X, Z, k, kend, prm, D.red, D.urow, kind, dd);
-        if (go) go = panel_pivots<T, NT, R, NBP, (NBP < 8 ? NBP : 8)>(X, Z, k, kend, prm, D.red, D.urow, kind, dd);
+        Global<int8_t>* gkind = uni_ptr(D.args.kind);
+        Global<T>* gdd = uni_ptr(D.args.dd);
+        if constexpr (NBP > 8) go = panel_pivots<T, NT, R, NBP, NBP>(X, Z, k, kend, prm, D.red, D.urow, D.ctype, gkind, gdd);
+        if (go) go = panel_pivots<T, NT, R, NBP, (NBP < 8 ? NBP : 8)>(X, Z, k, kend, prm, D.red, D.urow, D.ctype, gkind, gdd);
         __syncthreads();  // the L columns are stored, the LDS words of the last pivot read
         npos += X.npos;
         nneg += X.nneg;
@@ -1630,11 +1638,11 @@ __global__ void __launch_bounds__(512) k_ldlt_panel(DevSym S, const Task* __rest
             }
         }
         __syncthreads();
-        k = uni(panel_general<T, R, NBP>(A, k, nu));
+        k = uni(panel_general<T, R, NBP>(k, nu));
         nu = k - k0;
     }
     // the rest of the pivot rows for the columns after the panel
-    if (nu < k - k0 && k < w) Z.form_urows(nu, k - k0);
+    if (nu < k - k0 && k < w) panel_front<T, R, NBP>().form_urows(nu, k - k0);
     if (tid == 0) {
         st[ST_NPOS] += npos;
         st[ST_NNEG] += nneg;
@@ -1866,15 +1874,20 @@ void launch_ldlt_pivot(hipStream_t st, const DevSym& S, const Task* tasks, int n
 }
 
 template <typename T>
-void launch_ldlt_panel(hipStream_t st, const DevSym& S, const Task* tasks, int n, int first, int cols, T* factor,
-                       T* dvec, int32_t* piv, int8_t* kind, int64_t* stats, int32_t* lstep, T* scratch, int pivot,
+void launch_ldlt_panel(hipStream_t st, const DevSym& S, const Task* tasks, int n, int first, int cols, int rows,
+                       T* factor, T* dvec, int32_t* piv, int8_t* kind, int64_t* stats, int32_t* lstep, T* scratch, int pivot,
                        double u, double eps, int scaled, const double* aux, const int8_t* psign) {
     LdltPrm p{pivot, u, eps};
 #define PANEL(R, C)                                                                                                  \
     hipLaunchKernelGGL((k_ldlt_panel<T, R, C>), dim3(n), dim3(512), 0, st, S, tasks, first, factor, dvec, piv, kind, \
                        stats, lstep, scratch, p, scaled, aux, psign)
     switch (cols) {
-        case 16: PANEL(6, 16); break;
+        case 16:
+            if (rows <= 3 * 512)
+                PANEL(3, 16);
+            else
+                PANEL(6, 16);
+            break;
         case 8: PANEL(10, 8); break;
         default: PANEL(14, 4); break;
     }
@@ -1943,8 +1956,8 @@ void launch_info_from_stats(hipStream_t st, const DevSym& S, const int64_t* stat
                                        const int8_t*);                                                             \
     template void launch_ldlt_update<T>(hipStream_t, const DevSym&, const Task*, int, T*, const int32_t*);        \
     template void launch_ldlt_mirror<T>(hipStream_t, const DevSym&, const Task*, int, T*);                        \
-    template void launch_ldlt_panel<T>(hipStream_t, const DevSym&, const Task*, int, int, int, T*, T*, int32_t*,   \
-                                       int8_t*, int64_t*, int32_t*, T*, int, double, double, int, const double*,   \
+    template void launch_ldlt_panel<T>(hipStream_t, const DevSym&, const Task*, int, int, int, int, T*, T*,        \
+                                       int32_t*, int8_t*, int64_t*, int32_t*, T*, int, double, double, int, const double*,   \
                                        const int8_t*);                                                             \
     template void launch_ldlt_trail<T>(hipStream_t, const DevSym&, const Task*, int, T*, const int8_t*,           \
                                        const int32_t*, const T*);                                                  \

@@ -53,14 +53,34 @@ __device__ inline int wave_min_last(int v) {
     return dpp_min_step<0x143, 0xc>(v);
 }
 
+// pointers into global memory that say so: one that was itself read from memory is otherwise taken for
+// a pointer to anything, its accesses become flat ones, and those are waited for together with the LDS
+template <typename T>
+using Global = __attribute__((address_space(1))) T;
+// such a pointer from an address every lane holds, in scalar registers
+template <typename T>
+__device__ inline Global<T>* uni_ptr(T* p) {
+    const uint64_t a = reinterpret_cast<uint64_t>(p);
+    const uint32_t lo = __builtin_amdgcn_readfirstlane((int)a), hi = __builtin_amdgcn_readfirstlane((int)(a >> 32));
+    return (Global<T>*)((uint64_t)hi << 32 | lo);
+}
+
 // entry `off` bytes into the column `col` (a wave-uniform address: scalar base, 32-bit offset)
 template <typename T>
 __device__ inline T load_at(const T* col, uint32_t off) {
     return *reinterpret_cast<const T*>(reinterpret_cast<const char*>(col) + off);
 }
 template <typename T>
+__device__ inline T load_at(const Global<T>* col, uint32_t off) {
+    return *(const Global<T>*)((const Global<char>*)col + off);
+}
+template <typename T>
 __device__ inline void store_at(T* col, uint32_t off, T v) {
     *reinterpret_cast<T*>(reinterpret_cast<char*>(col) + off) = v;
+}
+template <typename T>
+__device__ inline void store_at(Global<T>* col, uint32_t off, T v) {
+    *(Global<T>*)((Global<char>*)col + off) = v;
 }
 
 // a thread's rows k0 + tid + NT u of a front: their byte offsets in a column and how many lie above an

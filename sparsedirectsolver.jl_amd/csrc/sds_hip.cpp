@@ -89,6 +89,7 @@ struct Launch {
     double flops, bytes;  // algorithmic work of the launch
     int nstep = 0, ncopy = 0;  // k_big_step launches: step tasks, then copies, then update tiles; panel columns
     int k = 0;                 // pivot step of the pivot and panel launches
+    int rows = 0;              // panel launches: most rows of a front from that step on
 };
 
 struct Level {
@@ -1001,6 +1002,8 @@ int build_schedule(sds_handle* h, int dtype) {
                 L.plan.push_back({panel ? L_LDLT_PANEL : L_LDLT_PIVOT, off_p, (int)tp.size(), 0.0, 0.0});
                 L.plan.back().k = k;
                 L.plan.back().nstep = cols;
+                for (int32_t s : L.big)
+                    if (h->fncols[s] > k) L.plan.back().rows = std::max(L.plan.back().rows, h->fnrows[s] - k);
                 if (k + cols < wmax)
                     L.plan.push_back({panel ? L_LDLT_TRAIL : L_LDLT_UPDATE, off_u, n_u, fl1, by1});
             }
@@ -1549,7 +1552,7 @@ int factorize_ldlt(sds_handle* h, const double* nz, int pivot, double u, double 
                     case L_LDLT_UPDATE: launch_ldlt_update<T>(st, h->dsym, t, ln.n, factor, h->lstep); break;
                     case L_LDLT_MIRROR: launch_ldlt_mirror<T>(st, h->dsym, t, ln.n, factor); break;
                     case L_LDLT_PANEL:
-                        launch_ldlt_panel<T>(st, h->dsym, t, ln.n, ln.k == 0, ln.nstep, factor, dv, h->piv, h->pkind,
+                        launch_ldlt_panel<T>(st, h->dsym, t, ln.n, ln.k == 0, ln.nstep, ln.rows, factor, dv, h->piv, h->pkind,
                                              h->stats, h->lstep, static_cast<T*>(h->lscratch), pivot, u, eps, scaled, h->aux,
                                              psign);
                         break;

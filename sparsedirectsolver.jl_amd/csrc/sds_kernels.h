@@ -71,8 +71,8 @@ void launch_ldlt_mirror(hipStream_t st, const DevSym& S, const Task* tasks, int 
 // offset); `first`: the fronts' first launch), then their update of the columns after them (task
 // (s, I0, J0, scratch offset))
 template <typename T>
-void launch_ldlt_panel(hipStream_t st, const DevSym& S, const Task* tasks, int n, int first, int cols, T* factor,
-                       T* dvec, int32_t* piv, int8_t* kind, int64_t* stats, int32_t* lstep, T* scratch, int pivot,
+void launch_ldlt_panel(hipStream_t st, const DevSym& S, const Task* tasks, int n, int first, int cols, int rows,
+                       T* factor, T* dvec, int32_t* piv, int8_t* kind, int64_t* stats, int32_t* lstep, T* scratch, int pivot,
                        double u, double eps, int scaled, const double* aux, const int8_t* psign);
 template <typename T>
 void launch_ldlt_trail(hipStream_t st, const DevSym& S, const Task* tasks, int n, T* factor, const int8_t* kind,

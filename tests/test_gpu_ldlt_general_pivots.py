@@ -1,0 +1,53 @@
+"""LDL^T of a dense front where hardly any pivot is its column's own 1x1: the default form must not be slower than
+the other one (they give the same factor; only the launches differ). The cases are far from the line:
+the fault each was written for made the default 1.6 times as slow or slower.
+"""
+import time
+
+import numpy as np
+import pytest
+
+import sparsedirectsolver as sds
+from sparsedirectsolver.solver import set_tiles
+
+pytestmark = pytest.mark.gpu
+
+TILES = dict(extend_add_rows=1024, cb_k_chunk=32, trailing_split=0, step_two_per_cu=0)
+
+
+def _seconds(s):
+    import torch
+    sds.execute("factorization", s)
+    best = np.inf
+    for _ in range(3):
+        torch.cuda.synchronize()
+        t = time.perf_counter()
+        sds.execute("refactorization", s)
+        torch.cuda.synchronize()
+        best = min(best, time.perf_counter() - t)
+    return best
+
+
+# a zero diagonal takes 2x2 pivots and interchanges nearly everywhere
+@pytest.mark.parametrize("n,diag,ptype,threshold", [(1500, 0.0, "A", 0.01)])
+def test_default_form_is_not_slower_than_the_other(n, diag, ptype, threshold):
+    rng = np.random.default_rng(n)
+    A = rng.standard_normal((n, n))
+    A = A + A.T
+    A[np.arange(n), np.arange(n)] = diag * rng.standard_normal(n)
+    cols = np.concatenate([np.arange(1, i + 2) for i in range(n)])
+    rowptr = 1 + np.concatenate([[0], np.cumsum(np.arange(1, n + 1))])
+    s = sds.DirectSolver((rowptr, cols, A[np.tril_indices(n)], n), "S", "L")
+    sds.setparam(s, "user_perm", np.arange(1, n + 1))
+    sds.setparam(s, "pivot_pairs", "none")
+    sds.setparam(s, "pivot_type", ptype)
+    sds.setparam(s, "pivot_threshold", threshold)
+    sds.execute("analysis", s)
+    default = _seconds(s)
+    forms = []
+    for form in (0, 1):
+        set_tiles(s, dict(TILES, pivot_panels=form))
+        forms.append(_seconds(s))
+    print(f"n={n} diag={diag} {ptype} u={threshold}: default {1e3 * default:.1f} ms, forms "
+          f"{[round(1e3 * t, 1) for t in forms]} ms", flush=True)
+    assert default <= 1.25 * min(forms)
