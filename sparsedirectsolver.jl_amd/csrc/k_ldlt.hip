@@ -876,6 +876,7 @@ struct PanelFront {
     T* Lr;          // L(r, .) of the pivot row whose U row is being formed
     T (*Ls)[MAXP];  // Ls[r][q] = L(k0 + r, k0 + q), q < r, of the panel's pivots
     double* pk;     // picked entries (pick)
+    double (*mx3)[NT / 64];  // the waves' maxima, three at a time
 
     // x minus the panel's first np pivots in order, l(q) = L(row, k0 + q) and u(q) = U(k0 + q,
     // column) (the operations and their order of ldlt_front's updates); eight pivots' entries are
@@ -987,8 +988,8 @@ struct PanelFront {
             y[u] = mb && u == ub ? va : y[u];
         }
     }
-    // largest |y_i| over the rows k..f-1 but s1 and s2, NaN-propagating (ldlt.jl:240-260)
-    __device__ __attribute__((always_inline)) double colmax(const T (&y)[R], int k, int end, int s1, int s2) const {
+    // largest |y_i| over the thread's rows k..end-1 but s1 and s2, NaN-propagating (ldlt.jl:240-260)
+    __device__ __attribute__((always_inline)) double rows_max(const T (&y)[R], int k, int end, int s1, int s2) const {
         // (rows above k: only among the first slot's, the panel is narrower than the block)
         double m = 0.0;
         const int n = rows().count(end);
@@ -1004,7 +1005,11 @@ struct PanelFront {
             if (u == u2) on = on && !m2;
             m = on ? jmax(m, fabs((double)y[u])) : m;
         }
-        return block_jmax<NT>(m, *rb);
+        return m;
+    }
+    // the same over the whole front
+    __device__ __attribute__((always_inline)) double colmax(const T (&y)[R], int k, int end, int s1, int s2) const {
+        return block_jmax<NT>(rows_max(y, k, end, s1, s2), *rb);
     }
     // current diagonal entries of the columns k..w-1 into DG (all threads; ends with a barrier)
     __device__ __attribute__((always_inline)) void form_diag(int k) const {
@@ -1098,33 +1103,140 @@ struct PanelFront {
             }
         }
     }
-    // best_1x1 (ldlt.jl:264-276) on the current diagonal (formed here): the acceptable 1x1 pivot of
-    // k..w-1 with the largest |a_jj|, first on ties, -1 if none: the candidates (|a_jj| >= eps) in
-    // that order, each one's current column formed in y (which holds the answer's on return) and
-    // tested by the whole block. The first one is usually the answer, and where none is, few are
-    // left (KKT, n = 12,000: the first of 367 of 619 searches, none of 6 candidates on average in 169).
-    __device__ __attribute__((always_inline)) int best_1x1(int k, const LdltPrm& p, T (&y)[R]) const {
-        form_diag(k);
-        double last = 0.0;
-        int lj = -1;
-        while (true) {
-            double v = -1.0;
-            int bi = -1;
-            for (int j = k + threadIdx.x; j < w; j += NT) {
-                const double a = fabs((double)DG[j]);
-                if (a >= p.eps && (lj < 0 || a < last || (a == last && j > lj)) && vi_better(a, j, v, bi)) {
-                    v = a;
-                    bi = j;
+    // the current entries (rows i[t], columns j[c]) of NC columns from their stored ones in x, by one wave; the
+    // columns share the loads of L, four pivots' at a time. ul[c]: U(., j[c]), a pivot a lane
+    template <int NC, int NR>
+    __device__ __attribute__((always_inline)) void wave_apply(int np, const int (&i)[NR], const T (&ul)[NC],
+                                                              T (&x)[NC][NR]) const {
+#pragma unroll 1
+        for (int q0 = 0; q0 < np; q0 += 4) {
+            T l[5][NR];  // (the fifth: the second column of a 2x2)
+#pragma unroll
+            for (int g = 0; g < 5; ++g)
+#pragma unroll
+                for (int t = 0; t < NR; ++t) l[g][t] = P[(int64_t)(k0 + min(q0 + g, np - 1)) * f + i[t]];
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int g = 0; g < 4; ++g) {
+                const int q1 = min(q0 + g, np - 1), q2 = min(q0 + g + 1, np - 1);
+                if (one >> (q0 + g) & 1) {
+#pragma unroll
+                    for (int c = 0; c < NC; ++c)
+#pragma unroll
+                        for (int t = 0; t < NR; ++t) x[c][t] = x[c][t] - l[g][t] * lane_bcast(ul[c], q1);
+                } else if (two >> (q0 + g) & 1) {
+#pragma unroll
+                    for (int c = 0; c < NC; ++c)
+#pragma unroll
+                        for (int t = 0; t < NR; ++t)
+                            x[c][t] = x[c][t] - (l[g][t] * lane_bcast(ul[c], q1) + l[g + 1][t] * lane_bcast(ul[c], q2));
                 }
             }
-            block_argmax<NT>(v, bi, *rb);
-            bi = uni(bi);
-            if (bi < 0) return -1;
-            form_col(bi, k - k0, y);
-            if (uni(v >= p.u * colmax(y, k, f, bi, bi))) return bi;
-            last = v;
-            lj = bi;
         }
+    }
+    // the best acceptable 1x1 pivot among the columns k..w-1 but `first`, their current diagonal in DG, each
+    // tested by one wave unless it cannot beat the wave's best: eight columns together on 64 rows, where
+    // most of those that fail do, the others on all rows. A column passes where a = |a_jj| >= u |a_ij| for
+    // every other row, which is the test of the largest (a product with u is monotone). All threads get
+    // the answer (-1 if none)
+    __device__ __attribute__((always_inline)) int search_1x1(int k, int first, const LdltPrm& p) const {
+        constexpr int NC = 8;
+        const int wv = uni(threadIdx.x >> 6), lane = threadIdx.x & 63, np = k - k0;
+        double bv = -1.0;
+        int bj = -1;
+#pragma unroll 1
+        for (int j0 = k + NC * wv; j0 < w; j0 += NC * (NT / 64)) {
+            double a[NC];
+            T x[NC][1], ul[NC];
+            const int i[1] = {min(k + lane, f - 1)};
+#pragma unroll
+            for (int c = 0; c < NC; ++c) {
+                const int j = min(j0 + c, w - 1);
+                a[c] = fabs((double)DG[j]);
+                x[c][0] = P[(int64_t)j * f + i[0]];
+                ul[c] = np > 0 ? U[(int64_t)min(lane, np - 1) * w + j] : T(0);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+            wave_apply(np, i, ul, x);
+            uint32_t left = 0;
+#pragma unroll
+            for (int c = 0; c < NC; ++c) {
+                const int j = j0 + c;
+                const bool live = j < w && j != first && a[c] >= p.eps && (bj < 0 || a[c] > bv);
+                const bool fails = i[0] != j && !(a[c] >= p.u * fabs((double)x[c][0]));
+                if (uni(live) && !__any(fails)) left |= 1u << c;
+            }
+#pragma unroll 1
+            for (; left; left &= left - 1) {
+                const int j = j0 + __builtin_ctz(left);
+                const double aj = fabs((double)DG[j]);
+                if (uni(bj >= 0 && !(aj > bv))) continue;
+                const T ur[1] = {np > 0 ? U[(int64_t)min(lane, np - 1) * w + j] : T(0)};
+                bool ok = true;
+#pragma unroll 1
+                for (int i0 = k + 64; ok && i0 < f; i0 += 256) {
+                    int ir[4];
+                    T xr[1][4];
+#pragma unroll
+                    for (int t = 0; t < 4; ++t) {
+                        ir[t] = min(i0 + 64 * t + lane, f - 1);
+                        xr[0][t] = P[(int64_t)j * f + ir[t]];
+                    }
+                    wave_apply(np, ir, ur, xr);
+                    bool fails = false;
+#pragma unroll
+                    for (int t = 0; t < 4; ++t) fails |= ir[t] != j && !(aj >= p.u * fabs((double)xr[0][t]));
+                    ok = !__any(fails);
+                }
+                if (ok) {
+                    bv = aj;
+                    bj = j;
+                }
+            }
+        }
+        if (lane == 0) {
+            rb->v[wv] = bv;
+            rb->i[wv] = bj;
+        }
+        __syncthreads();
+        bv = rb->v[0];
+        bj = rb->i[0];
+        for (int q = 1; q < NT / 64; ++q)
+            if (vi_better(rb->v[q], rb->i[q], bv, bj)) {
+                bv = rb->v[q];
+                bj = rb->i[q];
+            }
+        __syncthreads();
+        return uni(bj);
+    }
+    // best_1x1 (ldlt.jl:264-276) on the current diagonal (formed here): the acceptable 1x1 pivot of
+    // k..w-1 with the largest |a_jj|, first on ties, -1 if none; on return y holds the answer's current
+    // column. The largest candidate (|a_jj| >= eps) is tested first, by the whole block: it is usually the
+    // answer (KKT, n = 12,000: in 367 of 619 searches). Where it is not, the others are tested by a wave
+    // each. (One candidate after another by the whole block: a front of 600 columns under a threshold that
+    // nearly all of them fail took 89 ms instead of 16.)
+    __device__ __attribute__((always_inline)) int best_1x1(int k, const LdltPrm& p, T (&y)[R]) const {
+        form_diag(k);
+        double v = -1.0;
+        int bi = -1;
+        for (int j = k + threadIdx.x; j < w; j += NT) {
+            const double a = fabs((double)DG[j]);
+            if (a >= p.eps && vi_better(a, j, v, bi)) {
+                v = a;
+                bi = j;
+            }
+        }
+        block_argmax<NT>(v, bi, *rb);
+        bi = uni(bi);
+        bool tested = false;
+#pragma unroll 1
+        while (bi >= 0) {
+            form_col(bi, k - k0, y);
+            if (tested || uni(v >= p.u * colmax(y, k, f, bi, bi))) return bi;
+            tested = true;
+            bi = search_1x1(k, bi, p);
+        }
+        return -1;
     }
     // pivot choice at column k (ldlt.jl:280-325), as Front::choose on the current columns, column k
     // in xa: c = pivot column, r = 2x2 partner or -1; on return the column c is in xa (1x1), or the
@@ -1136,12 +1248,13 @@ struct PanelFront {
         c = k;
         if (p.pivot == PV_NONE) return;
         pick(xa, k, 0);
-        const double mk = colmax(xa, k, f, k, k);
-        const double akk = fabs(pk[0]);
+        double mk = rows_max(xa, k, f, k, k), akk;
         bool ok, two2 = false;
         double det = 0.0, mx = 0.0;
         int rr = -1;
         if (p.pivot == PV_DIAG) {
+            mk = block_jmax<NT>(mk, *rb);
+            akk = fabs(pk[0]);
             ok = akk >= p.eps && akk >= p.u * mk;
         } else {
             const double alpha = (1.0 + sqrt(17.0)) / 8.0;  // Bunch-Kaufman constant (ldlt.jl:22)
@@ -1159,7 +1272,12 @@ struct PanelFront {
                 }
                 if (rr >= 0) rr = k0 + (int)threadIdx.x + NT * rr;
             }
+            mk = wave_jmax(mk);
+            if ((threadIdx.x & 63) == 0) mx3[0][threadIdx.x >> 6] = mk;
             block_argmax<NT>(lambda, rr, *rb);
+            mk = mx3[0][0];
+            for (int q = 1; q < NT / 64; ++q) mk = jmax(mk, mx3[0][q]);
+            akk = fabs(pk[0]);
             rr = uni(rr);
             if (rr < 0) lambda = 0.0;
             if (rr < 0 || uni(akk >= alpha * lambda)) {
@@ -1169,13 +1287,25 @@ struct PanelFront {
                 pick(xa, rr, 1);
                 pick(xb, k, 2);
                 pick(xb, rr, 3);
-                const double sigma = colmax(xb, k, w, rr, rr);
-                const double arr = pk[3], ark = pk[1], akr = pk[2];
+                // the maxima of column rr's fully summed rows and of the two columns below a 2x2 pivot together
+                double m[3] = {rows_max(xb, k, w, rr, rr), rows_max(xa, k, f, k, rr), rows_max(xb, k, f, rr, k)};
+#pragma unroll
+                for (int q = 0; q < 3; ++q) {
+                    m[q] = wave_jmax(m[q]);
+                    if ((threadIdx.x & 63) == 0) mx3[q][threadIdx.x >> 6] = m[q];
+                }
+                __syncthreads();
+#pragma unroll
+                for (int q = 0; q < 3; ++q) {
+                    m[q] = mx3[q][0];
+                    for (int v = 1; v < NT / 64; ++v) m[q] = jmax(m[q], mx3[q][v]);
+                }
+                const double sigma = m[0], arr = pk[3], ark = pk[1], akr = pk[2];
                 if (uni(akk * sigma >= alpha * lambda * lambda)) {
                     ok = akk >= p.eps && akk >= p.u * mk;
                 } else if (uni(fabs(arr) >= alpha * sigma)) {
                     c = rr;
-                    ok = fabs(arr) >= p.eps && fabs(arr) >= p.u * colmax(xb, k, f, rr, rr);
+                    ok = fabs(arr) >= p.eps && fabs(arr) >= p.u * jmax(m[2], fabs(akr));
                 } else {
                     two2 = true;
                     det = pk[0] * arr - akr * ark;
@@ -1184,8 +1314,7 @@ struct PanelFront {
                     if (uni(ok)) {
                         const double e11 = fabs(arr / det), e12 = fabs(akr / det), e21 = fabs(ark / det),
                                      e22 = fabs(pk[0] / det);
-                        const double m1 = colmax(xa, k, f, k, rr), m2 = colmax(xb, k, f, rr, k);
-                        ok = p.u * (e11 * m1 + e21 * m2) <= 1.0 && p.u * (e12 * m1 + e22 * m2) <= 1.0;
+                        ok = p.u * (e11 * m[1] + e21 * m[2]) <= 1.0 && p.u * (e12 * m[1] + e22 * m[2]) <= 1.0;
                     }
                 }
             }
@@ -1390,7 +1519,7 @@ template <typename T, int NBP>
 struct PanelLds {
     PanelArgs<T> args;
     RedBuf<512> rb;
-    double pk[4];
+    double pk[4], mx3[3][512 / 64];
     int ctype[NBP + 1];
     T Uc[NBP + 1], Lr[NBP + 1];
     T Ls[NBP + 1][NBP + 1];
@@ -1410,7 +1539,7 @@ __device__ __attribute__((always_inline)) inline PanelFront<T, 512, R, NBP + 1> 
     Global<T>*U = uni_ptr(A.U), *DG = U + (int64_t)LP_MAXP * w;
     return PanelFront<T, 512, R, NBP + 1>{uni_ptr(A.P), uni(A.f), w, uni(A.k0), uni_ptr(A.lp), &S.rb, U, DG, DG + w,
                                           (uint32_t)__ballot(lane <= NBP && ct == 1),
-                                          (uint32_t)__ballot(lane <= NBP && ct == 2), S.Uc, S.Lr, S.Ls, S.pk};
+                                          (uint32_t)__ballot(lane <= NBP && ct == 2), S.Uc, S.Lr, S.Ls, S.pk, S.mx3};
 }
 
 // any pivot but the usual one, at column k, from the panel memory (V holds the panel's columns from k

@@ -28,8 +28,9 @@ def _seconds(s):
     return best
 
 
-# a zero diagonal takes 2x2 pivots and interchanges nearly everywhere
-@pytest.mark.parametrize("n,diag,ptype,threshold", [(1500, 0.0, "A", 0.01)])
+# a zero diagonal takes 2x2 pivots and interchanges nearly everywhere; under diagonal pivoting a weak
+# one fails a high threshold for nearly every candidate of every pivot
+@pytest.mark.parametrize("n,diag,ptype,threshold", [(1500, 0.0, "A", 0.01), (600, 0.3, "D", 0.9)])
 def test_default_form_is_not_slower_than_the_other(n, diag, ptype, threshold):
     rng = np.random.default_rng(n)
     A = rng.standard_normal((n, n))
