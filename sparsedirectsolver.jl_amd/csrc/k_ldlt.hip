@@ -25,6 +25,7 @@
 #pragma clang fp contract(off)
 #include "k_front.h"
 #include "k_panel.h"
+#include "panel_plan.h"
 #include "sds_common.h"
 #include "sds_kernels.h"
 
@@ -1712,7 +1713,7 @@ __global__ void __launch_bounds__(512) k_ldlt_panel(DevSym S, const Task* __rest
     const int k0 = k, kend = min(w, k0 + NBP);
     PanelLds<T, NBP>& D = panel_lds<T, NBP>();
     for (int q = tid; q < MAXP; q += NT) D.ctype[q] = 0;
-    if (tid == 0) D.args = {P, scratch + tk.a, dd, ee, f, w, k0, lp, kind, st, psign, S.perm + c0, prm};
+    if (tid == 0) D.args = {P, scratch + (int64_t)tk.a * PANEL_SCR_UNIT, dd, ee, f, w, k0, lp, kind, st, psign, S.perm + c0, prm};
     const int nr = (f - k0 + NT - 1) / NT;
     int nu = 0;  // U rows formed
     int kv = k0;  // the last general pivot
@@ -1804,7 +1805,7 @@ __global__ void __launch_bounds__(256) k_ldlt_trail(DevSym S, const Task* __rest
     if (I0 + TILE <= kend || J0 + TILE <= kend) return;
     T* P = factor + S.panel_off[s];
     const int8_t* kind = pkind + S.super_ptr[s];
-    const T* U = scratch + t.c;
+    const T* U = scratch + (int64_t)t.c * PANEL_SCR_UNIT;
     const int tid = threadIdx.x, i = I0 + (tid & 63), ic = min(i, f - 1), cb = (tid >> 6) * 16;
     for (int q = tid; q < np * TILE; q += 256) {
         const int pp = q / TILE, c = q - pp * TILE;

@@ -19,6 +19,7 @@
 #pragma clang fp contract(off)
 #include "k_front.h"
 #include "k_panel.h"
+#include "panel_plan.h"
 #include "sds_common.h"
 #include "sds_kernels.h"
 
@@ -846,7 +847,7 @@ __global__ void __launch_bounds__(64) k_lu_urows(DevSym S, const Task* __restric
     const T* P = factor + S.panel_off[s];
     T* Q = ufactor + S.panel_off[s];
     const T* dd = dvec + S.super_ptr[s] + k0;
-    T* U = scratch + t.c;
+    T* U = scratch + (int64_t)t.c * PANEL_SCR_UNIT;
     const bool on = j >= k0 + np && j < f;
     const int jc = min(max(j, k0 + np), f - 1);  // (np < f - k0 in a front with columns after the panel)
     // row r of the column in P (fully summed) or of U12, stored by rows, in Q; blocks of eight rows up to
@@ -915,7 +916,7 @@ __global__ void __launch_bounds__(256) k_lu_trail(DevSym S, const Task* __restri
     if (I0 + TILE <= kend || J0 + TILE <= kend) return;
     T* P = factor + S.panel_off[s];
     T* Q = ufactor + S.panel_off[s];
-    const T* U = scratch + t.c;
+    const T* U = scratch + (int64_t)t.c * PANEL_SCR_UNIT;
     const int tid = threadIdx.x, lane = tid & 63, cb = (tid >> 6) * 16;
     const bool u12 = J0 >= w;
     // element c of the thread: row `lane`, column cb + c (P), or column `lane`, row cb + c (Q); A: the

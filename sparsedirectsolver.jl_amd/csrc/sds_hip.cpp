@@ -17,6 +17,7 @@
 #include <vector>
 
 #include "../../include/sds_hip.h"
+#include "panel_plan.h"
 #include "sds_common.h"
 #include "sds_kernels.h"
 
@@ -258,6 +259,7 @@ struct sds_handle {
     int panel_block = 0;  // Cholesky large fronts: panel block width (a multiple of NB; 0 = one block)
     int pivot_panels = 0;  // LDL^T and LU large fronts: 0 panels of pivot columns, 1 one pivot per launch pair
     int64_t ldlt_scr = 0;  // LDL^T and LU panels' scratch (elements)
+    int64_t scr_max = INT64_MAX;  // ... and the most of it a level may take (sds_alloc_numeric)
     void* lscratch = nullptr;
     int32_t* status = nullptr;
     void* dvec = nullptr;        // D: 2n entries of the factor type (diagonal, 2x2 subdiagonals)
@@ -826,14 +828,12 @@ int build_schedule(sds_handle* h, int dtype) {
         for (int32_t s : L.big) wmax = std::max(wmax, h->fncols[s]);
         int fmax = 0;
         for (int32_t s : L.big) fmax = std::max(fmax, h->fnrows[s]);
-        if (lu && !h->pivot_panels && lu_panel_cols(fmax, wmax) > 0) {
-            // pivoted LU of the large fronts in panels: the panel's pivots (one workgroup per front), the
-            // U rows of those pivots in the columns after it (64 columns a task), its update of the
-            // fully summed columns and of U12 (64 x 64 tiles; the lists start anew every 64 columns)
-            std::vector<Task> tp, td;
-            std::vector<int32_t> off;
-            int64_t o = 0;
-            int maxcols = 0;
+        std::vector<int64_t> scr;   // the fronts' panel scratch, and where it lies
+        std::vector<int32_t> off;
+        int64_t scr_total = 0;
+        int maxcols = 0;
+        bool lu_panels = lu && !h->pivot_panels && lu_panel_cols(fmax, wmax) > 0;
+        if (lu_panels) {
             for (int k = 0; k < wmax;) {
                 int rows = 0;
                 for (int32_t s : L.big)
@@ -842,15 +842,20 @@ int build_schedule(sds_handle* h, int dtype) {
                 maxcols = std::max(maxcols, cols);
                 k += cols;
             }
+            for (int32_t s : L.big) scr.push_back((int64_t)maxcols * h->fnrows[s]);
+            lu_panels = panel_offsets(scr, h->scr_max, off, scr_total);
+        }
+        if (lu_panels) {
+            // pivoted LU of the large fronts in panels: the panel's pivots (one workgroup per front), the
+            // U rows of those pivots in the columns after it (64 columns a task), its update of the
+            // fully summed columns and of U12 (64 x 64 tiles; the lists start anew every 64 columns)
+            std::vector<Task> tp, td;
             for (int32_t s : L.big) {
                 tp.push_back({s, 0, 0, 0});
-                off.push_back((int32_t)o);
-                o += (int64_t)maxcols * h->fnrows[s];
                 for (int J0 = 0; J0 < h->fncols[s]; J0 += 64)
                     for (int I0 = 0; I0 <= J0; I0 += 64) td.push_back({s, I0, J0, 0});
             }
-            if (o >= ((int64_t)1 << 31)) return fail(h, SDS_NOT_SUPPORTED, "panel scratch beyond 2^31 entries");
-            h->ldlt_scr = std::max(h->ldlt_scr, o);
+            h->ldlt_scr = std::max(h->ldlt_scr, scr_total);
             const int64_t off_p = (int64_t)tasks.size();
             tasks.insert(tasks.end(), tp.begin(), tp.end());
             int64_t off_r = 0, off_u = 0;
@@ -905,8 +910,8 @@ int build_schedule(sds_handle* h, int dtype) {
             push_launch(L, L_LU_UNIT, td, 0.0, 0.0);
             wmax = 0;
         } else if (lu) {
-            // fronts too tall for a panel's registers (or pivot_panels = 1): pivoted LU one step at a time over all of them: the pivot
-            // (one workgroup per front) and the rank-1 update tiles (every front's remaining
+            // a front too tall for a panel's registers (the whole level then), no room for the scratch, or
+            // pivot_panels = 1: pivoted LU one step at a time over all of them: the pivot (one workgroup per front) and the rank-1 update tiles (every front's remaining
             // fully summed columns and U12, 64 x 64 tiles; one tile list per 64 steps)
             std::vector<Task> tp;
             for (int32_t s : L.big) tp.push_back({s, 0, 0, 0});
@@ -951,26 +956,35 @@ int build_schedule(sds_handle* h, int dtype) {
             // left than a panel's registers hold (or with pivot_panels = 1): one pivot (1x1 or 2x2)
             // per launch pair, the choice by one workgroup per front, its update by the same tiles.
             std::vector<std::pair<int, int>> pan;  // the launches: first column at least, panel columns (0: a pair)
-            int maxcols = 0;
-            for (int k = 0; k < wmax;) {
-                int rows = 0;
-                for (int32_t s : L.big)
-                    if (h->fncols[s] > k) rows = std::max(rows, h->fnrows[s] - k);
-                pan.push_back({k, h->pivot_panels ? 0 : ldlt_panel_cols(rows, wmax - k)});
-                maxcols = std::max(maxcols, pan.back().second);
-                k += std::max(pan.back().second, 1);
+            auto plan_panels = [&](bool panels) {
+                pan.clear();
+                maxcols = 0;
+                for (int k = 0; k < wmax;) {
+                    int rows = 0;
+                    for (int32_t s : L.big)
+                        if (h->fncols[s] > k) rows = std::max(rows, h->fnrows[s] - k);
+                    pan.push_back({k, panels ? ldlt_panel_cols(rows, wmax - k) : 0});
+                    maxcols = std::max(maxcols, pan.back().second);
+                    k += std::max(pan.back().second, 1);
+                }
+            };
+            plan_panels(!h->pivot_panels);
+            for (int32_t s : L.big)
+                scr.push_back(maxcols ? ldlt_panel_scratch(h->fnrows[s], h->fncols[s], maxcols) : 0);
+            if (!panel_offsets(scr, h->scr_max, off, scr_total)) {  // (no room: launch pairs)
+                plan_panels(false);
+                scr_total = 0;
+                off.assign(L.big.size(), 0);
             }
             std::vector<Task> tp, tm;
-            int64_t off = 0;
-            for (int32_t s : L.big) {
-                tp.push_back({s, (int32_t)off, 0, 0});
-                if (maxcols) off += ldlt_panel_scratch(h->fnrows[s], h->fncols[s], maxcols);
+            for (size_t q = 0; q < L.big.size(); ++q) {
+                const int32_t s = L.big[q];
+                tp.push_back({s, off[q], 0, 0});
                 const int w = h->fncols[s];
                 for (int J0 = 0; J0 < w; J0 += 64)
                     for (int I0 = J0; I0 < w; I0 += 64) tm.push_back({s, I0, J0, 0});
             }
-            if (off >= ((int64_t)1 << 31)) return fail(h, SDS_NOT_SUPPORTED, "panel scratch beyond 2^31 entries");
-            h->ldlt_scr = std::max(h->ldlt_scr, off);
+            h->ldlt_scr = std::max(h->ldlt_scr, scr_total);
             push_launch(L, L_LDLT_MIRROR, tm, 0.0, 0.0);
             const int64_t off_p = (int64_t)tasks.size();
             tasks.insert(tasks.end(), tp.begin(), tp.end());
@@ -2083,6 +2097,55 @@ int solve_t(sds_handle* h, const SolveWork& W, int32_t phase, int transposed, co
     return SDS_SUCCESS;
 }
 
+// the launch plan and the numeric storage of it; NO_ROOM: the panels' scratch (at most h->scr_max a level)
+// does not fit
+constexpr int NO_ROOM = -1;
+int alloc_numeric(sds_handle* h, int32_t dtype) {
+    free_numeric(h);
+    int rc = build_schedule(h, dtype);
+    if (rc) return rc;
+
+    size_t es = dtype == SDS_R64 ? 8 : 4;
+    void* p;
+    if ((rc = dev_alloc(h, h->numbufs, es * std::max<int64_t>(h->factor_len, 1), &h->factor))) return rc;
+    if ((rc = dev_alloc(h, h->numbufs, es * std::max<int64_t>(h->cb_len, 1), &h->cbpool))) return rc;
+    h->ufactor = nullptr;
+    if (h->method == M_LU &&
+        (rc = dev_alloc(h, h->numbufs, es * std::max<int64_t>(h->factor_len, 1), &h->ufactor)))
+        return rc;
+    if ((rc = dev_alloc(h, h->numbufs, es * NB * std::max<int64_t>(h->n, 1), &h->dbuf))) return rc;
+    if ((rc = dev_alloc(h, h->numbufs, es * NB * std::max<int64_t>(h->n, 1), &h->lnbuf))) return rc;
+    if ((rc = dev_alloc(h, h->numbufs, sizeof(int32_t) * 3 * (h->ns + 1), &p))) return rc;
+    h->lstep = static_cast<int32_t*>(p);
+    h->lscratch = nullptr;
+    if ((rc = dev_alloc(h, h->numbufs, sizeof(int32_t) * (h->ns + 1), &p))) return rc;
+    h->status = static_cast<int32_t*>(p);
+    if ((rc = dev_alloc(h, h->numbufs, es * 2 * std::max<int64_t>(h->n, 1), &h->dvec))) return rc;
+    if ((rc = dev_alloc(h, h->numbufs, sizeof(int32_t) * std::max<int64_t>(h->n, 1), &p))) return rc;
+    h->piv = static_cast<int32_t*>(p);
+    if ((rc = dev_alloc(h, h->numbufs, std::max<int64_t>(h->n, 1), &p))) return rc;
+    h->pkind = static_cast<int8_t*>(p);
+    if ((rc = dev_alloc(h, h->numbufs, std::max<int64_t>(h->n, 1), &p))) return rc;
+    h->psign = static_cast<int8_t*>(p);
+    if ((rc = dev_alloc(h, h->numbufs, sizeof(double) * 2, &p))) return rc;
+    h->aux = static_cast<double*>(p);
+    if ((rc = dev_alloc(h, h->numbufs, sizeof(int64_t) * NF * (h->ns + 1), &p))) return rc;
+    h->stats = static_cast<int64_t*>(p);
+    if ((rc = dev_alloc(h, h->numbufs, sizeof(int64_t) * (8 + INFO_BLOCKS), &p))) return rc;
+    h->d_info = static_cast<int64_t*>(p);
+    HIPCHK(h, hipHostMalloc((void**)&h->h_info, sizeof(int64_t) * 8, hipHostMallocDefault));
+    HIPCHK(h, hipHostMalloc((void**)&h->h_norms, sizeof(double) * 2 * MAX_NRHS, hipHostMallocDefault));
+    if (h->ldlt_scr > 0) {
+        // the panels' scratch takes at most a quarter of what is left (the solves need workspaces too)
+        size_t room = 0, all = 0;
+        HIPCHK(h, hipMemGetInfo(&room, &all));
+        if (es * h->ldlt_scr > room / 4) return NO_ROOM;
+        if (dev_alloc(h, h->numbufs, es * h->ldlt_scr, &h->lscratch)) return NO_ROOM;
+    }
+    h->dtype = dtype;
+    return SDS_SUCCESS;
+}
+
 }  // namespace
 
 extern "C" {
@@ -2312,43 +2375,14 @@ int sds_alloc_numeric(sds_handle_t h, int32_t dtype, int32_t nbatch) {
     if (nbatch != 1)
         return fail(h, SDS_NOT_SUPPORTED,
                     "nbatch must be 1: upload a uniform batch as the block-diagonal forest of its members");
-    free_numeric(h);
-    int rc = build_schedule(h, dtype);
-    if (rc) return rc;
-
-    size_t es = dtype == SDS_R64 ? 8 : 4;
-    void* p;
-    if ((rc = dev_alloc(h, h->numbufs, es * std::max<int64_t>(h->factor_len, 1), &h->factor))) return rc;
-    if ((rc = dev_alloc(h, h->numbufs, es * std::max<int64_t>(h->cb_len, 1), &h->cbpool))) return rc;
-    h->ufactor = nullptr;
-    if (h->method == M_LU &&
-        (rc = dev_alloc(h, h->numbufs, es * std::max<int64_t>(h->factor_len, 1), &h->ufactor)))
-        return rc;
-    if ((rc = dev_alloc(h, h->numbufs, es * NB * std::max<int64_t>(h->n, 1), &h->dbuf))) return rc;
-    if ((rc = dev_alloc(h, h->numbufs, es * NB * std::max<int64_t>(h->n, 1), &h->lnbuf))) return rc;
-    if ((rc = dev_alloc(h, h->numbufs, sizeof(int32_t) * 3 * (h->ns + 1), &p))) return rc;
-    h->lstep = static_cast<int32_t*>(p);
-    h->lscratch = nullptr;
-    if (h->ldlt_scr > 0 && (rc = dev_alloc(h, h->numbufs, es * h->ldlt_scr, &h->lscratch))) return rc;
-    if ((rc = dev_alloc(h, h->numbufs, sizeof(int32_t) * (h->ns + 1), &p))) return rc;
-    h->status = static_cast<int32_t*>(p);
-    if ((rc = dev_alloc(h, h->numbufs, es * 2 * std::max<int64_t>(h->n, 1), &h->dvec))) return rc;
-    if ((rc = dev_alloc(h, h->numbufs, sizeof(int32_t) * std::max<int64_t>(h->n, 1), &p))) return rc;
-    h->piv = static_cast<int32_t*>(p);
-    if ((rc = dev_alloc(h, h->numbufs, std::max<int64_t>(h->n, 1), &p))) return rc;
-    h->pkind = static_cast<int8_t*>(p);
-    if ((rc = dev_alloc(h, h->numbufs, std::max<int64_t>(h->n, 1), &p))) return rc;
-    h->psign = static_cast<int8_t*>(p);
-    if ((rc = dev_alloc(h, h->numbufs, sizeof(double) * 2, &p))) return rc;
-    h->aux = static_cast<double*>(p);
-    if ((rc = dev_alloc(h, h->numbufs, sizeof(int64_t) * NF * (h->ns + 1), &p))) return rc;
-    h->stats = static_cast<int64_t*>(p);
-    if ((rc = dev_alloc(h, h->numbufs, sizeof(int64_t) * (8 + INFO_BLOCKS), &p))) return rc;
-    h->d_info = static_cast<int64_t*>(p);
-    HIPCHK(h, hipHostMalloc((void**)&h->h_info, sizeof(int64_t) * 8, hipHostMallocDefault));
-    HIPCHK(h, hipHostMalloc((void**)&h->h_norms, sizeof(double) * 2 * MAX_NRHS, hipHostMallocDefault));
-    h->dtype = dtype;
-    return SDS_SUCCESS;
+    // levels whose panels' scratch finds no room take one pivot per launch pair, as small as that may be
+    h->scr_max = INT64_MAX;
+    int rc;
+    while ((rc = alloc_numeric(h, dtype)) == NO_ROOM) {
+        (void)hipGetLastError();
+        h->scr_max = h->ldlt_scr / 2;
+    }
+    return rc;
 }
 
 }  // extern "C"

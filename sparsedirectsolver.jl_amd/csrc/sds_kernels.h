@@ -68,7 +68,7 @@ void launch_ldlt_update(hipStream_t st, const DevSym& S, const Task* tasks, int 
 template <typename T>
 void launch_ldlt_mirror(hipStream_t st, const DevSym& S, const Task* tasks, int n, T* factor);
 // panels of the large fronts: the next `cols` pivot columns of every front (task (s, scratch
-// offset); `first`: the fronts' first launch), then their update of the columns after them (task
+// offset in units of PANEL_SCR_UNIT entries); `first`: the fronts' first launch), then their update of the columns after them (task
 // (s, I0, J0, scratch offset))
 template <typename T>
 void launch_ldlt_panel(hipStream_t st, const DevSym& S, const Task* tasks, int n, int first, int cols, int rows,
