@@ -2880,7 +2880,7 @@ int sds_memory_estimates(sds_handle_t h, int64_t* est) {
     est[9] = maps;
     est[10] = (int64_t)(h->ns + 1) * NF * 8 + (h->ns + 1) * 4 + h->n * 6;
     est[0] = est[6] + est[7] + est[9] + est[10];
-    est[1] = est[0] + est[8];
+    est[1] = est[0] + est[8] + (int64_t)es * h->ldlt_scr;  // (the pivot panels' scratch: held by the factorization only)
     est[4] = est[1];
     return SDS_SUCCESS;
 }
