@@ -259,7 +259,7 @@ int sds_autotune(sds_handle_t handle, const double* nzval, const sds_factor_para
  * {extend-add rows (512, 1024, 2048 or 4096), K chunk (16, 32 or 64), trailing split (0 = never,
  * else >= 1), two-per-CU steps (0 = never, else >= 1), small-front kernels (0, 1 or 2), subtree
  * KiB (0, 16, 32 or 64), panel block (0 or a multiple of 64 up to 4096), pivot panels (LDL^T and LU
- * large fronts: 0 = panels of 4 to 32 columns, one workgroup per front, the default; 1 = one pivot
+ * large fronts: 1 = panels of 4 to 32 columns, one workgroup per front, the default; 0 = one pivot
  * per pair of launches; both give the same factor bit for bit)}. No
  * counterpart in the reference (whose kernels have fixed shapes); it restores a saved tuning
  * without timing again. Takes effect at the next sds_alloc_numeric (the launch plan depends on it).

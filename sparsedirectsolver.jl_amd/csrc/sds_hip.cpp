@@ -257,7 +257,7 @@ struct sds_handle {
     int small_kind = 0;  // small-front kernels (Cholesky): 0 one wave per tiny front + blocked,
                          // 1 one wave per tiny front + column by column, 2 column by column
     int panel_block = 0;  // Cholesky large fronts: panel block width (a multiple of NB; 0 = one block)
-    int pivot_panels = 0;  // LDL^T and LU large fronts: 0 panels of pivot columns, 1 one pivot per launch pair
+    int pivot_panels = 1;  // LDL^T and LU large fronts: 1 panels of pivot columns, 0 one pivot per launch pair
     int64_t ldlt_scr = 0;  // LDL^T and LU panels' scratch (elements)
     int64_t scr_max = INT64_MAX;  // ... and the most of it a level may take (sds_alloc_numeric)
     void* lscratch = nullptr;
@@ -832,7 +832,7 @@ int build_schedule(sds_handle* h, int dtype) {
         std::vector<int32_t> off;
         int64_t scr_total = 0;
         int maxcols = 0;
-        bool lu_panels = lu && !h->pivot_panels && lu_panel_cols(fmax, wmax) > 0;
+        bool lu_panels = lu && h->pivot_panels && lu_panel_cols(fmax, wmax) > 0;
         if (lu_panels) {
             for (int k = 0; k < wmax;) {
                 int rows = 0;
@@ -911,7 +911,7 @@ int build_schedule(sds_handle* h, int dtype) {
             wmax = 0;
         } else if (lu) {
             // a front too tall for a panel's registers (the whole level then), no room for the scratch, or
-            // pivot_panels = 1: pivoted LU one step at a time over all of them: the pivot (one workgroup per front) and the rank-1 update tiles (every front's remaining
+            // pivot_panels = 0: pivoted LU one step at a time over all of them: the pivot (one workgroup per front) and the rank-1 update tiles (every front's remaining
             // fully summed columns and U12, 64 x 64 tiles; one tile list per 64 steps)
             std::vector<Task> tp;
             for (int32_t s : L.big) tp.push_back({s, 0, 0, 0});
@@ -953,7 +953,7 @@ int build_schedule(sds_handle* h, int dtype) {
             // after (64 x 64 tiles: the remaining fully summed columns, all rows; one tile list per
             // 64 columns). A panel takes at least `cols` columns (a 2x2 pivot at its end one more),
             // so the panels' widths add up to the level's widest front. While a front has more rows
-            // left than a panel's registers hold (or with pivot_panels = 1): one pivot (1x1 or 2x2)
+            // left than a panel's registers hold (or with pivot_panels = 0): one pivot (1x1 or 2x2)
             // per launch pair, the choice by one workgroup per front, its update by the same tiles.
             std::vector<std::pair<int, int>> pan;  // the launches: first column at least, panel columns (0: a pair)
             auto plan_panels = [&](bool panels) {
@@ -968,7 +968,7 @@ int build_schedule(sds_handle* h, int dtype) {
                     k += std::max(pan.back().second, 1);
                 }
             };
-            plan_panels(!h->pivot_panels);
+            plan_panels(h->pivot_panels);
             for (int32_t s : L.big)
                 scr.push_back(maxcols ? ldlt_panel_scratch(h->fnrows[s], h->fncols[s], maxcols) : 0);
             if (!panel_offsets(scr, h->scr_max, off, scr_total)) {  // (no room: launch pairs)
