@@ -13,10 +13,11 @@
 // block formed in one workgroup; large fronts are assembled in global memory by the
 // shared column-chunk and extend-add kernels and factored on the panel in place (the full
 // w x w fully summed block lives in the panel's top rows, the upper triangle being the
-// mirror the reference keeps), one pivot per pair of launches: the pivot choice by one
-// workgroup per front, its update by 64 x 64 tiles over the GPU; then their contribution
-// block is updated by 64 x 64 tiles, each entry subtracting the terms W[i, k] L[j, k] in
-// the order k = 0, 1, ... of the reference.
+// mirror the reference keeps), in panels of 4 to 16 pivot columns held in one workgroup's registers,
+// each followed by its update of the columns after it by 64 x 64 tiles over the GPU (fronts too
+// tall for that: one pivot per pair of launches); then their contribution block is updated by
+// 64 x 64 tiles, each entry subtracting the terms W[i, k] L[j, k] in the order k = 0, 1, ... of the
+// reference.
 //
 // Reference counterparts: ref_ldlt! and _ldlt_front! (src/reference/ldlt.jl:121-202,
 // :384-454), _choose_pivot (:280-325), _best_1x1 (:264-276), the threshold test
@@ -1545,8 +1546,9 @@ __device__ __attribute__((always_inline)) inline PanelFront<T, 512, R, NBP + 1> 
 
 // any pivot but the usual one, at column k, from the panel memory (V holds the panel's columns from k
 // on, nu pivot rows are formed); returns the next column. Part of the kernel: the panel's registers are free
-// meanwhile. As a function of its own, its pointers in a struct, it had its columns and the caller's
-// registers in scratch memory and every access a flat one (36 us a pivot instead of 23).
+// meanwhile. (As a function of its own, its pointers in a struct, it had its columns and the caller's
+// registers in scratch memory and every access a flat one: a dense front of 1,500 columns with hardly a
+// usual pivot took 41.7 ms, 24.5 now, 26.6 with one pivot per launch pair.)
 template <typename T, int R, int NBP>
 __device__ __attribute__((always_inline)) inline int panel_general(int k, int nu) {
     const auto Z = panel_front<T, R, NBP>();
@@ -1668,8 +1670,9 @@ __device__ __attribute__((always_inline)) inline int panel_general(int k, int nu
 //
 // Bound: latency, one workgroup per front walks the pivots one after another. NT = 512 (two waves
 // per SIMD) leaves 256 registers a thread, 192 of them for the panel: NBP R <= 96. KKT, n = 12,000,
-// FP64: a usual pivot 3.5 us, another 36 us, a launch 129 us (16 columns), 79 (8), 59 (4); one pivot
-// per launch pair took 17.9 us, refactorization and solve 157 ms instead of 118.
+// FP64, one pivot in six not a usual one: a launch takes 78 us (16 columns, 3 rows a thread), 113 (6 rows), 64
+// (8 columns), 43 (4), refactorization and solve 98 ms (157 with one pivot per launch pair). A
+// usual pivot takes 3.5 us, another about 23 us with 3 rows a thread and 35 with 6.
 template <typename T, int R, int NBP>
 __global__ void __launch_bounds__(512) k_ldlt_panel(DevSym S, const Task* __restrict__ tasks, int first,
                                                     T* __restrict__ factor, T* __restrict__ dvec,
@@ -2012,7 +2015,7 @@ void launch_ldlt_panel(hipStream_t st, const DevSym& S, const Task* tasks, int n
     hipLaunchKernelGGL((k_ldlt_panel<T, R, C>), dim3(n), dim3(512), 0, st, S, tasks, first, factor, dvec, piv, kind, \
                        stats, lstep, scratch, p, scaled, aux, psign)
     switch (cols) {
-        case 16:
+        case 16:  // (3 rows a thread do half the work of 6: 78 us a launch instead of 113)
             if (rows <= 3 * 512)
                 PANEL(3, 16);
             else
@@ -2034,8 +2037,10 @@ int64_t ldlt_panel_scratch(int f, int w, int cols) { return lp_scratch(f, w, col
 // columns of the next panel of fronts with at most `rows` rows and `cols` columns left (0: too tall
 // for the registers of one workgroup). The widest panel whose rows fit: a panel pays two launches
 // and its loads and stores once, whatever its columns; no wider than the columns left need. Measured
-// per pivot on the KKT fronts: 16 columns 8 us, 8 columns 10, 4 columns (5,121 to 7,168 rows) 15 us
-// against 17.9 us of a launch pair; taller fronts do not fit the registers.
+// per column on the KKT fronts, with the update: 16 columns 5.4 to 7.6 us, 8 columns 9, 4 columns (5,121 to
+// 7,168 rows) 13 us against 17.9 us of a launch pair; taller fronts do not fit the registers. Where hardly a pivot is
+// a usual one (a dense front with zero diagonal) panels take 0.76 to 1.0 of the pairs' time, under a
+// threshold that most of the diagonal fails up to 1.2 (n = 2,000, 0.9).
 int ldlt_panel_cols(int rows, int cols) {
     if (rows <= 6 * 512 && cols > 8) return 16;
     if (rows <= 10 * 512) return 8;
